@@ -124,6 +124,11 @@ void fill_kparams_from(KParams &k, const spc2_params &P, int n, int nx, int ny, 
   k.kappa = P.kappa;
   double outer = P.system == SPC2_VORTEX ? std::max(P.rho, P.xi_r) : P.rho;
   k.outer2 = outer * outer;
+  k.xa2 = P.xi_a * P.xi_a;
+  k.rxa2 = 1.0 / k.xa2;
+  k.rxa = 1.0 / P.xi_a;
+  k.wid = P.rho - P.xi_a;
+  k.rwid = 1.0 / k.wid;
   k.xa2f = (float)(P.xi_a * P.xi_a);
   k.xr2f = (float)(P.xi_r * P.xi_r);
   k.outer2f = (float)k.outer2;

@@ -48,7 +48,7 @@ struct Rep {
   int poff, n;          // first home / global id, particles
   int coff;             // first cell (all-pairs replicas own one cell)
   int soff, nseg;       // first row segment, segments (linked replicas)
-  int apoff, apblocks;  // first block and blocks of the all-pairs launch
+  int apoff, apblocks;  // first block (among its system's) and blocks of an all-pairs replica
   uint64_t seed;
   int64_t step;         // the replica's own step counter at the start of the call
   int64_t steps;        // steps the replica takes in the current call
@@ -143,66 +143,77 @@ __device__ __forceinline__ EpiCtx rep_ctx(const EpiCtx &e, const Rep &R, int k) 
   return c;
 }
 
-// All-pairs replicas (rho > L/4): a thread per particle (the FP32 chimera
-// pass 1: a group of allpairs_lanes lanes per particle); their homes are in id
-// order (one cell, sorted by id), so a particle's slot is its home.  Block ab
-// of the all-pairs blocks.
-template <int PREC, int EPI>
+// All-pairs replicas (rho > L/4): a wavefront sums one particle at a time, as a
+// single handle's, kApBatch particles in turn, and its first kApBatch lanes then
+// take their epilogues side by side: a batch fills the device with its linked
+// replicas, so what counts is the instructions issued, and an epilogue (about
+// 1000 of them) run by one lane per wavefront cost the 512-replica sweep 2.4%.
+// Their homes are in id order (one cell, sorted by id), so a particle's slot is
+// its home.  Block ab of the all-pairs blocks of the replicas of one system.
+constexpr int kApBatch = 8;
+constexpr int kApPerBlock = kB / kApLanes * kApBatch;  // particles per block
+template <int PREC, int SYS, int EPI>
 __device__ __forceinline__ void b_allpairs1(const Rep *reps, const int *ap_rep, int ab, const double *gx,
                                             const double *gy, const double *gp, const float4 *f4, const EpiCtx &e,
                                             int k) {
   const Rep &R = reps[ap_rep[ab]];
   if (k >= R.steps) return;
-  const int G = allpairs_lanes(PREC, R.system);  // lanes per particle, as a single handle's
-  const int t = (ab - R.apoff) * kB + threadIdx.x, i = t / G, g = t % G;
-  if (i >= R.n) return;  // whole lane groups
+  const int i0 = (ab - R.apoff) * kApPerBlock + threadIdx.x / kApLanes * kApBatch, g = threadIdx.x % kApLanes;
   const KParams P = R.kp;
   const EpiCtx c = rep_ctx(e, R, k);
   Pass1Out o{};
-  if (R.system == SPC2_CHIMERA) {  // the replica's one cell holds its particles in id order: tile j is id j
-    if constexpr (PREC == P32K)
-      allpairs_pass1_group(P, i, g, gx + R.poff, gy + R.poff, gp + R.poff, f4 + R.poff, o);
-    else
-      allpairs_pass1<PREC, SPC2_CHIMERA>(P, i, gx + R.poff, gy + R.poff, gp + R.poff, o);
-  } else {
-    allpairs_pass1<PREC, SPC2_VORTEX>(P, i, gx + R.poff, gy + R.poff, gp + R.poff, o);
+  for (int r = 0; r < kApBatch && i0 + r < R.n; ++r) {
+    // (the replica's one cell holds its particles in id order: tile j is id j)
+    Pass1Out q{};
+    allpairs_pass1<PREC, SYS>(P, i0 + r, g, gx + R.poff, gy + R.poff, gp + R.poff, f4 + R.poff, q);
+    if (g == r) o = q;
   }
-  if (g == 0) epilogue1<EPI>(P, c, R.poff + i, i, R.poff + i, o);
+  const int i = i0 + g;
+  if (g < kApBatch && i < R.n) epilogue1<EPI>(P, c, R.poff + i, i, R.poff + i, o);
 }
 
-template <int PREC>
+template <int SYS>
 __device__ __forceinline__ void b_allpairs2_srk(const Rep *reps, const int *ap_rep, int ab, const double *gx,
                                                 const double *gy, const double *gp, const EpiCtx &e, int k) {
   const Rep &R = reps[ap_rep[ab]];
   if (k >= R.steps) return;
-  const int G = allpairs_lanes(PREC, R.system);  // lanes per particle, as a single handle's
-  const int t = (ab - R.apoff) * kB + threadIdx.x, i = t / G, g = t % G;
-  if (i >= R.n) return;  // whole lane groups
+  const int i0 = (ab - R.apoff) * kApPerBlock + threadIdx.x / kApLanes * kApBatch, g = threadIdx.x % kApLanes;
   const KParams P = R.kp;
   const EpiCtx c = rep_ctx(e, R, k);
   const int o0 = R.poff;
-  Pass2Out o;
-  if (R.system == SPC2_CHIMERA) {
-    if constexpr (PREC == P32K)
-      allpairs_pass2_group(P, i, g, gx + o0, gy + o0, gp + o0, e.aphi_slot + o0, e.n_slot + o0, 0.0, 0.0, o);
-    else
-      allpairs_pass2<SPC2_CHIMERA>(P, i, gx + o0, gy + o0, gp + o0, e.aphi_slot + o0, e.n_slot + o0,
-                                   e.n2_slot + o0, 0.0, 0.0, o);
-  } else {
-    allpairs_pass2<SPC2_VORTEX>(P, i, gx + o0, gy + o0, gp + o0, e.aphi_slot + o0, e.n_slot + o0, e.n2_slot + o0,
-                                0.0, 0.0, o);
+  Pass2Out o{};
+  for (int r = 0; r < kApBatch && i0 + r < R.n; ++r) {
+    Pass2Out q;
+    allpairs_pass2<SYS>(P, i0 + r, g, gx + o0, gy + o0, gp + o0, e.aphi_slot + o0, e.n_slot + o0, e.n2_slot + o0,
+                        0.0, 0.0, q);
+    if (g == r) o = q;
   }
-  if (g == 0) epilogue2<EPI_SRK>(P, c, o0 + i, i, o);
+  const int i = i0 + g;
+  if (g < kApBatch && i < R.n) epilogue2<EPI_SRK>(P, c, o0 + i, i, o);
 }
 
-// The all-pairs blocks lead the pass launches: the first ap.pad blocks (ap.n
-// of them used, ap.pad a multiple of 8 so that the row segments keep their XCD
-// mapping) take all-pairs replicas.  They are few and long, and starting first
-// they run beside the row segments instead of after them.
+// The chimera all-pairs blocks lead the pass launches: the first ap.pad blocks
+// (ap.n of them used, ap.pad a multiple of 8 so that the row segments keep
+// their XCD mapping) take all-pairs replicas and run beside the row segments.
+// Vortex all-pairs replicas (rare: N < 160 at the workloads' density) have a
+// launch of their own, since their registers (150) would leave the merged
+// kernel 2 wavefronts per SIMD instead of 3: 1.69 against 1.22 ms per step of
+// the 512-replica sweep.
 struct ApBlocks {
   const int *rep;
   int n, pad;
 };
+
+template <int PREC, int EPI>
+__global__ __launch_bounds__(kB) void k_b_pass1_ap_vortex(const Rep *reps, const int *ap_rep, const double *gx,
+                                                          const double *gy, const double *gp, EpiCtx e, int k) {
+  b_allpairs1<PREC, SPC2_VORTEX, EPI>(reps, ap_rep, blockIdx.x, gx, gy, gp, nullptr, e, k);
+}
+
+__global__ __launch_bounds__(kB) void k_b_pass2_ap_vortex(const Rep *reps, const int *ap_rep, const double *gx,
+                                                          const double *gy, const double *gp, EpiCtx e, int k) {
+  b_allpairs2_srk<SPC2_VORTEX>(reps, ap_rep, blockIdx.x, gx, gy, gp, e, k);
+}
 
 // Pass 1 over every row segment of every linked replica: pair sums and the SE
 // update (EPI_SE), or the SRK step's Ito intermediates by slot (EPI_ITO1).
@@ -212,7 +223,7 @@ __global__ __launch_bounds__(kB) void k_b_pass1(const Rep *reps, const int *seg_
                                                 const double *gy, const double *gp, EpiCtx e, int k, ApBlocks ap) {
   extern __shared__ float4 dyn_lds[];
   if ((int)blockIdx.x < ap.pad) {
-    if ((int)blockIdx.x < ap.n) b_allpairs1<PREC, EPI>(reps, ap.rep, blockIdx.x, gx, gy, gp, t.f4, e, k);
+    if ((int)blockIdx.x < ap.n) b_allpairs1<PREC, SPC2_CHIMERA, EPI>(reps, ap.rep, blockIdx.x, gx, gy, gp, t.f4, e, k);
     return;
   }
   const int sg = xcd_segment(blockIdx.x - ap.pad, gridDim.x - ap.pad);
@@ -236,7 +247,7 @@ __global__ __launch_bounds__(kB) void k_b_pass2_srk(const Rep *reps, const int *
                                                     ApBlocks ap) {
   extern __shared__ float4 dyn_lds[];
   if ((int)blockIdx.x < ap.pad) {
-    if ((int)blockIdx.x < ap.n) b_allpairs2_srk<PREC>(reps, ap.rep, blockIdx.x, gx, gy, gp, e, k);
+    if ((int)blockIdx.x < ap.n) b_allpairs2_srk<SPC2_CHIMERA>(reps, ap.rep, blockIdx.x, gx, gy, gp, e, k);
     return;
   }
   const int sg = xcd_segment(blockIdx.x - ap.pad, gridDim.x - ap.pad);
@@ -362,7 +373,8 @@ __global__ __launch_bounds__(kB) void k_b_iota(int n, int *a, int *b) {
 
 struct spc2_batch {
   int count = 0, prec = P32K;
-  int nt = 0, nct = 0, nseg = 0, nap = 0;  // particles, cells, row segments, all-pairs blocks
+  int nt = 0, nct = 0, nseg = 0;  // particles, cells, row segments
+  int nap = 0, napv = 0;  // all-pairs blocks of chimera and of vortex replicas (in that order in ap_rep)
   hipStream_t stream = nullptr;
   std::vector<spc2_params> params;
   std::vector<Rep> reps;
@@ -425,7 +437,8 @@ spc2_status check_launch(const char *what) {
 // Replica layout: KParams, cells and segments of each replica (tile targets
 // from b.target), the segment -> replica and all-pairs block -> replica maps.
 spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &ap_rep) {
-  int poff = 0, coff = 0, soff = 0, apoff = 0;
+  int poff = 0, coff = 0, soff = 0;
+  std::vector<int> ap_vortex;
   size_t lds_cap = 0;
   seg_rep.clear();
   ap_rep.clear();
@@ -453,10 +466,10 @@ spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &a
       lds_cap = std::max(lds_cap, (size_t)R.kp.lds_cap);
     } else {
       R.soff = R.nseg = 0;
-      R.apoff = apoff;
-      R.apblocks = bfor((long long)R.n * allpairs_lanes(b.prec, p.system));
-      for (int q = 0; q < R.apblocks; ++q) ap_rep.push_back(r);
-      apoff += R.apblocks;
+      std::vector<int> &list = p.system == SPC2_CHIMERA ? ap_rep : ap_vortex;
+      R.apoff = (int)list.size();
+      R.apblocks = (R.n + kApPerBlock - 1) / kApPerBlock;
+      list.insert(list.end(), (size_t)R.apblocks, r);
       coff += 1;
     }
     poff += R.n;
@@ -464,7 +477,9 @@ spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &a
   b.nt = poff;
   b.nct = coff;
   b.nseg = soff;
-  b.nap = apoff;
+  b.nap = (int)ap_rep.size();
+  b.napv = (int)ap_vortex.size();
+  ap_rep.insert(ap_rep.end(), ap_vortex.begin(), ap_vortex.end());
   b.lds = lds_cap * (size_t)lds_elem_bytes(b.prec);
   return SPC2_OK;
 }
@@ -551,7 +566,7 @@ void launch_step_kernels(spc2_batch &b, const EpiCtx &e, int k, bool srk, bool s
                      (const double *)b.gx, (const double *)b.gy, (const double *)b.gp, b.slot_h, b.slot_id, b.t);
   const ApBlocks ap{b.ap_rep, b.nap, (b.nap + 7) / 8 * 8};
   const dim3 gpass(ap.pad + b.nseg);
-  if (gpass.x == 0) return;
+  const int *ap_vortex = b.ap_rep + b.nap;
   EpiCtx es = e;  // the state-writing pass's context
   if (fuse) {
     es.bgx = b.spare[0];
@@ -562,6 +577,11 @@ void launch_step_kernels(spc2_batch &b, const EpiCtx &e, int k, bool srk, bool s
     es.blocal = b.local;
   }
   if (!srk) {
+    if (b.napv)
+      hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1_ap_vortex<PREC, EPI_SE>), dim3(b.napv), blk, 0, b.stream,
+                         (const Rep *)b.d_reps, ap_vortex, (const double *)b.gx, (const double *)b.gy,
+                         (const double *)b.gp, es, k);
+    if (gpass.x == 0) return;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1<PREC, EPI_SE>), gpass, blk, b.lds, b.stream, (const Rep *)b.d_reps,
                        (const int *)b.seg_rep, (const int *)b.start, b.t, (const int *)b.slot_h,
                        (const int *)b.slot_id, (const double *)b.gx, (const double *)b.gy, (const double *)b.gp, es,
@@ -572,6 +592,14 @@ void launch_step_kernels(spc2_batch &b, const EpiCtx &e, int k, bool srk, bool s
   // stage tiles; pass 2 reads every replica's pass-1 values
   EpiCtx e1 = e;
   e1.sa.zero_in = 1;  // derivative zero-filled each step
+  if (b.napv) {
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1_ap_vortex<PREC, EPI_ITO1>), dim3(b.napv), blk, 0, b.stream,
+                       (const Rep *)b.d_reps, ap_vortex, (const double *)b.gx, (const double *)b.gy,
+                       (const double *)b.gp, e1, k);
+    hipLaunchKernelGGL(k_b_pass2_ap_vortex, dim3(b.napv), blk, 0, b.stream, (const Rep *)b.d_reps, ap_vortex,
+                       (const double *)b.gx, (const double *)b.gy, (const double *)b.gp, es, k);
+  }
+  if (gpass.x == 0) return;
   hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1<PREC, EPI_ITO1>), gpass, blk, b.lds, b.stream, (const Rep *)b.d_reps,
                      (const int *)b.seg_rep, (const int *)b.start, b.t, (const int *)b.slot_h,
                      (const int *)b.slot_id, (const double *)b.gx, (const double *)b.gy, (const double *)b.gp, e1, k,
@@ -633,7 +661,7 @@ spc2_status run_steps(spc2_batch &b, int method, double dt, int64_t nsteps, cons
     e.sa.omega = b.omega;
     // the next step's stage and bins come from this step's state-writing pass
     // when every replica takes that step and no re-homing comes between
-    const bool fuse = k + 1 < kmin && b.since_rehome + 1 < kRehomeEvery && b.nap + b.nseg > 0;
+    const bool fuse = k + 1 < kmin && b.since_rehome + 1 < kRehomeEvery && b.nap + b.napv + b.nseg > 0;
     switch (b.prec) {
       case P64: launch_step_kernels<P64>(b, e, (int)k, srk, staged, fuse); break;
       case P64F: launch_step_kernels<P64F>(b, e, (int)k, srk, staged, fuse); break;

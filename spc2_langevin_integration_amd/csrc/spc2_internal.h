@@ -41,6 +41,7 @@ struct KParams {
   // vortex
   double mu_plus, mu_minus, xi_a, xi_r, kappa;
   double outer2;  // max(rho, xi_r)^2: widest test radius
+  double xa2, rxa2, rxa, wid, rwid;  // xi_a^2, its reciprocal, 1 / xi_a; rho - xi_a and its reciprocal
   float xa2f, xr2f, outer2f, xaf, rhof, mu_pf, mu_p_over_xa2f, c4f, kappaf, v0f, Df;
   // outer W(r) = c4 (r - xi_a)(rho - r) in Horner form r (w_a - c4 r) + w_b,
   // w_a = c4 (xi_a + rho), w_b = -c4 xi_a rho

@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include "spc2_device.h"
+#include "spc2_fp64_math.h"
 #include "spc2_internal.h"
 
 namespace spc2 {
@@ -59,18 +60,19 @@ struct SrcOf<P32K> {
   using type = Src32;
 };
 
-// AlignmentStrength, VortexArraysSystemPtr.cpp:737-749
+// AlignmentStrength, VortexArraysSystemPtr.cpp:737-749 (its divisions are by
+// launch constants)
 __device__ __forceinline__ double vortex_w(const KParams &P, double r) {
-  if (r < P.xi_a) return P.mu_plus * (1.0 - r * r / (P.xi_a * P.xi_a));
-  if (r < P.rho) return -P.mu_minus * 4.0 * (r - P.xi_a) * (P.rho - r) / (P.rho - P.xi_a) / (P.rho - P.xi_a);
-  return 0.0;
+  const double in = P.mu_plus * (1.0 - div_by(r * r, P.xa2, P.rxa2));
+  const double an = div_by(div_by(-P.mu_minus * 4.0 * (r - P.xi_a) * (P.rho - r), P.wid, P.rwid), P.wid, P.rwid);
+  return r < P.xi_a ? in : (r < P.rho ? an : 0.0);
 }
 
 // AlignmentStrengthDerivative, VortexArraysSystemPtr.cpp:751-763
 __device__ __forceinline__ double vortex_dw(const KParams &P, double r) {
-  if (r < P.xi_a) return P.mu_plus * (-2.0 * r / P.xi_a / P.xi_a);
-  if (r < P.rho) return -P.mu_minus * 4.0 * (-2.0 * r + P.rho + P.xi_a) / (P.rho - P.xi_a) / (P.rho - P.xi_a);
-  return 0.0;
+  const double in = P.mu_plus * div_by(div_by(-2.0 * r, P.xi_a, P.rxa), P.xi_a, P.rxa);
+  const double an = div_by(div_by(-P.mu_minus * 4.0 * (-2.0 * r + P.rho + P.xi_a), P.wid, P.rwid), P.wid, P.rwid);
+  return r < P.xi_a ? in : (r < P.rho ? an : 0.0);
 }
 
 // FP64 distance^2 of slots k and m with the reference min-image: decides the
@@ -1417,157 +1419,125 @@ void launch_pair(Sim &s, void (*kern)(KArgs...), dim3 grid, dim3 blk, size_t sh,
   }
 }
 
-// Lanes per particle of the FP32 chimera all-pairs pass (allpairs_group_lanes):
-// a group of kApLanes consecutive lanes shares one particle, lane g summing
-// partners j = g, g + kApLanes, ...; small all-pairs systems have too few
-// particles to fill the device one lane each.
-constexpr int kApLanes = 16;
-template <int PREC, int SYS>
-constexpr int allpairs_lanes() { return PREC == P32K && SYS == SPC2_CHIMERA ? kApLanes : 1; }
-__host__ __device__ inline int allpairs_lanes(int prec, int sys) {
-  return prec == P32K && sys == SPC2_CHIMERA ? kApLanes : 1;
+// All pairs (rho > L/4): a wavefront per particle, lane g summing partners j =
+// g, g + 64, ... in ascending order, then the lanes' sums added in a fixed
+// butterfly (the same total in every lane).  These systems are small (a few
+// hundred to a few thousand particles), so that a lane per particle leaves most
+// of the device idle and one lane's serial chain of partners sets the time; 64
+// lanes per particle cut the chain 64-fold and read the partners coalesced.
+// Measured per step, a lane per particle against a wavefront (the FP64 term
+// functions of spc2_fp64_math.h included): chimera SRK in FP64 at N = 1500
+// 1186 -> 41 us, vortex RK4 at N = 1000 2740 -> 80 us.  Unrolling the partner
+// loop by four raises the registers (149 to 157 and 67 to 96) and is 8% slower.
+constexpr int kApLanes = 64;
+
+__device__ __forceinline__ double group_sum(double v) {
+#pragma unroll
+  for (int d = 1; d < kApLanes; d <<= 1) v += __shfl_xor(v, d, kApLanes);
+  return v;
+}
+__device__ __forceinline__ int group_sum(int v) {
+#pragma unroll
+  for (int d = 1; d < kApLanes; d <<= 1) v += __shfl_xor(v, d, kApLanes);
+  return v;
 }
 
-// The FP32 chimera all-pairs pass 1 of particle i by its group's lane g (every
-// lane of the group calls it): each lane's Kahan sums over its partners, in
-// ascending j, then the lanes' FP64 values and counts added across the group in
-// a fixed butterfly (the same total in every lane).  Geometry and the cos, sin
-// of phi_j as allpairs_pass1 forms them.
-__device__ __forceinline__ void allpairs_pass1_group(const KParams &P, int i, int g, const double *gx,
-                                                     const double *gy, const double *gp, const float4 *tiles,
-                                                     Pass1Out &o) {
+// Pass 1 of particle i by lane g of its wavefront (every lane calls it): stage
+// positions not wrapped (ChimeraSystem.cpp:131-167, :184-254); arrays by
+// particle id; FP64 geometry in every precision form.  tiles (the FP32 chimera
+// form): FP32 tiles by particle id whose cos and sin are (float) of the FP64
+// sincos of gp, summed in each lane's Kahan sums.
+template <int PREC, int SYS>
+__device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, int g, const double *gx, const double *gy,
+                                               const double *gp, const float4 *tiles, Pass1Out &o) {
   const double xi = gx[i], yi = gy[i], pi = gp[i];
-  Kahan Sf, Cf;
-  Sf.init();
-  Cf.init();
-  int n = 0;
-  for (int j = g; j < P.n; j += kApLanes) {
-    if (j == i) continue;
-    double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-    double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
-    double r2 = dx * dx + dy * dy;
-    if (r2 <= P.rho2) {
-      const float4 tj = tiles[j];
-      Sf.add(tj.w);
-      Cf.add(tj.z);
-      ++n;
-    }
-  }
-  double S = Sf.value(), C = Cf.value();
-#pragma unroll
-  for (int d = 1; d < kApLanes; d <<= 1) {
-    S += __shfl_xor(S, d, kApLanes);
-    C += __shfl_xor(C, d, kApLanes);
-    n += __shfl_xor(n, d, kApLanes);
-  }
-  double sa, ca;
-  sincos(pi + P.alpha, &sa, &ca);
-  o.n = n;
-  o.written = n != 0;
-  o.aphi = n != 0 ? P.sigma * (ca * S - sa * C) / (double)n : 0.0;
   o.n2 = 0;
   o.vortex_add = 0;
   o.phase = pi;
-}
-
-// All pairs (rho > L/4): thread per particle, j = 0..N-1 ascending, stage
-// positions not wrapped (ChimeraSystem.cpp:131-167, :184-254); arrays by
-// particle id.
-// tiles (FP32 form, optional): FP32 tiles by particle id whose cos and sin are
-// (float) of the FP64 sincos of gp, read instead of forming them per pair (the
-// same values).
-template <int PREC, int SYS>
-__device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, const double *gx, const double *gy,
-                                               const double *gp, Pass1Out &o, const float4 *tiles = nullptr) {
-  const double xi = gx[i], yi = gy[i], pi = gp[i];
-  if (SYS == SPC2_CHIMERA) {
-    if (PREC == P64) {
-      double A = 0.0;
-      int n = 0;
-      for (int j = 0; j < P.n; ++j) {
-        if (j == i) continue;
-        double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-        double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
-        double r2 = dx * dx + dy * dy;
-        if (r2 <= P.rho2) {
-          A += sin(gp[j] - pi - P.alpha);
-          ++n;
+  if constexpr (SYS == SPC2_CHIMERA) {
+    // sum of sin(phi_j - phi_i - alpha) over |r_ij| <= rho: per pair (P64), or
+    // from the sums of sin phi_j and cos phi_j (the factored forms)
+    double S = 0.0, C = 0.0;
+    Kahan Sf, Cf;
+    Sf.init();
+    Cf.init();
+    int n = 0;
+#pragma unroll 1
+    for (int j = g; j < P.n; j += kApLanes) {
+      const double pj = PREC == P32K ? 0.0 : gp[j];
+      const float4 tj = PREC == P32K ? tiles[j] : float4{};
+      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double r2 = dx * dx + dy * dy;
+      if ((r2 <= P.rho2) & (j != i)) {
+        if constexpr (PREC == P64) {
+          S += sin_term(pj - pi - P.alpha);
+        } else if constexpr (PREC == P32K) {
+          Sf.add(tj.w);
+          Cf.add(tj.z);
+        } else {
+          S += sin_term(pj);
+          C += cos_term(pj);
         }
+        ++n;
       }
-      o.n = n;
-      o.written = n != 0;
-      o.aphi = n != 0 ? P.sigma * A / (double)n : 0.0;
-    } else {
-      // factored form; the FP32 variant accumulates in Kahan FP32 over FP64 geometry
-      double S = 0.0, C = 0.0;
-      Kahan Sf, Cf;
-      Sf.init();
-      Cf.init();
-      int n = 0;
-      for (int j = 0; j < P.n; ++j) {
-        if (j == i) continue;
-        double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-        double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
-        double r2 = dx * dx + dy * dy;
-        if (r2 <= P.rho2) {
-          if (PREC == P32K && tiles) {
-            const float4 tj = tiles[j];
-            Sf.add(tj.w);
-            Cf.add(tj.z);
-            ++n;
-            continue;
-          }
-          double sj, cj;
-          sincos(gp[j], &sj, &cj);
-          if (PREC == P32K) {
-            Sf.add((float)sj);
-            Cf.add((float)cj);
-          } else {
-            S += sj;
-            C += cj;
-          }
-          ++n;
-        }
-      }
-      if (PREC == P32K) {
-        S = Sf.value();
-        C = Cf.value();
-      }
+    }
+    if constexpr (PREC == P32K) {
+      S = Sf.value();
+      C = Cf.value();
+    }
+    n = group_sum(n);
+    double A = group_sum(S);
+    if constexpr (PREC != P64) {
       double sa, ca;
       sincos(pi + P.alpha, &sa, &ca);
-      o.n = n;
-      o.written = n != 0;
-      o.aphi = n != 0 ? P.sigma * (ca * S - sa * C) / (double)n : 0.0;
+      A = ca * A - sa * group_sum(C);
     }
-    o.n2 = 0;
-    o.vortex_add = 0;
+    o.n = n;
+    o.written = n != 0;
+    o.aphi = n != 0 ? P.sigma * A / (double)n : 0.0;
   } else {
     double A = 0.0, B = 0.0, Cc = 0.0;
     int n0 = 0, n1 = 0, n2 = 0;
-    for (int j = 0; j < P.n; ++j) {
-      if (j == i) continue;
-      double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-      double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
-      double dr = sqrt(dx * dx + dy * dy);
-      if (dr <= P.xi_a) {
-        A += vortex_w(P, dr) * sin(gp[j] - pi);
+#pragma unroll 1
+    for (int j = g; j < P.n; j += kApLanes) {
+      const double pj = gp[j];
+      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double r2 = dx * dx + dy * dy;
+      // (partners beyond both radii cannot pass the tests of the root below)
+      if ((r2 > P.outer2 * 1.000000000001) | (j == i)) continue;
+      const double dr = sqrt_sep(r2);
+      if (dr <= P.rho) {
+        const double t = vortex_w(P, dr) * sin_term(pj - pi);
+        if (dr <= P.xi_a) {
+          A += t;
+          ++n0;
+        } else {
+          B += t;
+          ++n1;
+        }
+      } else if (dr <= P.xi_a) {  // xi_a beyond rho
+        A += vortex_w(P, dr) * sin_term(pj - pi);
         ++n0;
-      } else if (dr <= P.rho) {
-        B += vortex_w(P, dr) * sin(gp[j] - pi);
-        ++n1;
       }
       if (dr <= P.xi_r) {
         Cc += -P.kappa * sin(atan2(dy, dx) - pi);
         ++n2;
       }
     }
+    n0 = group_sum(n0);
+    n1 = group_sum(n1);
+    n2 = group_sum(n2);
+    A = group_sum(A);
+    B = group_sum(B);
+    Cc = group_sum(Cc);
     o.n = n0 + n1;
     o.n2 = n2;
     if (n0 + n1 > 0) {
       o.aphi = (A + B) / ((double)n0 + (double)n1);
       if (n2 > 0) o.aphi += Cc / (double)n2;
       o.written = 1;
-      o.vortex_add = 0;
     } else {
       o.aphi = 0.0;
       o.written = 0;
@@ -1575,106 +1545,70 @@ __device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, const do
       o.coh = n2 > 0 ? Cc / (double)n2 : 0.0;
     }
   }
-  o.phase = pi;
 }
 
-
-// All-pairs pass 2 (rho > L/4) of particle i, arrays by particle id (FP64 terms
-// for every precision: the small-N path; the FP32 chimera form spreads them over
-// a lane group, allpairs_pass2_group); in0, in1: the additional values before
-// the call (zero for the SRK step).
+// All-pairs pass 2 of particle i by lane g of its wavefront (FP64 terms for
+// every precision form); in0, in1: the additional values before the call (zero
+// for the SRK step), added to the lanes' total.
 template <int SYS>
-__device__ __forceinline__ void allpairs_pass2(const KParams &P, int i, const double *gx, const double *gy,
+__device__ __forceinline__ void allpairs_pass2(const KParams &P, int i, int g, const double *gx, const double *gy,
                                                const double *gp, const double *aphi, const double *nslot,
                                                const double *n2slot, double in0, double in1, Pass2Out &o) {
   const double xi = gx[i], yi = gy[i], pi = gp[i];
   const double ai = aphi[i], n = nslot[i];
-  double a0 = in0, a1 = in1;
-  if (SYS == SPC2_VORTEX) {
+  double s0 = 0.0, s1 = 0.0;
+  o.phase = pi;
+  o.ai = ai;
+  if constexpr (SYS == SPC2_VORTEX) {
     // VortexArraysSystemPtr.cpp:305-353
     const double n2 = n2slot[i];
-    const double vxi = P.v0 * cos(pi), vyi = P.v0 * sin(pi);
-    for (int j = 0; j < P.n; ++j) {
-      if (j == i) continue;
-      double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-      double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
-      double dr = sqrt(dx * dx + dy * dy);
+    const double vxi = P.v0 * cos_term(pi), vyi = P.v0 * sin_term(pi);
+#pragma unroll 1
+    for (int j = g; j < P.n; j += kApLanes) {
+      const double pj = gp[j], aj = aphi[j];
+      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double r2 = dx * dx + dy * dy;
+      if ((r2 > P.outer2 * 1.000000000001) | (j == i)) continue;
+      const double dr = sqrt_sep(r2);
       const bool al = (dr <= P.rho) && (n > 0.0), co = (dr <= P.xi_r) && (n2 > 0.0);
       if (!al && !co) continue;
-      const double pj = gp[j];
-      const double vxj = P.v0 * cos(pj), vyj = P.v0 * sin(pj);
+      const double vxj = P.v0 * cos_term(pj), vyj = P.v0 * sin_term(pj);
       if (al) {
-        double cph = cos(pj - pi);
-        double sph = sin(pj - pi);
-        double w = vortex_w(P, dr);
-        double dw = vortex_dw(P, dr);
-        a0 += -w * cph / n;
-        a1 += ((vxj - vxi) * dw * dx / dr + (vyj - vyi) * dw * dy / dr) * sph / n + (aphi[j] - ai) * w * cph / n -
+        const double cph = cos_term(pj - pi), sph = sin_term(pj - pi);
+        const double w = vortex_w(P, dr), dw = vortex_dw(P, dr);
+        s0 += -w * cph / n;
+        s1 += ((vxj - vxi) * dw * dx / dr + (vyj - vyi) * dw * dy / dr) * sph / n + (aj - ai) * w * cph / n -
               2.0 * P.D * sph * w / n;
       }
       if (co) {
-        double th = atan2(dy, dx);
-        double cpp = cos(th - pi);
-        double spp = sin(th - pi);
-        a0 += P.kappa * cpp / n2;
-        a1 += -P.kappa * ((vxj - vxi) * (-dy) / dr / dr + (vyj - vyi) * dx / dr / dr - ai) * cpp / n2 +
+        const double th = atan2(dy, dx);
+        const double cpp = cos(th - pi), spp = sin(th - pi);
+        s0 += P.kappa * cpp / n2;
+        s1 += -P.kappa * ((vxj - vxi) * (-dy) / dr / dr + (vyj - vyi) * dx / dr / dr - ai) * cpp / n2 +
               P.kappa * P.D * spp / n2;
       }
     }
-    o.phase = pi;
-    o.ai = ai;
-    o.a0 = a0 * sqrt(2.0 * P.D);
-    o.a1 = a1;
-    return;
-  }
-  // ChimeraSystem.cpp:223-254
-  for (int j = 0; j < P.n; ++j) {
-    if (j == i) continue;
-    double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-    double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
-    double r2 = dx * dx + dy * dy;
-    if ((r2 <= P.rho2) && (n != 0)) {
-      double cph = cos(gp[j] - pi - P.alpha);
-      a0 += cph / n;
-      a1 += (aphi[j] - ai) * cph / n;
+    o.a0 = (in0 + group_sum(s0)) * sqrt(2.0 * P.D);
+    o.a1 = in1 + group_sum(s1);
+  } else {
+    // ChimeraSystem.cpp:223-254
+    const double rn = 1.0 / n;
+#pragma unroll 1
+    for (int j = g; j < P.n; j += kApLanes) {
+      const double pj = gp[j], aj = aphi[j];
+      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double r2 = dx * dx + dy * dy;
+      if ((r2 <= P.rho2) & (n != 0) & (j != i)) {
+        const double cph = cos_term(pj - pi - P.alpha);
+        s0 += div_by(cph, n, rn);
+        s1 += div_by((aj - ai) * cph, n, rn);
+      }
     }
+    o.a0 = (in0 + group_sum(s0)) * -sqrt(2.0 * P.D);
+    o.a1 = (in1 + group_sum(s1)) + -2.0 * P.D * ai;
   }
-  o.phase = pi;
-  o.ai = ai;
-  o.a0 = a0 * -sqrt(2.0 * P.D);
-  o.a1 = a1 + -2.0 * P.D * ai;
-}
-
-// Chimera all-pairs pass 2 of particle i by lane g of its group (the FP32
-// form, allpairs_lanes lanes per particle; every lane of the group calls it):
-// allpairs_pass2's FP64 terms, each lane's over its partners j = g, g + G, ...,
-// added across the group in a fixed butterfly and then to in0, in1.
-__device__ __forceinline__ void allpairs_pass2_group(const KParams &P, int i, int g, const double *gx,
-                                                     const double *gy, const double *gp, const double *aphi,
-                                                     const double *nslot, double in0, double in1, Pass2Out &o) {
-  const double xi = gx[i], yi = gy[i], pi = gp[i];
-  const double ai = aphi[i], n = nslot[i];
-  double s0 = 0.0, s1 = 0.0;
-  for (int j = g; j < P.n; j += kApLanes) {
-    if (j == i) continue;
-    double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-    double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
-    double r2 = dx * dx + dy * dy;
-    if ((r2 <= P.rho2) && (n != 0)) {
-      double cph = cos(gp[j] - pi - P.alpha);
-      s0 += cph / n;
-      s1 += (aphi[j] - ai) * cph / n;
-    }
-  }
-#pragma unroll
-  for (int d = 1; d < kApLanes; d <<= 1) {
-    s0 += __shfl_xor(s0, d, kApLanes);
-    s1 += __shfl_xor(s1, d, kApLanes);
-  }
-  o.phase = pi;
-  o.ai = ai;
-  o.a0 = (in0 + s0) * -sqrt(2.0 * P.D);
-  o.a1 = (in1 + s1) + -2.0 * P.D * ai;
 }
 
 }  // namespace

@@ -41,39 +41,32 @@ __global__ __launch_bounds__(kBlock) void k_pass2_lds(KParams P, const int *__re
 }
 
 // =============================================================================
-// All pairs (rho > L/4): thread per particle (the FP32 chimera pass 1: a group
-// of allpairs_lanes lanes per particle), j = 0..N-1, stage positions not
-// wrapped (ChimeraSystem.cpp:131-167, :184-254)
+// All pairs (rho > L/4): a wavefront per particle (allpairs_pass1), four to a
+// workgroup.
 // =============================================================================
 
 template <int PREC, int SYS, int EPI>
 __global__ __launch_bounds__(kBlock) void k_pass1_allpairs(KParams P, const double *gx, const double *gy,
                                                            const double *gp, const float4 *tiles, EpiCtx e,
                                                            unsigned long long *counts) {
-  constexpr int G = allpairs_lanes<PREC, SYS>();  // lanes per particle
-  const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / G, g = t % G;
-  const bool active = i < P.n, lead = active && g == 0;  // whole lane groups
+  const int i = blockIdx.x * (kBlock / kApLanes) + threadIdx.x / kApLanes, g = threadIdx.x % kApLanes;
+  const bool active = i < P.n, lead = active && g == 0;  // whole wavefronts
   Pass1Out o{};
   if (active) {
-    if constexpr (G > 1) allpairs_pass1_group(P, i, g, gx, gy, gp, tiles, o);
-    else allpairs_pass1<PREC, SYS>(P, i, gx, gy, gp, o, tiles);
+    allpairs_pass1<PREC, SYS>(P, i, g, gx, gy, gp, tiles, o);
     if (lead) epilogue1<EPI>(P, e, i, i, i, o);  // all pairs: home order is the id order
   }
   if (counts) count_add(counts, lead ? P.n - 1 : 0, lead ? o.n : 0, lead ? o.n2 : 0);
 }
 
-template <int PREC, int SYS, int EPI>
+template <int SYS, int EPI>
 __global__ __launch_bounds__(kBlock) void k_pass2_allpairs(KParams P, const double *gx, const double *gy,
                                                            const double *gp, EpiCtx e) {
-  constexpr int G = allpairs_lanes<PREC, SYS>();  // lanes per particle
-  const int t = blockIdx.x * blockDim.x + threadIdx.x, i = t / G, g = t % G;
-  if (i >= P.n) return;  // whole lane groups
+  const int i = blockIdx.x * (kBlock / kApLanes) + threadIdx.x / kApLanes, g = threadIdx.x % kApLanes;
+  if (i >= P.n) return;  // whole wavefronts
   Pass2Out o;
   const double in0 = EPI == EPI_ITO2 ? e.a0[i] : 0.0, in1 = EPI == EPI_ITO2 ? e.a1[i] : 0.0;
-  if constexpr (G > 1)
-    allpairs_pass2_group(P, i, g, gx, gy, gp, e.aphi_slot, e.n_slot, in0, in1, o);
-  else
-    allpairs_pass2<SYS>(P, i, gx, gy, gp, e.aphi_slot, e.n_slot, e.n2_slot, in0, in1, o);
+  allpairs_pass2<SYS>(P, i, g, gx, gy, gp, e.aphi_slot, e.n_slot, e.n2_slot, in0, in1, o);
   if (g == 0) epilogue2<EPI>(P, e, i, i, o);
 }
 
@@ -100,7 +93,7 @@ void pass1_typed(Sim &s, const EpiCtx &e) {
                   (const int *)s.slot_h, (const int *)s.slot_id, (const double *)s.gp, e, cnt);
   } else {
     // the FP32 form reads cos and sin of phi_j from the stage's tiles
-    launch_pair(s, k_pass1_allpairs<PREC, SYS, EPI>, dim3(blocks_for((long long)s.n * allpairs_lanes<PREC, SYS>())),
+    launch_pair(s, k_pass1_allpairs<PREC, SYS, EPI>, dim3(blocks_for((long long)s.n * kApLanes)),
                 dim3(kBlock), 0, s.kp,
                 (const double *)s.gx, (const double *)s.gy, (const double *)s.gp,
                 PREC == P32K ? (const float4 *)s.t.f4 : nullptr, e, cnt);
@@ -137,8 +130,7 @@ void pass2_typed(Sim &s, const EpiCtx &e) {
       launch_pair(s, k_pass2_lds<Vort2Acc<PREC>, PREC, EPI>, grid, blk, sh, s.kp, (const int *)s.start, s.t,
                   (const int *)s.slot_h, (const int *)s.slot_id, (const double *)s.gp, e);
   } else {
-    launch_pair(s, k_pass2_allpairs<PREC, SYS, EPI>, dim3(blocks_for((long long)s.n * allpairs_lanes<PREC, SYS>())),
-                dim3(kBlock), 0, s.kp, (const double *)s.gx,
+    launch_pair(s, k_pass2_allpairs<SYS, EPI>, dim3(blocks_for((long long)s.n * kApLanes)), dim3(kBlock), 0, s.kp, (const double *)s.gx,
                 (const double *)s.gy, (const double *)s.gp, e);
   }
 }
