@@ -106,6 +106,8 @@ void fill_kparams_from(KParams &k, const spc2_params &P, int n, int nx, int ny, 
   k.Ly = P.Ly;
   k.rLx = 1.0 / P.Lx;
   k.rLy = 1.0 / P.Ly;
+  k.r2Lx = 2.0 * k.rLx;
+  k.r2Ly = 2.0 * k.rLy;
   k.hx = nx > 0 ? P.Lx / nx : P.Lx;
   k.hy = ny > 0 ? P.Ly / ny : P.Ly;
   k.hxf = (float)k.hx;

@@ -480,7 +480,7 @@ spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &a
   b.nap = (int)ap_rep.size();
   b.napv = (int)ap_vortex.size();
   ap_rep.insert(ap_rep.end(), ap_vortex.begin(), ap_vortex.end());
-  b.lds = lds_cap * (size_t)lds_elem_bytes(b.prec);
+  b.lds = lds_cap * (size_t)lds_elem_bytes(b.prec) + (size_t)lds_near_bytes(b.prec);
   return SPC2_OK;
 }
 

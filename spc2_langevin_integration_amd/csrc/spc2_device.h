@@ -22,9 +22,10 @@ struct Box {
 // dx = x_j - x_i; dx -= int(dx * 2.0 / L) * L (truncation toward zero).  Three
 // instructions: the truncation stays in FP64, and the fused product rounds as
 // the separate one does, since the count of boxes (0, +-1; +-2 at most for
-// stage positions just outside the box) times L is exact.
-__device__ __forceinline__ double min_image(double d, double L, double rL) {
-  return __builtin_fma(-__builtin_trunc(d * (2.0 * rL)), L, d);
+// stage positions just outside the box) times L is exact.  r2L = 2 (1 / L), a
+// launch constant: the product is that of d * 2.0 * (1 / L).
+__device__ __forceinline__ double min_image(double d, double L, double r2L) {
+  return __builtin_fma(-__builtin_trunc(d * r2L), L, d);
 }
 
 // Scalar wrap, PeriodicBoundaryConditions.cpp:117-121: x - floor(x / L) * L.

@@ -17,21 +17,29 @@ namespace spc2 {
 // nearest whole number, whose parity is then bit 0 of the sum.
 constexpr double kPiHi = 0x1.921fb54442d18p+1, kPiLo = 0x1.1a62633145c07p-53, kInvPi = 0x1.45f306dc9c883p-2;
 constexpr double kRound = 0x1.8p+52;
-constexpr double kTrigMax = 1048576.0;  // larger arguments, infinities and NaN take the library functions
+constexpr double kTrigMax = 0x1p+45;  // larger arguments, infinities and NaN take the library functions
+
+// a * b + c with c in its own registers.  The compiler forms an accumulating
+// v_fmac for these and copies each coefficient into its destination first, 7
+// more instructions per sine.
+__device__ __forceinline__ double fma3(double a, double b, double c) {
+  double d;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  return d;
+}
 
 // sin(r) for |r| <= pi / 2 (and a hair beyond): r + r^3 p(r^2), p the degree-7
 // minimax polynomial of (sin(r) / r - 1) / r^2 in relative error of sin, found
 // by a Remez exchange in 60-digit arithmetic; the fit's error is 2^-61.6.
 __device__ __forceinline__ double sin_half_turn(double r) {
   const double z = r * r;
-  double p = 0x1.882935a9c68d3p-49;
-  p = __builtin_fma(p, z, -0x1.ae43199df130ap-41);
-  p = __builtin_fma(p, z, 0x1.6123cb1a05428p-33);
-  p = __builtin_fma(p, z, -0x1.ae6454cb1cd5fp-26);
-  p = __builtin_fma(p, z, 0x1.71de3a52874a4p-19);
-  p = __builtin_fma(p, z, -0x1.a01a01a0148abp-13);
-  p = __builtin_fma(p, z, 0x1.11111111110c1p-7);
-  p = __builtin_fma(p, z, -0x1.5555555555555p-3);
+  double p = fma3(0x1.882935a9c68d3p-49, z, -0x1.ae43199df130ap-41);
+  p = fma3(p, z, 0x1.6123cb1a05428p-33);
+  p = fma3(p, z, -0x1.ae6454cb1cd5fp-26);
+  p = fma3(p, z, 0x1.71de3a52874a4p-19);
+  p = fma3(p, z, -0x1.a01a01a0148abp-13);
+  p = fma3(p, z, 0x1.11111111110c1p-7);
+  p = fma3(p, z, -0x1.5555555555555p-3);
   return __builtin_fma(r * z, p, r);
 }
 
@@ -44,25 +52,38 @@ __device__ __forceinline__ double flip_sign(double s, int odd) {
   return __hiloint2double(__double2hiint(s) ^ (odd << 31), __double2loint(s));
 }
 
-// sin(x): x = k pi + r, k the nearest whole number.  k pi_hi is a multiple of
-// 2^-51, so x - k pi_hi is exact in one fma for |x| <= kTrigMax.  18 FP64-rate
-// instructions; at most 1.64 ulp off and 3.8e-17 rms over |x| <= 2000 (a
-// correctly rounded sine: 2.7e-17), far below the rounding of the sums of 30 to
-// 150 such terms.
-__device__ __forceinline__ double sin_term(double x) {
-  if (__builtin_expect(!(__builtin_fabs(x) <= kTrigMax), 0)) return sin_any(x);
+// sin(x) for |x| <= kTrigMax: x = k pi + r, k the nearest whole number.  k pi_hi
+// is a multiple of 2^-51, so x - k pi_hi is exact in one fma, and the part of
+// k pi beyond pi_hi + pi_lo stays below 2^-62.  18 FP64-rate instructions; at
+// most 1.64 ulp off and 3.8e-17 rms over |x| <= 2000 (a correctly rounded sine:
+// 2.7e-17), far below the rounding of the sums of 30 to 150 such terms.
+__device__ __forceinline__ double sin_fast(double x) {
   const double kr = __builtin_fma(x, kInvPi, kRound), k = kr - kRound;
   const double r = __builtin_fma(-k, kPiLo, __builtin_fma(-k, kPiHi, x));
   return flip_sign(sin_half_turn(r), __double2loint(kr));
 }
 
-// cos(x): x = (k + 1/2) pi + r, cos(x) = -(-1)^k sin(r).
-__device__ __forceinline__ double cos_term(double x) {
-  if (__builtin_expect(!(__builtin_fabs(x) <= kTrigMax), 0)) return cos_any(x);
+// cos(x) for |x| <= kTrigMax: x = (k + 1/2) pi + r, cos(x) = -(-1)^k sin(r).
+__device__ __forceinline__ double cos_fast(double x) {
   const double kr = __builtin_fma(x, kInvPi, -0.5) + kRound, k = (kr - kRound) + 0.5;
   const double r = __builtin_fma(-k, kPiLo, __builtin_fma(-k, kPiHi, x));
   return flip_sign(sin_half_turn(r), ~__double2loint(kr));
 }
+
+// The same for any x.  FAST: the caller has checked the phases (phase_fits).
+template <bool FAST = false>
+__device__ __forceinline__ double sin_term(double x) {
+  if (!FAST && __builtin_expect(!(__builtin_fabs(x) <= kTrigMax), 0)) return sin_any(x);
+  return sin_fast(x);
+}
+template <bool FAST = false>
+__device__ __forceinline__ double cos_term(double x) {
+  if (!FAST && __builtin_expect(!(__builtin_fabs(x) <= kTrigMax), 0)) return cos_any(x);
+  return cos_fast(x);
+}
+
+// Whether differences of such phases stay within kTrigMax.
+__device__ __forceinline__ bool phase_fits(double p) { return __builtin_fabs(p) <= kTrigMax / 4; }
 
 // sqrt(a) of a squared separation: the hardware estimate of 1 / sqrt(a) and two
 // Goldschmidt steps with a residual correction, the correctly rounded root for

@@ -33,7 +33,7 @@ enum Epi : int {
 // Scalars every force kernel needs (one copy per launch, by value).
 struct KParams {
   int n, nx, ny, linked;
-  double Lx, Ly, rLx, rLy, hx, hy;
+  double Lx, Ly, rLx, rLy, r2Lx, r2Ly, hx, hy;  // rL = 1 / L, r2L = 2 rL
   float hxf, hyf;
   double rho, rho2;
   float rho2f;
@@ -56,6 +56,7 @@ struct KParams {
   // row) or, with chunk 0, row segments of seg_w cells; LDS capacity in tile
   // elements per workgroup
   int seg_w, segs, lds_cap, chunk;
+  int lanes;  // lanes per centre particle of the FP64 cell walks (a power of two; 1 in the FP32 form)
 };
 
 // Tile arrays in cell-sorted slot order, written by the rank kernel.
@@ -228,6 +229,7 @@ void launch_rank_tiles(Sim &s);
 constexpr double kSegTarget = 256.0;  // default particles per pair workgroup (row chunk or segment)
 constexpr int kLdsBytes = 60 * 1024;  // dynamic LDS of one pair workgroup at most
 int lds_elem_bytes(int prec);
+int lds_near_bytes(int prec);
 void configure_segments_kp(KParams &k, int prec, double target);
 void configure_segments(Sim &s);
 void launch_pass1(Sim &s, int epi, double *ox, double *oy, double *op, const StepArgs &sa, double *const k1[3],

@@ -245,56 +245,170 @@ __device__ __forceinline__ void cell_run(Acc &acc, const Src32 &src, int a, int 
 }
 
 // Visits the candidates of the centre particle at LDS index ei (halo column qi)
-// in reference order; returns the number of candidates.
-template <class Acc, class S>
-__device__ __forceinline__ int visit_lds(Acc &acc, const S &src, const SegShared &sh, int ncol, int qi, int ei,
+// in reference order, the FP32 forms; returns the number of candidates.
+template <class Acc>
+__device__ __forceinline__ int visit_lds(Acc &acc, const Src32 &src, const SegShared &sh, int ncol, int qi, int ei,
                                          const KParams &P) {
   int cand = 0;
-  if constexpr (std::is_same<S, Src32>::value) {
-    // FP32 form: one loop per stencil cell, its column offset computed once
-    // (the value the per-candidate selection gives inside that cell), its
-    // terms summed in FP32 partials that are added to the compensated sums
-    // after the cell
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      const int base = r * ncol + qi;
-      const int lo = sh.off[base - 1], b1 = sh.off[base], b2 = sh.off[base + 1], hi = sh.off[base + 2];
-      acc.row(r - 1, b1, b2, P);
-      cand += hi - lo;
-      const float ol = acc.co.col(-1), oc = acc.co.col(0), orr = acc.co.col(1);
-      cell_run<false>(acc, src, lo, b1, ol, ei, P);
-      if (r == 1) cell_run<true>(acc, src, b1, b2, oc, ei, P);
-      else cell_run<false>(acc, src, b1, b2, oc, ei, P);
-      cell_run<false>(acc, src, b2, hi, orr, ei, P);
-    }
-    return cand - 1;
-  }
+  // one loop per stencil cell, its column offset computed once (the value the
+  // per-candidate selection gives inside that cell), its terms summed in FP32
+  // partials that are added to the compensated sums after the cell
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
     const int base = r * ncol + qi;
     const int lo = sh.off[base - 1], b1 = sh.off[base], b2 = sh.off[base + 1], hi = sh.off[base + 2];
     acc.row(r - 1, b1, b2, P);
     cand += hi - lo;
-    if (r == 1) {
+    const float ol = acc.co.col(-1), oc = acc.co.col(0), orr = acc.co.col(1);
+    cell_run<false>(acc, src, lo, b1, ol, ei, P);
+    if (r == 1) cell_run<true>(acc, src, b1, b2, oc, ei, P);
+    else cell_run<false>(acc, src, b1, b2, oc, ei, P);
+    cell_run<false>(acc, src, b2, hi, orr, ei, P);
+  }
+  return cand - 1;
+}
+
+// The FP64 forms: lane g of the particle's P.lanes lanes takes the g-th of
+// P.lanes equal runs of each stencil row's candidates.  The factored form sums a
+// candidate where it meets it.  The plain form's terms (a sine or cosine and
+// more, 20 to 90 instructions) would run at nearly every candidate if they stood
+// behind the distance test, since some lane of the wavefront has a partner there
+// although only a third of the candidates are partners.  So the lane first tests
+// its candidates, a bit each (8 instructions), then sums the set ones: a
+// wavefront runs the terms about as often as its longest lane has partners.
+// `near` (LDS, a column per thread): the words of bits with the LDS index of
+// each word's first candidate; when they are full the partners so far are
+// summed.
+// Bound by FP64 issue and its latency at 3 wavefronts per SIMD (58-65% issue).
+// Chimera SRK at N = 262,144: pass 1 371 -> 142 us, pass 2 499 -> 163 us; at N =
+// 1000 (SE, 16 lanes per particle) 45.6 -> 12.6 us.  Also tried: candidates
+// interleaved over the lanes (186 and 220 us: three address instructions per
+// candidate), one partner a turn (145 and 177 us), the next turn's partners read
+// ahead (151 and 174 us: more registers), 4 wavefronts per SIMD forced (spills,
+// 146 and 182 us), 4 lanes at least (136 and 179 us).
+constexpr int kNearWords = 8;
+struct NearWords {
+  uint32_t bits[kNearWords][kPairBlock];
+  uint16_t first[kNearWords][kPairBlock];
+};
+
+// The run [a, b) of lane g among `len` candidates.
+__device__ __forceinline__ void lane_run(int len, int g, int lg, int &a, int &b) {
+  const int per = (len + (1 << lg) - 1) >> lg;
+  a = min(g * per, len);
+  b = min(a + per, len);
+}
+
+template <class Acc>
+__device__ __forceinline__ int visit_lds64(Acc &acc, const Src64 &src, const SegShared &sh, int ncol, int qi, int ei,
+                                           int g, bool wraps, NearWords *near, const KParams &P) {
+  const int lg = __builtin_ctz((unsigned)P.lanes);
+  int cand = 0;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) cand += sh.off[r * ncol + qi + 2] - sh.off[r * ncol + qi - 1];
+  const auto row_run = [&](int r, int &m0, int &hi) {
+    const int lo = sh.off[r * ncol + qi - 1];
+    int a, b;
+    lane_run(sh.off[r * ncol + qi + 2] - lo, g, lg, a, b);
+    m0 = lo + a;
+    hi = lo + b;
+  };
+  if constexpr (HasNear<Acc>::value) {
+    const int me = threadIdx.x;
+    CohQueue64 cq;
+    int r = 0, m0, hi;
+    row_run(0, m0, hi);
+    bool more = true;  // candidates left (of any lane)
+    while (more) {
+      int words = 0;
+      while (words < kNearWords) {
+        while (m0 >= hi && r < 2) {
+          ++r;
+          row_run(r, m0, hi);
+        }
+        if (m0 >= hi) break;
+        const int cnt = min(32, hi - m0);
+        uint32_t word = 0;
+        // four at a time; those past the run (read from the LDS that follows)
+        // are masked off
+        for (int u = 0; u < cnt; u += 4) {
+          uint32_t b = 0;
+          if (wraps) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) b |= acc.template near<true>(src, m0 + u + k, P) ? 1u << k : 0u;
+          } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) b |= acc.template near<false>(src, m0 + u + k, P) ? 1u << k : 0u;
+          }
+          word |= b << u;
+        }
+        if (cnt < 32) word &= (1u << cnt) - 1u;
+        if ((unsigned)(ei - m0) < 32u) word &= ~(1u << (ei - m0));  // not the particle itself
+        near->bits[words][me] = word;
+        near->first[words][me] = (uint16_t)m0;
+        ++words;
+        m0 += 32;
+      }
+      more = __any(m0 < hi || r < 2);
+      // the set bits in turn, the wavefront's lanes in step, two partners (of one
+      // word) a turn; the cohesion queue is emptied when it may overflow and after
+      // the last partner
+      using In = typename Acc::In;
+      uint32_t m = 0;
+      int w = 0, first = 0;
+      bool left = true;
+      while (left) {
+        if (m == 0 && w < words) {  // (an empty word leaves the lane idle for a turn)
+          m = near->bits[w][me];
+          first = near->first[w][me];
+          ++w;
+        }
+        if (m != 0) {
+          const int c0 = first + __builtin_ctz(m);
+          m &= m - 1u;
+          const bool two = m != 0;
+          const int c1 = two ? first + __builtin_ctz(m) : c0;
+          m &= m - 1u;  // (0 stays 0)
+          const In v0(src, c0), v1(src, c1);
+          const bool q0 = acc.template term<true>(v0, true, P), q1 = acc.template term<true>(v1, two, P);
+          if (q0) cq.push(c0);
+          if (q1) cq.push(c1);
+        }
+        left = __any(m != 0 || w < words);
+        if (!left || __any(cq.n > CohQueue64::kFull - 2)) cq.drain(acc, src, P);
+      }
+    }
+  } else {
+#pragma unroll 1
+    for (int r = 0; r < 3; ++r) {
+      int m0, hi;
+      row_run(r, m0, hi);
 #pragma unroll 2
-      for (int m = lo; m < ei; ++m) acc.pair(src, m, P);
-#pragma unroll 2
-      for (int m = ei + 1; m < hi; ++m) acc.pair(src, m, P);
-    } else {
-#pragma unroll 2
-      for (int m = lo; m < hi; ++m) acc.pair(src, m, P);
+      for (int m = m0; m < hi; ++m)
+        if (m != ei) acc.pair(src, m, P);
     }
   }
   return cand - 1;
 }
 
-// Same visit over the global tiles, cell by cell (slot k in cell c).
+// Same visit over the global tiles, cell by cell (slot k in cell c); the FP64
+// forms' lane g takes the run of each stencil row that visit_lds64 gives it.
 template <class Acc, class S>
-__device__ __forceinline__ int visit_global(Acc &acc, const S &src, const int *start, int c, int k, const KParams &P) {
+__device__ __forceinline__ int visit_global(Acc &acc, const S &src, const int *start, int c, int k, int g,
+                                            const KParams &P) {
   const int cx = c % P.nx, cy = c / P.nx;
   int cand = 0;
   for (int dyo = -1; dyo <= 1; ++dyo) {
     const int row = adjust_cell(cy + dyo, P.ny) * P.nx;
+    int pos = 0, ra = 0, rb = 0;  // the row's candidates before this cell; the lane's run of the row
+    if constexpr (!std::is_same<S, Src32>::value) {
+      int len = 0;
+      for (int dxo = -1; dxo <= 1; ++dxo) {
+        const int jc = row + adjust_cell(cx + dxo, P.nx);
+        len += start[jc + 1] - start[jc];
+      }
+      lane_run(len, g, __builtin_ctz((unsigned)P.lanes), ra, rb);
+    }
     for (int dxo = -1; dxo <= 1; ++dxo) {
       const int jc = row + adjust_cell(cx + dxo, P.nx);
       const int m0 = start[jc], m1 = start[jc + 1];
@@ -310,12 +424,26 @@ __device__ __forceinline__ int visit_global(Acc &acc, const S &src, const int *s
           if (m != k) acc.template pair<SUM_GROUP>(src, m, P);
         acc.flush();
       } else {
-        for (int m = m0; m < m1; ++m)
+        const int e = m0 + min(m1 - m0, rb - pos);
+        for (int m = m0 + max(0, ra - pos); m < e; ++m)
           if (m != k) acc.pair(src, m, P);
+        pos += m1 - m0;
       }
     }
   }
   return cand - 1;
+}
+
+// A halo column or row of the workgroup wraps: without one the candidates'
+// separations need no min-image.
+__device__ __forceinline__ bool wraps(const KParams &P, const Seg &g) {
+  return g.cx0 < 1 || g.cx0 + g.W >= P.nx || g.cy < 1 || g.cy + 1 >= P.ny;
+}
+
+// The plain FP64 form's words, after the staged tiles.
+template <int PREC, int PASS>
+__device__ __forceinline__ NearWords *near_words(void *dyn_lds, const KParams &P) {
+  return (NearWords *)((char *)dyn_lds + (size_t)P.lds_cap * LdsTile<PREC, PASS>::bytes);
 }
 
 // =============================================================================
@@ -333,22 +461,29 @@ __device__ __forceinline__ void pass1_segment(const KParams &P, const int *__res
   const bool fits = b.W <= kMaxSegW;
   Seg g{};
   if (fits) g = halo_setup(P, start, b.cy, b.cx0, b.W, sh);
-  const bool staged = fits && g.total <= P.lds_cap;
+  bool staged = fits && g.total <= P.lds_cap;
   LdsTile<PREC, 1> lt(dyn_lds, P.lds_cap);
+  bool fit = true;  // phases (and alpha) the staged walk's sine takes
   if (staged) {
     for (int el = threadIdx.x; el < g.total; el += kPairBlock) {
       int s = find_slot(sh, g.ns, el);
       lt.load(el, sh.gst[s] + (el - sh.off[s]), t, e);
+      if constexpr (PREC == P64) fit &= phase_fits(lt.a[el]);
     }
   }
-  __syncthreads();
+  if constexpr (PREC == P64)
+    staged = __syncthreads_and(staged && fit && phase_fits(P.alpha));
+  else
+    __syncthreads();
   // the centre slots are contiguous from the first centre cell's, k0 its slot
   // (k0 - gst) of the cell
   const int e0 = staged ? sh.off[g.ncol + 1] + (b.k0 - sh.gst[g.ncol + 1]) : 0;
   const int ncen = b.k1 - b.k0;
   const int k0 = b.k0;
+  // FP64 forms: P.lanes lanes per particle, lane 0 of them writes it
+  const int lg = PREC == P32K ? 0 : __builtin_ctz((unsigned)P.lanes), gl = threadIdx.x & ((1 << lg) - 1);
   long long cand_sum = 0, n_sum = 0, n2_sum = 0;
-  for (int p = threadIdx.x; p < ncen; p += kPairBlock) {
+  for (int p = threadIdx.x >> lg; p < ncen; p += kPairBlock >> lg) {
     const int k = k0 + p, ei = e0 + p;
     Acc acc;
     int cand;
@@ -360,11 +495,18 @@ __device__ __forceinline__ void pass1_segment(const KParams &P, const int *__res
         else hi = mid - 1;
       }
       acc.init(lt.src(), ei, k, t, P);
-      cand = visit_lds(acc, lt.src(), sh, g.ncol, lo, ei, P);
+      if constexpr (PREC == P32K)
+        cand = visit_lds(acc, lt.src(), sh, g.ncol, lo, ei, P);
+      else
+        cand = visit_lds64(acc, lt.src(), sh, g.ncol, lo, ei, gl, wraps(P, g), near_words<PREC, 1>(dyn_lds, P), P);
     } else {
       auto gs = global_src<PREC>(t, e, 1);
       acc.init(gs, k, k, t, P);
-      cand = visit_global(acc, gs, start, t.cell[k], k, P);
+      cand = visit_global(acc, gs, start, t.cell[k], k, gl, P);
+    }
+    if constexpr (PREC != P32K) {
+      acc.reduce(P.lanes);
+      if (gl) continue;  // lane 0 of the particle's lanes writes it
     }
     const int h = slot_h[k], id = slot_id[k];
     Pass1Out o{};
@@ -387,19 +529,25 @@ __device__ __forceinline__ void pass2_segment(const KParams &P, const int *__res
   const bool fits = b.W <= kMaxSegW;
   Seg g{};
   if (fits) g = halo_setup(P, start, b.cy, b.cx0, b.W, sh);
-  const bool staged = fits && g.total <= P.lds_cap;
+  bool staged = fits && g.total <= P.lds_cap;
   LdsTile<PREC, 2> lt(dyn_lds, P.lds_cap);
+  bool fit = true;  // phases (and alpha) the staged walk's sine takes
   if (staged) {
     for (int el = threadIdx.x; el < g.total; el += kPairBlock) {
       int s = find_slot(sh, g.ns, el);
       lt.load(el, sh.gst[s] + (el - sh.off[s]), t, e);
+      if constexpr (PREC == P64) fit &= phase_fits(lt.a[el]);
     }
   }
-  __syncthreads();
+  if constexpr (PREC == P64)
+    staged = __syncthreads_and(staged && fit && phase_fits(P.alpha));
+  else
+    __syncthreads();
   const int e0 = staged ? sh.off[g.ncol + 1] + (b.k0 - sh.gst[g.ncol + 1]) : 0;
   const int ncen = b.k1 - b.k0;
   const int k0 = b.k0;
-  for (int p = threadIdx.x; p < ncen; p += kPairBlock) {
+  const int lg = PREC == P32K ? 0 : __builtin_ctz((unsigned)P.lanes), gl = threadIdx.x & ((1 << lg) - 1);
+  for (int p = threadIdx.x >> lg; p < ncen; p += kPairBlock >> lg) {
     const int k = k0 + p, ei = e0 + p;
     const int h = slot_h[k], id = slot_id[k];
     Pass2In in{e.aphi_slot[k], e.n_slot[k], e.n2_slot[k], 0.0, 0.0};
@@ -416,11 +564,18 @@ __device__ __forceinline__ void pass2_segment(const KParams &P, const int *__res
         else hi = mid - 1;
       }
       acc.init(lt.src(), ei, k, t, P, in);
-      visit_lds(acc, lt.src(), sh, g.ncol, lo, ei, P);
+      if constexpr (PREC == P32K)
+        visit_lds(acc, lt.src(), sh, g.ncol, lo, ei, P);
+      else
+        visit_lds64(acc, lt.src(), sh, g.ncol, lo, ei, gl, wraps(P, g), near_words<PREC, 2>(dyn_lds, P), P);
     } else {
       auto gs = global_src<PREC>(t, e, 2);
       acc.init(gs, k, k, t, P, in);
-      visit_global(acc, gs, start, t.cell[k], k, P);
+      visit_global(acc, gs, start, t.cell[k], k, gl, P);
+    }
+    if constexpr (PREC != P32K) {
+      acc.reduce(P.lanes);
+      if (gl) continue;
     }
     Pass2Out o;
     acc.finish(P, PREC == P32K ? gp[h] : 0.0, o);

@@ -17,6 +17,8 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "spc2_device.h"
 #include "spc2_fp64_math.h"
 #include "spc2_internal.h"
@@ -77,10 +79,10 @@ __device__ __forceinline__ double vortex_dw(const KParams &P, double r) {
 
 // FP64 distance^2 of slots k and m with the reference min-image: decides the
 // rare FP32 pairs that fall inside a cutoff band.
-__device__ __forceinline__ double exact_r2(const double *tx, const double *ty, int k, int m, double Lx, double rLx,
-                                           double Ly, double rLy) {
-  double dx = min_image(tx[m] - tx[k], Lx, rLx);
-  double dy = min_image(ty[m] - ty[k], Ly, rLy);
+__device__ __forceinline__ double exact_r2(const double *tx, const double *ty, int k, int m, double Lx, double r2Lx,
+                                           double Ly, double r2Ly) {
+  double dx = min_image(tx[m] - tx[k], Lx, r2Lx);
+  double dy = min_image(ty[m] - ty[k], Ly, r2Ly);
   return dx * dx + dy * dy;
 }
 
@@ -90,8 +92,62 @@ __device__ __forceinline__ double exact_r2(const double *tx, const double *ty, i
 // beyond 1e-6 of the term.
 __device__ __forceinline__ void exact_d(const double *tx, const double *ty, int k, int m, const KParams &P, double &dx,
                                         double &dy) {
-  dx = min_image(tx[m] - tx[k], P.Lx, P.rLx);
-  dy = min_image(ty[m] - ty[k], P.Ly, P.rLy);
+  dx = min_image(tx[m] - tx[k], P.Lx, P.r2Lx);
+  dy = min_image(ty[m] - ty[k], P.Ly, P.r2Ly);
+}
+
+// FP64 squared separation of candidate m from (xi, yi): the reference min-image,
+// or with IMG = false the plain difference, the same value where no candidate of
+// the workgroup lies across the box's edge (the whole count of boxes is 0).
+template <bool IMG>
+__device__ __forceinline__ double sep2(const Src64 &s, int m, double xi, double yi, const KParams &P) {
+  double dx = s.x[m] - xi, dy = s.y[m] - yi;
+  if (IMG) {
+    dx = min_image(dx, P.Lx, P.r2Lx);
+    dy = min_image(dy, P.Ly, P.r2Ly);
+  }
+  return dx * dx + dy * dy;
+}
+
+// What a plain FP64 pass reads of a partner, so that walks can request it ahead.
+struct InP {
+  double p = 0.0;
+  __device__ __forceinline__ InP() {}
+  __device__ __forceinline__ InP(const Src64 &s, int m) : p(s.p[m]) {}
+};
+struct InPA {
+  double p = 0.0, aj = 0.0;
+  __device__ __forceinline__ InPA() {}
+  __device__ __forceinline__ InPA(const Src64 &s, int m) : p(s.p[m]), aj(s.aj[m]) {}
+};
+struct InXYP {
+  double x = 0.0, y = 0.0, p = 0.0;
+  __device__ __forceinline__ InXYP() {}
+  __device__ __forceinline__ InXYP(const Src64 &s, int m) : x(s.x[m]), y(s.y[m]), p(s.p[m]) {}
+  __device__ __forceinline__ double sep2(double xi, double yi, const KParams &P) const {
+    const double dx = min_image(x - xi, P.Lx, P.r2Lx), dy = min_image(y - yi, P.Ly, P.r2Ly);
+    return dx * dx + dy * dy;
+  }
+};
+struct InXYPA {
+  double x = 0.0, y = 0.0, p = 0.0, aj = 0.0;
+  __device__ __forceinline__ InXYPA() {}
+  __device__ __forceinline__ InXYPA(const Src64 &s, int m) : x(s.x[m]), y(s.y[m]), p(s.p[m]), aj(s.aj[m]) {}
+};
+
+// The sum over G consecutive lanes in a fixed butterfly, the same in each.
+template <int G, class T>
+__device__ __forceinline__ T lanes_sum(T v) {
+#pragma unroll
+  for (int d = 1; d < G; d <<= 1) v += __shfl_xor(v, d, 64);
+  return v;
+}
+
+// The same for a lane count known at run time (a power of two, uniform).
+template <class T>
+__device__ __forceinline__ T lanes_total(T v, int G) {
+  for (int d = 1; d < G; d <<= 1) v += __shfl_xor(v, d, 64);
+  return v;
 }
 
 // Per-particle result of pass 1.
@@ -179,7 +235,10 @@ __device__ __forceinline__ float in_vgpr(float x) {
 template <int PREC>
 struct ChimAcc;
 
-// FP64 reference form: A += sin(phi_j - phi_i - alpha) over |r_ij| <= rho
+// FP64 reference form: A += sin(phi_j - phi_i - alpha) over |r_ij| <= rho.
+// near() / term() are pair()'s two halves: the walks test candidates first and
+// take the terms two at a time, without a branch between them (two chains in
+// flight); a term that is not `on` adds zero.
 template <>
 struct ChimAcc<P64> {
   double xi, yi, pi, A;
@@ -192,14 +251,26 @@ struct ChimAcc<P64> {
     n = 0;
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
+  template <bool IMG>
+  __device__ __forceinline__ bool near(const Src64 &s, int m, const KParams &P) const {
+    return sep2<IMG>(s, m, xi, yi, P) <= P.rho2;
+  }
+  using In = InP;
+  template <bool FAST>
+  __device__ __forceinline__ bool term(const In &v, bool on, const KParams &P) {
+    const double t = sin_term<FAST>(v.p - pi - P.alpha);
+    A += on ? t : 0.0;
+    n += on;
+    return false;
+  }
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
-    double r2 = dx * dx + dy * dy;
-    if (r2 <= P.rho2) {
-      A += sin(s.p[m] - pi - P.alpha);
-      ++n;
-    }
+    if (near<true>(s, m, P)) term<false>(In(s, m), true, P);
+  }
+  __device__ __forceinline__ void cohesion(const Src64 &, int, const KParams &) {}
+  // the totals of a particle's lanes
+  __device__ __forceinline__ void reduce(int G) {
+    A = lanes_total(A, G);
+    n = lanes_total(n, G);
   }
   __device__ __forceinline__ void finish(const KParams &P, double, Pass1Out &o) const {
     o.phase = pi;
@@ -227,14 +298,19 @@ struct ChimAcc<P64F> {
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
+    double dx = min_image(s.x[m] - xi, P.Lx, P.r2Lx);
+    double dy = min_image(s.y[m] - yi, P.Ly, P.r2Ly);
     double r2 = dx * dx + dy * dy;
     if (r2 <= P.rho2) {
       S += s.s[m];
       C += s.c[m];
       ++n;
     }
+  }
+  __device__ __forceinline__ void reduce(int G) {
+    S = lanes_total(S, G);
+    C = lanes_total(C, G);
+    n = lanes_total(n, G);
   }
   __device__ __forceinline__ void finish(const KParams &P, double, Pass1Out &o) const {
     double sa, ca;
@@ -321,8 +397,8 @@ struct ChimAcc<P32K> {
     const bool ba = (r2a >= P.rho2f_lo) & ina, bb = (r2b >= P.rho2f_lo) & inb;
     if (ba | bb) {
       const int m = (int)(t2 - s.f4);
-      if (ba) ina = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy) <= P.rho2;
-      if (bb) inb = exact_r2(tx, ty, k, s.gslot(m + 1), P.Lx, P.rLx, P.Ly, P.rLy) <= P.rho2;
+      if (ba) ina = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
+      if (bb) inb = exact_r2(tx, ty, k, s.gslot(m + 1), P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
     }
     const float fa = ina ? 1.0f : 0.0f, fb = inb ? 1.0f : 0.0f;
     ps = __builtin_fmaf(fa, a.w, ps);
@@ -336,7 +412,7 @@ struct ChimAcc<P32K> {
                                          const KParams &P) {
     float r2 = __builtin_fmaf(dx, dx, dy * dy);
     bool in = r2 <= P.rho2f_hi;  // outside the band, the same as r2 <= rho2f
-    if ((r2 >= P.rho2f_lo) & in) in = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy) <= P.rho2;
+    if ((r2 >= P.rho2f_lo) & in) in = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
     if constexpr (MODE == SUM_KAHAN) {
       S.add(in ? v.w : 0.0f);
       C.add(in ? v.z : 0.0f);
@@ -378,24 +454,42 @@ struct VortAcc<P64> {
     n0 = n1 = n2 = 0;
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
+  // near(): the widest radius, with room for the root's rounding; term(): the
+  // alignment term, and whether the partner lies within xi_r, whose term
+  // cohesion() adds (one chain of its own, so that walks may add it later, in the
+  // same order: the few cohesion partners then cost their arctangent once per
+  // wavefront, not at every partner where one lane has one)
+  template <bool IMG>
+  __device__ __forceinline__ bool near(const Src64 &s, int m, const KParams &P) const {
+    return sep2<IMG>(s, m, xi, yi, P) <= P.outer2 * 1.000000000001;
+  }
+  using In = InXYP;
+  template <bool FAST>
+  __device__ __forceinline__ bool term(const In &v, bool on, const KParams &P) {
+    const double dr = sqrt_sep(v.sep2(xi, yi, P));
+    const bool in = on & (dr <= P.xi_a), an = on & !in & (dr <= P.rho);
+    const double t = vortex_w(P, dr) * sin_term<FAST>(v.p - pi);
+    A += in ? t : 0.0;
+    B += an ? t : 0.0;
+    n0 += in;
+    n1 += an;
+    return on & (dr <= P.xi_r);
+  }
+  __device__ __forceinline__ void cohesion(const Src64 &s, int m, const KParams &P) {
+    const double dx = min_image(s.x[m] - xi, P.Lx, P.r2Lx), dy = min_image(s.y[m] - yi, P.Ly, P.r2Ly);
+    Cc += -P.kappa * sin_term(atan2(dy, dx) - pi);
+    ++n2;
+  }
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
-    double r2 = dx * dx + dy * dy;
-    if (r2 > P.outer2 * 1.000000000001) return;  // cannot pass the sqrt tests below
-    double dr = sqrt(r2);
-    double pj = s.p[m];
-    if (dr <= P.xi_a) {
-      A += vortex_w(P, dr) * sin(pj - pi);
-      ++n0;
-    } else if (dr <= P.rho) {
-      B += vortex_w(P, dr) * sin(pj - pi);
-      ++n1;
-    }
-    if (dr <= P.xi_r) {
-      Cc += -P.kappa * sin(atan2(dy, dx) - pi);
-      ++n2;
-    }
+    if (near<true>(s, m, P) && term<false>(In(s, m), true, P)) cohesion(s, m, P);
+  }
+  __device__ __forceinline__ void reduce(int G) {
+    A = lanes_total(A, G);
+    B = lanes_total(B, G);
+    Cc = lanes_total(Cc, G);
+    n0 = lanes_total(n0, G);
+    n1 = lanes_total(n1, G);
+    n2 = lanes_total(n2, G);
   }
   __device__ __forceinline__ void finish(const KParams &, double, Pass1Out &o) const {
     o.phase = pi;
@@ -431,11 +525,11 @@ struct VortAcc<P64F> {
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
+    double dx = min_image(s.x[m] - xi, P.Lx, P.r2Lx);
+    double dy = min_image(s.y[m] - yi, P.Ly, P.r2Ly);
     double r2 = dx * dx + dy * dy;
     if (r2 > P.outer2 * 1.000000000001) return;
-    double dr = sqrt(r2);
+    double dr = sqrt_sep(r2);
     if (dr <= P.rho) {
       double w = vortex_w(P, dr);
       SW += w * s.s[m];
@@ -451,6 +545,14 @@ struct VortAcc<P64F> {
       }
       ++n2;
     }
+  }
+  __device__ __forceinline__ void reduce(int G) {
+    SW = lanes_total(SW, G);
+    CW = lanes_total(CW, G);
+    Tx = lanes_total(Tx, G);
+    Ty = lanes_total(Ty, G);
+    n01 = lanes_total(n01, G);
+    n2 = lanes_total(n2, G);
   }
   __device__ __forceinline__ void finish(const KParams &P, double, Pass1Out &o) const {
     double sp, cp;
@@ -549,7 +651,7 @@ struct VortAcc<P32K> {
     return (r2 >= P.rho2f_lo) & inr;
   }
   __device__ __forceinline__ bool rho_exact(const Src32 &s, int m, const KParams &P) const {
-    return sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy)) <= P.rho;
+    return sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly)) <= P.rho;
   }
   template <int MODE>
   __device__ __forceinline__ void term(const float4 &v, float r2, bool inr, const KParams &P) {
@@ -571,8 +673,8 @@ struct VortAcc<P32K> {
     const bool ba = (r2a >= P.rho2f_lo) & ina, bb = (r2b >= P.rho2f_lo) & inb;
     if (ba | bb) {
       const int m = (int)(t2 - s.f4);
-      if (ba) ina = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy)) <= P.rho;
-      if (bb) inb = sqrt(exact_r2(tx, ty, k, s.gslot(m + 1), P.Lx, P.rLx, P.Ly, P.rLy)) <= P.rho;
+      if (ba) ina = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly)) <= P.rho;
+      if (bb) inb = sqrt(exact_r2(tx, ty, k, s.gslot(m + 1), P.Lx, P.r2Lx, P.Ly, P.r2Ly)) <= P.rho;
     }
     const float wa = weight(r2a, ina, P), wb = weight(r2b, inb, P);
     psw = __builtin_fmaf(wa, a.w, psw);
@@ -595,7 +697,7 @@ struct VortAcc<P32K> {
     // r2 <= rho2 - band); inside it the reference's FP64 test sqrt(r^2) <= rho
     // does (VortexArraysSystemPtr.cpp:473-488).
     bool inr = r2 <= P.rho2f_hi;
-    if ((r2 >= P.rho2f_lo) & inr) inr = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy)) <= P.rho;
+    if ((r2 >= P.rho2f_lo) & inr) inr = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly)) <= P.rho;
     float r = __builtin_amdgcn_sqrtf(r2);
     float w_in = __builtin_fmaf(-P.mu_p_over_xa2f, r2, mu_pv);
     // c4 (r - xi_a)(rho - r) in Horner form (two FMAs; the same FP32 error bound)
@@ -621,7 +723,7 @@ struct VortAcc<P32K> {
   // decided as for rho.
   __device__ __forceinline__ void cohesion(const Src32 &s, int m, float dx, float dy, float r2, const KParams &P) {
     bool inc = r2 <= P.xr2f;
-    if (r2 >= P.xr2f - P.band_xr2f) inc = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy)) <= P.xi_r;
+    if (r2 >= P.xr2f - P.band_xr2f) inc = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly)) <= P.xi_r;
     if (inc) {
       if (r2 >= P.close2f) {
         float ir = __builtin_amdgcn_rsqf(r2);
@@ -684,32 +786,44 @@ struct Chim2Acc;
 
 template <>
 struct Chim2Acc<P64> {
-  double xi, yi, pi, ai, n, a0, a1;
+  double xi, yi, pi, ai, n, in0, in1, a0, a1;  // a0, a1: the sums, divided by n once
   __device__ __forceinline__ void init(const Src64 &s, int e, int, const Tiles &, const KParams &, const Pass2In &in) {
     xi = s.x[e];
     yi = s.y[e];
     pi = s.p[e];
     ai = in.ai;
     n = in.n;
-    a0 = in.in0;
-    a1 = in.in1;
+    in0 = in.in0;
+    in1 = in.in1;
+    a0 = a1 = 0.0;
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
+  template <bool IMG>
+  __device__ __forceinline__ bool near(const Src64 &s, int m, const KParams &P) const {
+    return sep2<IMG>(s, m, xi, yi, P) <= P.rho2;
+  }
+  using In = InPA;
+  template <bool FAST>
+  __device__ __forceinline__ bool term(const In &v, bool on, const KParams &P) {
+    const double c = cos_term<FAST>(v.p - pi - P.alpha), cph = on ? c : 0.0;
+    a0 += cph;
+    a1 = __builtin_fma(v.aj - ai, cph, a1);
+    return false;
+  }
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
-    double r2 = dx * dx + dy * dy;
-    if ((r2 <= P.rho2) && (n != 0)) {
-      double cph = cos(s.p[m] - pi - P.alpha);
-      a0 += cph / n;
-      a1 += (s.aj[m] - ai) * cph / n;
-    }
+    if (near<true>(s, m, P)) term<false>(In(s, m), true, P);
+  }
+  __device__ __forceinline__ void cohesion(const Src64 &, int, const KParams &) {}
+  __device__ __forceinline__ void reduce(int G) {
+    a0 = lanes_total(a0, G);
+    a1 = lanes_total(a1, G);
   }
   __device__ __forceinline__ void finish(const KParams &P, double, Pass2Out &o) const {
     o.phase = pi;
     o.ai = ai;
-    o.a0 = a0 * -sqrt(2.0 * P.D);
-    o.a1 = a1 + -2.0 * P.D * ai;
+    const bool any = n != 0.0;
+    o.a0 = (any ? in0 + a0 / n : in0) * -sqrt(2.0 * P.D);
+    o.a1 = (any ? in1 + a1 / n : in1) + -2.0 * P.D * ai;
   }
 };
 
@@ -728,8 +842,8 @@ struct Chim2Acc<P64F> {
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
+    double dx = min_image(s.x[m] - xi, P.Lx, P.r2Lx);
+    double dy = min_image(s.y[m] - yi, P.Ly, P.r2Ly);
     double r2 = dx * dx + dy * dy;
     if (r2 <= P.rho2) {
       double aj = s.aj[m];
@@ -738,6 +852,12 @@ struct Chim2Acc<P64F> {
       Pc += aj * s.c[m];
       Qs += aj * s.s[m];
     }
+  }
+  __device__ __forceinline__ void reduce(int G) {
+    C = lanes_total(C, G);
+    S = lanes_total(S, G);
+    Pc = lanes_total(Pc, G);
+    Qs = lanes_total(Qs, G);
   }
   __device__ __forceinline__ void finish(const KParams &P, double, Pass2Out &o) const {
     double sa, ca;
@@ -799,7 +919,7 @@ struct Chim2Acc<P32K> {
     float dx = v.x + ox, dy = v.y + co.oy;
     float r2 = __builtin_fmaf(dx, dx, dy * dy);
     bool in = r2 <= P.rho2f_hi;  // outside the band, the same as r2 <= rho2f
-    if ((r2 >= P.rho2f_lo) & in) in = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy) <= P.rho2;
+    if ((r2 >= P.rho2f_lo) & in) in = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
     sum<MODE>(v, in, in ? s.aj[m] : 0.0f);
   }
   // the cell walks' partial sums over one stencil cell start at zero
@@ -811,7 +931,7 @@ struct Chim2Acc<P32K> {
     float dx = v.x + co.cdx(fx, P.hxf), dy = v.y - co.yf;
     float r2 = __builtin_fmaf(dx, dx, dy * dy);
     bool in = r2 <= P.rho2f_hi;  // outside the band, the same as r2 <= rho2f
-    if ((r2 >= P.rho2f_lo) & in) in = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy) <= P.rho2;
+    if ((r2 >= P.rho2f_lo) & in) in = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
     sum<MODE>(v, in, ajv);  // aj multiplies cos, sin terms that are zero outside rho
   }
   // a list entry with pass 1's rho decision: v = (cos, sin, aj, 0) of the partner
@@ -842,8 +962,8 @@ struct Chim2Acc<P32K> {
     bool ina = r2a <= P.rho2f_hi, inb = r2b <= P.rho2f_hi;
     const bool ba = (r2a >= P.rho2f_lo) & ina, bb = (r2b >= P.rho2f_lo) & inb;
     if (ba | bb) {
-      if (ba) ina = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy) <= P.rho2;
-      if (bb) inb = exact_r2(tx, ty, k, s.gslot(m + 1), P.Lx, P.rLx, P.Ly, P.rLy) <= P.rho2;
+      if (ba) ina = exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
+      if (bb) inb = exact_r2(tx, ty, k, s.gslot(m + 1), P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
     }
     const float fa = ina ? 1.0f : 0.0f, fb = inb ? 1.0f : 0.0f;
     const float ga = fa * s.aj[m], gb = fb * s.aj[m + 1];
@@ -900,53 +1020,67 @@ struct Vort2Acc;
 // FP64 reference form
 template <>
 struct Vort2Acc<P64> {
-  double xi, yi, pi, vxi, vyi, ai, n1, n2, a0, a1;
+  double xi, yi, pi, vxi, vyi, ai, n1, n2, in0, in1;
+  double a0, a1;  // the alignment sums, divided by n1 once
+  double c0, c1;  // the cohesion terms, a chain of their own (VortAcc<P64>)
   __device__ __forceinline__ void init(const Src64 &s, int e, int, const Tiles &, const KParams &P, const Pass2In &in) {
     xi = s.x[e];
     yi = s.y[e];
     pi = s.p[e];
-    vxi = P.v0 * cos(pi);
-    vyi = P.v0 * sin(pi);
+    vxi = P.v0 * cos_term(pi);
+    vyi = P.v0 * sin_term(pi);
     ai = in.ai;
     n1 = in.n;
     n2 = in.n2;
-    a0 = in.in0;
-    a1 = in.in1;
+    in0 = in.in0;
+    in1 = in.in1;
+    a0 = a1 = c0 = c1 = 0.0;
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
+  template <bool IMG>
+  __device__ __forceinline__ bool near(const Src64 &s, int m, const KParams &P) const {
+    return sep2<IMG>(s, m, xi, yi, P) <= P.outer2 * 1.000000000001;
+  }
+  using In = InXYPA;
+  template <bool FAST>
+  __device__ __forceinline__ bool term(const In &v, bool on, const KParams &P) {
+    const double dx = min_image(v.x - xi, P.Lx, P.r2Lx), dy = min_image(v.y - yi, P.Ly, P.r2Ly);
+    const double dr = sqrt_sep(dx * dx + dy * dy), rdr = 1.0 / dr;
+    const double pj = v.p;
+    const double vxj = P.v0 * cos_term<FAST>(pj), vyj = P.v0 * sin_term<FAST>(pj);
+    const double cph = cos_term<FAST>(pj - pi), sph = sin_term<FAST>(pj - pi);
+    const double w = vortex_w(P, dr), dw = vortex_dw(P, dr);
+    const bool al = on & (dr <= P.rho) & (n1 > 0.0);
+    const double g = div_by((vxj - vxi) * dw * dx, dr, rdr) + div_by((vyj - vyi) * dw * dy, dr, rdr);
+    a0 += al ? -w * cph : 0.0;
+    a1 += al ? g * sph + (v.aj - ai) * w * cph - 2.0 * P.D * sph * w : 0.0;
+    return on & (dr <= P.xi_r) & (n2 > 0.0);
+  }
+  __device__ __forceinline__ void cohesion(const Src64 &s, int m, const KParams &P) {
+    const double dx = min_image(s.x[m] - xi, P.Lx, P.r2Lx), dy = min_image(s.y[m] - yi, P.Ly, P.r2Ly);
+    const double dr = sqrt(dx * dx + dy * dy), pj = s.p[m];
+    const double vxj = P.v0 * cos_term(pj), vyj = P.v0 * sin_term(pj);
+    const double th = atan2(dy, dx);
+    const double cpp = cos_term(th - pi), spp = sin_term(th - pi);
+    c0 += P.kappa * cpp / n2;
+    c1 += -P.kappa * ((vxj - vxi) * (-dy) / dr / dr + (vyj - vyi) * dx / dr / dr - ai) * cpp / n2 +
+          P.kappa * P.D * spp / n2;
+  }
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
-    double r2 = dx * dx + dy * dy;
-    if (r2 > P.outer2 * 1.000000000001) return;
-    double dr = sqrt(r2);
-    const bool al = (dr <= P.rho) && (n1 > 0.0), co = (dr <= P.xi_r) && (n2 > 0.0);
-    if (!al && !co) return;
-    const double pj = s.p[m];
-    const double vxj = P.v0 * cos(pj), vyj = P.v0 * sin(pj);
-    if (al) {
-      double cph = cos(pj - pi);
-      double sph = sin(pj - pi);
-      double w = vortex_w(P, dr);
-      double dw = vortex_dw(P, dr);
-      a0 += -w * cph / n1;
-      a1 += ((vxj - vxi) * dw * dx / dr + (vyj - vyi) * dw * dy / dr) * sph / n1 + (s.aj[m] - ai) * w * cph / n1 -
-            2.0 * P.D * sph * w / n1;
-    }
-    if (co) {
-      double th = atan2(dy, dx);
-      double cpp = cos(th - pi);
-      double spp = sin(th - pi);
-      a0 += P.kappa * cpp / n2;
-      a1 += -P.kappa * ((vxj - vxi) * (-dy) / dr / dr + (vyj - vyi) * dx / dr / dr - ai) * cpp / n2 +
-            P.kappa * P.D * spp / n2;
-    }
+    if (near<true>(s, m, P) && term<false>(In(s, m), true, P)) cohesion(s, m, P);
+  }
+  __device__ __forceinline__ void reduce(int G) {
+    a0 = lanes_total(a0, G);
+    a1 = lanes_total(a1, G);
+    c0 = lanes_total(c0, G);
+    c1 = lanes_total(c1, G);
   }
   __device__ __forceinline__ void finish(const KParams &P, double, Pass2Out &o) const {
     o.phase = pi;
     o.ai = ai;
-    o.a0 = a0 * sqrt(2.0 * P.D);
-    o.a1 = a1;
+    const bool any = n1 > 0.0;
+    o.a0 = (in0 + ((any ? a0 / n1 : 0.0) + c0)) * sqrt(2.0 * P.D);
+    o.a1 = in1 + ((any ? a1 / n1 : 0.0) + c1);
   }
 };
 
@@ -971,11 +1105,11 @@ struct Vort2Acc<P64F> {
   }
   __device__ __forceinline__ void row(int, int, int, const KParams &) {}
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
-    double dx = min_image(s.x[m] - xi, P.Lx, P.rLx);
-    double dy = min_image(s.y[m] - yi, P.Ly, P.rLy);
+    double dx = min_image(s.x[m] - xi, P.Lx, P.r2Lx);
+    double dy = min_image(s.y[m] - yi, P.Ly, P.r2Ly);
     double r2 = dx * dx + dy * dy;
     if (r2 > P.outer2 * 1.000000000001) return;
-    double dr = sqrt(r2);
+    double dr = sqrt_sep(r2);
     const bool al = dr <= P.rho, co = dr <= P.xi_r;
     if (!al && !co) return;
     const double cj = s.c[m], sj = s.s[m];
@@ -995,6 +1129,12 @@ struct Vort2Acc<P64F> {
       C0 += cpp;
       C1 += -P.kappa * ((dvy * dx - dvx * dy) / r2 - ai) * cpp + P.kappa * P.D * spp;
     }
+  }
+  __device__ __forceinline__ void reduce(int G) {
+    A0 = lanes_total(A0, G);
+    A1 = lanes_total(A1, G);
+    C0 = lanes_total(C0, G);
+    C1 = lanes_total(C1, G);
   }
   __device__ __forceinline__ void finish(const KParams &P, double, Pass2Out &o) const {
     double a0 = in0, a1 = in1;
@@ -1074,7 +1214,7 @@ struct Vort2Acc<P32K> {
     bool inr = r2 <= P.rho2f, inc = r2 <= P.xr2f, inner = r2 < P.xa2f;
     if ((__builtin_fabsf(r2 - P.rho2f) <= P.band_rho2f) | (__builtin_fabsf(r2 - P.xr2f) <= P.band_xr2f) |
         (__builtin_fabsf(r2 - P.xa2f) <= P.band_xa2f)) {
-      double d = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.rLx, P.Ly, P.rLy));
+      double d = sqrt(exact_r2(tx, ty, k, s.gslot(m), P.Lx, P.r2Lx, P.Ly, P.r2Ly));
       inr = d <= P.rho;
       inc = d <= P.xi_r;
       inner = d < P.xi_a;
@@ -1127,6 +1267,37 @@ struct Vort2Acc<P32K> {
     o.ai = ai;
     o.a0 = a0 * sqrt(2.0 * P.D);
     o.a1 = a1;
+  }
+};
+
+// Accumulators whose pair() comes in two halves, near() and term().
+template <class Acc>
+struct HasNear : std::false_type {};
+template <>
+struct HasNear<ChimAcc<P64>> : std::true_type {};
+template <>
+struct HasNear<VortAcc<P64>> : std::true_type {};
+template <>
+struct HasNear<Chim2Acc<P64>> : std::true_type {};
+template <>
+struct HasNear<Vort2Acc<P64>> : std::true_type {};
+
+// A lane's cohesion partners waiting for their terms: up to four 16-bit LDS
+// indices in two registers, summed in the order they came.
+struct CohQueue64 {
+  static constexpr int kFull = 4;
+  uint64_t q = 0;
+  int n = 0;
+  __device__ __forceinline__ void push(int m) {
+    q = (q << 16) | (uint32_t)m;
+    ++n;
+  }
+  template <class Acc>
+  __device__ __forceinline__ void drain(Acc &acc, const Src64 &s, const KParams &P) {
+    while (n > 0) {
+      --n;
+      acc.cohesion(s, (int)((q >> (16 * n)) & 0xffffu), P);
+    }
   }
 };
 
@@ -1431,17 +1602,6 @@ void launch_pair(Sim &s, void (*kern)(KArgs...), dim3 grid, dim3 blk, size_t sh,
 // loop by four raises the registers (149 to 157 and 67 to 96) and is 8% slower.
 constexpr int kApLanes = 64;
 
-__device__ __forceinline__ double group_sum(double v) {
-#pragma unroll
-  for (int d = 1; d < kApLanes; d <<= 1) v += __shfl_xor(v, d, kApLanes);
-  return v;
-}
-__device__ __forceinline__ int group_sum(int v) {
-#pragma unroll
-  for (int d = 1; d < kApLanes; d <<= 1) v += __shfl_xor(v, d, kApLanes);
-  return v;
-}
-
 // Pass 1 of particle i by lane g of its wavefront (every lane calls it): stage
 // positions not wrapped (ChimeraSystem.cpp:131-167, :184-254); arrays by
 // particle id; FP64 geometry in every precision form.  tiles (the FP32 chimera
@@ -1466,8 +1626,8 @@ __device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, int g, c
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = PREC == P32K ? 0.0 : gp[j];
       const float4 tj = PREC == P32K ? tiles[j] : float4{};
-      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       if ((r2 <= P.rho2) & (j != i)) {
         if constexpr (PREC == P64) {
@@ -1486,12 +1646,12 @@ __device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, int g, c
       S = Sf.value();
       C = Cf.value();
     }
-    n = group_sum(n);
-    double A = group_sum(S);
+    n = lanes_sum<kApLanes>(n);
+    double A = lanes_sum<kApLanes>(S);
     if constexpr (PREC != P64) {
       double sa, ca;
       sincos(pi + P.alpha, &sa, &ca);
-      A = ca * A - sa * group_sum(C);
+      A = ca * A - sa * lanes_sum<kApLanes>(C);
     }
     o.n = n;
     o.written = n != 0;
@@ -1502,8 +1662,8 @@ __device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, int g, c
 #pragma unroll 1
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = gp[j];
-      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       // (partners beyond both radii cannot pass the tests of the root below)
       if ((r2 > P.outer2 * 1.000000000001) | (j == i)) continue;
@@ -1526,12 +1686,12 @@ __device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, int g, c
         ++n2;
       }
     }
-    n0 = group_sum(n0);
-    n1 = group_sum(n1);
-    n2 = group_sum(n2);
-    A = group_sum(A);
-    B = group_sum(B);
-    Cc = group_sum(Cc);
+    n0 = lanes_sum<kApLanes>(n0);
+    n1 = lanes_sum<kApLanes>(n1);
+    n2 = lanes_sum<kApLanes>(n2);
+    A = lanes_sum<kApLanes>(A);
+    B = lanes_sum<kApLanes>(B);
+    Cc = lanes_sum<kApLanes>(Cc);
     o.n = n0 + n1;
     o.n2 = n2;
     if (n0 + n1 > 0) {
@@ -1566,8 +1726,8 @@ __device__ __forceinline__ void allpairs_pass2(const KParams &P, int i, int g, c
 #pragma unroll 1
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = gp[j], aj = aphi[j];
-      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       if ((r2 > P.outer2 * 1.000000000001) | (j == i)) continue;
       const double dr = sqrt_sep(r2);
@@ -1589,16 +1749,16 @@ __device__ __forceinline__ void allpairs_pass2(const KParams &P, int i, int g, c
               P.kappa * P.D * spp / n2;
       }
     }
-    o.a0 = (in0 + group_sum(s0)) * sqrt(2.0 * P.D);
-    o.a1 = in1 + group_sum(s1);
+    o.a0 = (in0 + lanes_sum<kApLanes>(s0)) * sqrt(2.0 * P.D);
+    o.a1 = in1 + lanes_sum<kApLanes>(s1);
   } else {
     // ChimeraSystem.cpp:223-254
     const double rn = 1.0 / n;
 #pragma unroll 1
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = gp[j], aj = aphi[j];
-      const double dx = min_image(gx[j] - xi, P.Lx, P.rLx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.rLy);
+      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       if ((r2 <= P.rho2) & (n != 0) & (j != i)) {
         const double cph = cos_term(pj - pi - P.alpha);
@@ -1606,8 +1766,8 @@ __device__ __forceinline__ void allpairs_pass2(const KParams &P, int i, int g, c
         s1 += div_by((aj - ai) * cph, n, rn);
       }
     }
-    o.a0 = (in0 + group_sum(s0)) * -sqrt(2.0 * P.D);
-    o.a1 = (in1 + group_sum(s1)) + -2.0 * P.D * ai;
+    o.a0 = (in0 + lanes_sum<kApLanes>(s0)) * -sqrt(2.0 * P.D);
+    o.a1 = (in1 + lanes_sum<kApLanes>(s1)) + -2.0 * P.D * ai;
   }
 }
 

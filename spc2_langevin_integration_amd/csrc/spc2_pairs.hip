@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kBlock) void k_pass2_allpairs(KParams P, const doub
 
 template <int PREC, int PASS>
 size_t lds_bytes(const Sim &s) {
-  return (size_t)s.kp.lds_cap * LdsTile<PREC, PASS>::bytes;
+  return (size_t)s.kp.lds_cap * LdsTile<PREC, PASS>::bytes + lds_near_bytes(PREC);
 }
 
 template <int PREC, int SYS, int EPI>
@@ -151,10 +151,19 @@ void pass2_sys(Sim &s, int epi, const EpiCtx &e) {
     pass2_epi<PREC, SPC2_VORTEX>(s, epi, e);
 }
 
+constexpr int kLanes64 = 2;
+constexpr long long kLanesFill = 131072;
+
 }  // namespace
 
-// The pair workgroups of a linked system: about `target` particles each and an
-// LDS capacity for their halo.
+// The pair workgroups of a linked system: about `target` lanes each and an LDS
+// capacity for their halo.
+// * The FP64 forms split each particle's candidates over `lanes` lanes: enough
+//   for kLanesFill lanes in all (two wavefronts on each of the 1024 SIMDs), at
+//   most 16, so that small systems fill the device; the plain form at least
+//   kLanes64, whose halved workgroups leave room for its words of bits.  The
+//   count depends on the system alone, so that a batch's replica sums as a single
+//   handle does.
 // * Rows of at least kChunkPerCell particles per cell are cut into chunks of
 //   `target` slots rounded to whole wavefronts, so that every wavefront but a
 //   row's last is full.  A row gets workgroups for its mean count plus four
@@ -165,17 +174,24 @@ void pass2_sys(Sim &s, int epi, const EpiCtx &e) {
 // whose halo exceeds it reads the same tiles from global memory.
 void configure_segments_kp(KParams &k, int prec, double target) {
   k.chunk = 0;
+  k.lanes = 1;
   if (!k.linked) {
     k.seg_w = k.segs = 1;
     k.lds_cap = 0;
     return;
   }
+  if (prec != P32K) {
+    const int least = prec == P64 ? kLanes64 : 1;
+    while (k.lanes < least || (k.lanes < 16 && (long long)k.n * k.lanes < kLanesFill)) k.lanes *= 2;
+  }
+  target /= k.lanes;  // particles per workgroup
   const double per_cell = (double)k.n / ((double)k.nx * (double)k.ny);
   double halo;
   if (per_cell >= kChunkPerCell) {
-    int chunk = 64 * std::max(1, (int)std::lround(target / 64.0));
+    const int unit = 64 / k.lanes;  // a wavefront's particles
+    int chunk = unit * std::max(1, (int)std::lround(target / unit));
     // at most kMaxSegW - 3 cells' worth, so a chunk's columns fit the halo tables
-    chunk = std::min(chunk, 64 * std::max(1, (int)std::floor((kMaxSegW - 3) * per_cell / 64.0)));
+    chunk = std::min(chunk, unit * std::max(1, (int)std::floor((kMaxSegW - 3) * per_cell / unit)));
     const double row = (double)k.n / (double)k.ny;
     k.chunk = chunk;
     k.segs = std::max(1, (int)std::ceil((row + 4.0 * std::sqrt(row) + 8.0) / chunk));
@@ -189,10 +205,12 @@ void configure_segments_kp(KParams &k, int prec, double target) {
     halo = 1.6 * 3.0 * (w + 2) * per_cell;
   }
   int cap = (int)std::ceil((halo + 160.0) / 64.0) * 64;
-  cap = std::min(cap, kLdsBytes / lds_elem_bytes(prec));
+  cap = std::min(cap, (kLdsBytes - lds_near_bytes(prec)) / lds_elem_bytes(prec));
   if (const char *env = std::getenv("SPC2_LDS_CAP")) cap = std::max(0, std::min(cap, std::atoi(env)));
   k.lds_cap = cap;
 }
+
+int lds_near_bytes(int prec) { return prec == P64 ? (int)sizeof(NearWords) : 0; }
 
 int lds_elem_bytes(int prec) {
   switch (prec) {

@@ -107,8 +107,8 @@ __device__ __forceinline__ void for_each_build_candidate(const KParams &P, const
         const int e = start[jc + 1];
 #pragma unroll 2
         for (int j = start[jc]; j < e; ++j) {
-          double dx = min_image(t.x[j] - xi, P.Lx, P.rLx);
-          double dy = min_image(t.y[j] - yi, P.Ly, P.rLy);
+          double dx = min_image(t.x[j] - xi, P.Lx, P.r2Lx);
+          double dy = min_image(t.y[j] - yi, P.Ly, P.r2Ly);
           f(j, code, (dx * dx + dy * dy <= rlist2) & (j != i));
         }
       }
@@ -1164,9 +1164,10 @@ constexpr size_t lds_pass64_bytes(int cap) {
 }
 
 template <int PREC, int PASS>
-__device__ __forceinline__ Src64 stage_halo64(const int *start, const int *bh_nrun, const int *bh_run,
-                                              const int *bh_off, int seg, const Tiles &t, const EpiCtx &e,
-                                              void *dyn, int cap, LdsTail **tail) {
+__device__ __forceinline__ Src64 stage_halo64(const KParams &P, const int *start, const int *bh_nrun,
+                                              const int *bh_run, const int *bh_off, int seg, const Tiles &t,
+                                              const EpiCtx &e, void *dyn, LdsTail **tail, bool &fit) {
+  const int cap = P.lds_cap;
   LdsTile<PREC, PASS> lt(dyn, cap);
   LdsTail *tl = (LdsTail *)((char *)dyn + (size_t)cap * LdsTile<PREC, PASS>::bytes);
   *tail = tl;
@@ -1178,24 +1179,49 @@ __device__ __forceinline__ Src64 stage_halo64(const int *start, const int *bh_nr
   }
   __syncthreads();
   const int nrun = tl->n, total = tl->off[nrun];
+  bool ok = true;  // every phase (and alpha) one that the fast sine takes (the plain form)
   for (int el = threadIdx.x; el < total; el += kBlock) {
     int k = 0;
     while (k + 1 < nrun && tl->off[k + 1] <= el) ++k;
     lt.load(el, tl->gst[k] + (el - tl->off[k]), t, e);
+    if constexpr (PREC == P64) ok &= phase_fits(lt.a[el]);
   }
-  __syncthreads();
+  fit = __syncthreads_and(ok && phase_fits(P.alpha));
   return lt.src();
 }
 
-// FP64 walk over an LDS list: the entries below the count, in list order.
-template <class Acc>
+// FP64 walk over an LDS list: the entries below the count, in list order.  The
+// plain form takes two entries at a time, their terms masked by the distance
+// test instead of branching on it (most entries pass: 31 of 45 in the vortex
+// workload), so that two chains of dependent FP64 instructions are in flight;
+// cohesion partners wait in a queue, emptied when it may overflow and after the
+// last entry.
+template <bool FAST, class Acc>
 __device__ __forceinline__ void walk64_lds(Acc &acc, const Src64 &src, const int4 *l, int cnt, const KParams &P) {
-  for (int q = 0; q < cnt; q += 8) {
-    const int4 g = l[(size_t)(q >> 3) * 64];
-    const uint32_t w[4] = {(uint32_t)g.x, (uint32_t)g.y, (uint32_t)g.z, (uint32_t)g.w};
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (q + u < cnt) acc.pair(src, EntLds::index((u & 1) ? w[u >> 1] >> 16 : w[u >> 1] & 0xffffu), P);
+  CohQueue64 cq;
+  uint64_t lo = 0, hi = 0;
+#pragma unroll 1
+  for (int q = 0; q < cnt; q += 2) {
+    if ((q & 7) == 0) {
+      const int4 g = l[(size_t)(q >> 3) * 64];
+      lo = (uint64_t)(uint32_t)g.y << 32 | (uint32_t)g.x;
+      hi = (uint64_t)(uint32_t)g.w << 32 | (uint32_t)g.z;
+    }
+    const bool two = q + 1 < cnt;
+    const int m0 = EntLds::index((uint32_t)lo & 0xffffu), m1 = two ? EntLds::index((uint32_t)lo >> 16) : m0;
+    lo = lo >> 32 | hi << 32;
+    hi >>= 32;
+    if constexpr (HasNear<Acc>::value) {
+      using In = typename Acc::In;
+      const bool q0 = acc.template term<FAST>(In(src, m0), acc.template near<true>(src, m0, P), P);
+      const bool q1 = acc.template term<FAST>(In(src, m1), two & acc.template near<true>(src, m1, P), P);
+      if (q0) cq.push(m0);
+      if (q1) cq.push(m1);
+      if (cq.n > CohQueue64::kFull - 2 || q + 2 >= cnt) cq.drain(acc, src, P);
+    } else {
+      acc.pair(src, m0, P);
+      if (two) acc.pair(src, m1, P);
+    }
   }
 }
 
@@ -1212,7 +1238,8 @@ __global__ __launch_bounds__(kBlock) void k_pass1_verlet_lds64(KParams P, const 
   extern __shared__ double dyn_lds64[];
   const int seg = xcd_segment(blockIdx.x, gridDim.x);
   LdsTail *tl;
-  const Src64 src = stage_halo64<PREC, 1>(start, bh_nrun, bh_run, bh_off, seg, t, e, dyn_lds64, P.lds_cap, &tl);
+  bool fit;
+  const Src64 src = stage_halo64<PREC, 1>(P, start, bh_nrun, bh_run, bh_off, seg, t, e, dyn_lds64, &tl, fit);
   const int slot = seg * kBlock + threadIdx.x;
   const bool active = slot < P.n;
   Pass1Out o{};
@@ -1222,7 +1249,9 @@ __global__ __launch_bounds__(kBlock) void k_pass1_verlet_lds64(KParams P, const 
     Acc acc;
     acc.init(verlet_src<PREC>(t, e, 1), i, i, t, P);
     cnt = vcnt[i];
-    walk64_lds(acc, src, (const int4 *)vlist + (size_t)wrow[slot >> 6] * 64 + (slot & 63), cnt, P);
+    const int4 *l = (const int4 *)vlist + (size_t)wrow[slot >> 6] * 64 + (slot & 63);
+    if (fit) walk64_lds<true>(acc, src, l, cnt, P);
+    else walk64_lds<false>(acc, src, l, cnt, P);
     acc.finish(P, 0.0, o);
     const EpiState r = epilogue1<EPI>(P, e, i, hid[i], i, o);
     if (EPI == EPI_K && e.next == 1) {
@@ -1247,7 +1276,8 @@ __global__ __launch_bounds__(kBlock) void k_pass2_verlet_lds64(KParams P, const 
   extern __shared__ double dyn_lds64[];
   const int seg = xcd_segment(blockIdx.x, gridDim.x);
   LdsTail *tl;
-  const Src64 src = stage_halo64<PREC, 2>(start, bh_nrun, bh_run, bh_off, seg, t, e, dyn_lds64, P.lds_cap, &tl);
+  bool fit;
+  const Src64 src = stage_halo64<PREC, 2>(P, start, bh_nrun, bh_run, bh_off, seg, t, e, dyn_lds64, &tl, fit);
   const int slot = seg * kBlock + threadIdx.x;
   if (slot >= P.n) return;
   const int i = vslot ? vslot[slot] : slot;
@@ -1258,7 +1288,9 @@ __global__ __launch_bounds__(kBlock) void k_pass2_verlet_lds64(KParams P, const 
   }
   Acc acc;
   acc.init(verlet_src<PREC>(t, e, 2), i, i, t, P, in);
-  walk64_lds(acc, src, (const int4 *)vlist + (size_t)wrow[slot >> 6] * 64 + (slot & 63), vcnt[i], P);
+  const int4 *l = (const int4 *)vlist + (size_t)wrow[slot >> 6] * 64 + (slot & 63);
+  if (fit) walk64_lds<true>(acc, src, l, vcnt[i], P);
+  else walk64_lds<false>(acc, src, l, vcnt[i], P);
   Pass2Out o;
   acc.finish(P, 0.0, o);
   const EpiState r = epilogue2<EPI>(P, e, i, hid[i], o);
@@ -1272,7 +1304,7 @@ __global__ __launch_bounds__(kBlock) void k_drift_partial(KParams P, const doubl
   __shared__ double sm[kBlock];
   double m = 0.0;
   for (int h = blockIdx.x * blockDim.x + threadIdx.x; h < P.n; h += gridDim.x * blockDim.x) {
-    double dx = min_image(sx[h] - xb[h], P.Lx, P.rLx), dy = min_image(sy[h] - yb[h], P.Ly, P.rLy);
+    double dx = min_image(sx[h] - xb[h], P.Lx, P.r2Lx), dy = min_image(sy[h] - yb[h], P.Ly, P.r2Ly);
     m = fmax(m, dx * dx + dy * dy);
   }
   sm[threadIdx.x] = m;
