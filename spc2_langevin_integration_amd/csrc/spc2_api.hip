@@ -67,7 +67,7 @@ void free_all(Sim &s) {
   for (auto &p : s.io) f(p);
   f(s.t.x); f(s.t.y); f(s.t.p); f(s.t.c); f(s.t.s); f(s.t.f4); f(s.t.cell);
   f(s.t2.x); f(s.t2.y); f(s.t2.p); f(s.t2.c); f(s.t2.s); f(s.t2.f4); f(s.gp2);
-  f(s.aphi_slot); f(s.n_slot); f(s.n2_slot); f(s.aphi_slot_f);
+  f(s.aphi_slot); f(s.n_slot); f(s.n2_slot); f(s.aphi_slot_f); f(s.aq);
   f(s.noise); f(s.counts); f(s.red); f(s.bsum); f(s.snap);
   f(s.vcnt); f(s.wmax); f(s.wrow); f(s.vlist); f(s.xb); f(s.yb); f(s.vmask);
   f(s.bh_nrun); f(s.bh_run); f(s.bh_off); f(s.bh_max); f(s.vslot); f(s.wmax_s); f(s.wrow_s);
@@ -197,6 +197,7 @@ spc2_status alloc_all(Sim &s) {
     s.t2.cell = s.t.cell;
   }
   A(s.aphi_slot, n); A(s.n_slot, n); A(s.n2_slot, n); A(s.aphi_slot_f, n);
+  if (s.kp.mfma) A(s.aq, n);
   A(s.counts, 3 * kCountSlots); A(s.red, 2 * 1024 + 8);
   A(s.bsum, (size_t)scan_blocks(std::max({s.nc, s.nw, 1})) + 1);
   if (s.verlet) {

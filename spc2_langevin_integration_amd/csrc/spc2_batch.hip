@@ -29,6 +29,7 @@
 #include <string>
 #include <vector>
 
+#include "spc2_chimera_mfma.h"
 #include "spc2_lds_stencil.h"
 
 using namespace spc2;
@@ -116,8 +117,9 @@ __global__ __launch_bounds__(kB) void k_b_rank_tiles(int n, const Rep *reps, con
     const int cx = lc % R.kp.nx, cy = lc / R.kp.nx;
     double sn, cs;
     sincos(p, &sn, &cs);
-    t.f4[dst] = make_float4((float)(x - (double)cx * R.kp.hx), (float)(y - (double)cy * R.kp.hy), (float)cs,
-                            (float)sn);
+    t.f4[dst] = make_float4((float)(x - (double)cx * R.kp.hx), (float)(y - (double)cy * R.kp.hy),
+                            R.kp.mfma ? __uint_as_float(pack_fixed(cs)) : (float)cs,
+                            R.kp.mfma ? __uint_as_float(pack_fixed(sn)) : (float)sn);
   } else {
     t.p[dst] = p;
     if (PREC == P64F) {
@@ -218,10 +220,11 @@ __global__ __launch_bounds__(kB) void k_b_pass2_ap_vortex(const Rep *reps, const
 // Pass 1 over every row segment of every linked replica: pair sums and the SE
 // update (EPI_SE), or the SRK step's Ito intermediates by slot (EPI_ITO1).
 template <int PREC, int EPI>
-__global__ __launch_bounds__(kB) void k_b_pass1(const Rep *reps, const int *seg_rep, const int *start, Tiles t,
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(PREC == P32K ? 3 : 1))) void k_b_pass1(const Rep *reps, const int *seg_rep, const int *start, Tiles t,
                                                 const int *slot_h, const int *slot_id, const double *gx,
                                                 const double *gy, const double *gp, EpiCtx e, int k, ApBlocks ap) {
   extern __shared__ float4 dyn_lds[];
+  __shared__ SegShared sh;
   if ((int)blockIdx.x < ap.pad) {
     if ((int)blockIdx.x < ap.n) b_allpairs1<PREC, SPC2_CHIMERA, EPI>(reps, ap.rep, blockIdx.x, gx, gy, gp, t.f4, e, k);
     return;
@@ -231,21 +234,26 @@ __global__ __launch_bounds__(kB) void k_b_pass1(const Rep *reps, const int *seg_
   if (k >= R.steps) return;  // the whole workgroup: the replica is done in this call
   const KParams P = R.kp;
   const EpiCtx c = rep_ctx(e, R, k);
+  if constexpr (PREC == P32K) {
+    if (P.mfma) {
+      mfma_segment<1, EPI>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
+      return;
+    }
+  }
   if (R.system == SPC2_CHIMERA)
-    pass1_segment<ChimAcc<PREC>, PREC, EPI>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff,
-                                            dyn_lds);
+    pass1_segment<ChimAcc<PREC>, PREC, EPI>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
   else
-    pass1_segment<VortAcc<PREC>, PREC, EPI>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff,
-                                            dyn_lds);
+    pass1_segment<VortAcc<PREC>, PREC, EPI>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
 }
 
 // Pass 2 of the SRK step over every row segment of every linked replica.
 template <int PREC>
-__global__ __launch_bounds__(kB) void k_b_pass2_srk(const Rep *reps, const int *seg_rep, const int *start, Tiles t,
+__global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(PREC == P32K ? 3 : 1))) void k_b_pass2_srk(const Rep *reps, const int *seg_rep, const int *start, Tiles t,
                                                     const int *slot_h, const int *slot_id, const double *gx,
                                                     const double *gy, const double *gp, EpiCtx e, int k,
                                                     ApBlocks ap) {
   extern __shared__ float4 dyn_lds[];
+  __shared__ SegShared sh;
   if ((int)blockIdx.x < ap.pad) {
     if ((int)blockIdx.x < ap.n) b_allpairs2_srk<SPC2_CHIMERA>(reps, ap.rep, blockIdx.x, gx, gy, gp, e, k);
     return;
@@ -255,10 +263,16 @@ __global__ __launch_bounds__(kB) void k_b_pass2_srk(const Rep *reps, const int *
   if (k >= R.steps) return;
   const KParams P = R.kp;
   const EpiCtx c = rep_ctx(e, R, k);
+  if constexpr (PREC == P32K) {
+    if (P.mfma) {
+      mfma_segment<2, EPI_SRK>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
+      return;
+    }
+  }
   if (R.system == SPC2_CHIMERA)
-    pass2_segment<Chim2Acc<PREC>, PREC, EPI_SRK>(P, start + R.coff, t, slot_h, slot_id, gp, c, sg - R.soff, dyn_lds);
+    pass2_segment<Chim2Acc<PREC>, PREC, EPI_SRK>(P, start + R.coff, t, slot_h, slot_id, gp, c, sg - R.soff, sh, dyn_lds);
   else
-    pass2_segment<Vort2Acc<PREC>, PREC, EPI_SRK>(P, start + R.coff, t, slot_h, slot_id, gp, c, sg - R.soff, dyn_lds);
+    pass2_segment<Vort2Acc<PREC>, PREC, EPI_SRK>(P, start + R.coff, t, slot_h, slot_id, gp, c, sg - R.soff, sh, dyn_lds);
 }
 
 // Re-homing of the SE arrays (x, y, phi, omega): slot k becomes home k.
@@ -392,10 +406,11 @@ struct spc2_batch {
   // the SRK step's Ito intermediates by slot (allocated at the first SRK step)
   double *aphi_slot = nullptr, *n_slot = nullptr, *n2_slot = nullptr;
   float *aphi_slot_f = nullptr;
+  uint2 *aq = nullptr;
   float *snap = nullptr;
   hipEvent_t snap_ev = nullptr;
   bool snap_pending = false;
-  size_t lds = 0;
+  size_t lds[2] = {};  // dynamic LDS of the pass-1 and pass-2 launches
   int since_rehome = 0;
 };
 
@@ -423,7 +438,7 @@ void bfree(spc2_batch &b) {
   f(b.hid); f(b.hpos); f(b.spare_i); f(b.bsum);
   f(b.t.x); f(b.t.y); f(b.t.p); f(b.t.c); f(b.t.s); f(b.t.f4); f(b.t.cell);
   f(b.io); f(b.red); f(b.snap);
-  f(b.aphi_slot); f(b.n_slot); f(b.n2_slot); f(b.aphi_slot_f);
+  f(b.aphi_slot); f(b.n_slot); f(b.n2_slot); f(b.aphi_slot_f); f(b.aq);
   if (b.snap_ev) (void)hipEventDestroy(b.snap_ev);
   if (b.stream) (void)hipStreamDestroy(b.stream);
 }
@@ -439,7 +454,7 @@ spc2_status check_launch(const char *what) {
 spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &ap_rep) {
   int poff = 0, coff = 0, soff = 0;
   std::vector<int> ap_vortex;
-  size_t lds_cap = 0;
+  b.lds[0] = b.lds[1] = 0;
   seg_rep.clear();
   ap_rep.clear();
   for (int r = 0; r < b.count; ++r) {
@@ -450,7 +465,7 @@ spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &a
     if (spc2_status st = cell_grid(p, linked, nx, ny)) return st;
     std::memset((void *)&R.kp, 0, sizeof(R.kp));
     fill_kparams_from(R.kp, p, (int)p.n, nx, ny, linked);
-    configure_segments_kp(R.kp, b.prec, b.target[r]);
+    configure_segments_kp(R.kp, b.prec, p.system, b.target[r]);
     R.system = p.system;
     R.poff = poff;
     R.n = (int)p.n;
@@ -463,7 +478,7 @@ spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &a
       for (int q = 0; q < R.nseg; ++q) seg_rep.push_back(r);
       soff += R.nseg;
       coff += nx * ny;
-      lds_cap = std::max(lds_cap, (size_t)R.kp.lds_cap);
+      for (int q = 0; q < 2; ++q) b.lds[q] = std::max(b.lds[q], pair_lds_bytes(R.kp, b.prec, q + 1));
     } else {
       R.soff = R.nseg = 0;
       std::vector<int> &list = p.system == SPC2_CHIMERA ? ap_rep : ap_vortex;
@@ -480,7 +495,6 @@ spc2_status layout(spc2_batch &b, std::vector<int> &seg_rep, std::vector<int> &a
   b.nap = (int)ap_rep.size();
   b.napv = (int)ap_vortex.size();
   ap_rep.insert(ap_rep.end(), ap_vortex.begin(), ap_vortex.end());
-  b.lds = lds_cap * (size_t)lds_elem_bytes(b.prec) + (size_t)lds_near_bytes(b.prec);
   return SPC2_OK;
 }
 
@@ -582,7 +596,7 @@ void launch_step_kernels(spc2_batch &b, const EpiCtx &e, int k, bool srk, bool s
                          (const Rep *)b.d_reps, ap_vortex, (const double *)b.gx, (const double *)b.gy,
                          (const double *)b.gp, es, k);
     if (gpass.x == 0) return;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1<PREC, EPI_SE>), gpass, blk, b.lds, b.stream, (const Rep *)b.d_reps,
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1<PREC, EPI_SE>), gpass, blk, b.lds[0], b.stream, (const Rep *)b.d_reps,
                        (const int *)b.seg_rep, (const int *)b.start, b.t, (const int *)b.slot_h,
                        (const int *)b.slot_id, (const double *)b.gx, (const double *)b.gy, (const double *)b.gp, es,
                        k, ap);
@@ -600,11 +614,11 @@ void launch_step_kernels(spc2_batch &b, const EpiCtx &e, int k, bool srk, bool s
                        (const double *)b.gx, (const double *)b.gy, (const double *)b.gp, es, k);
   }
   if (gpass.x == 0) return;
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1<PREC, EPI_ITO1>), gpass, blk, b.lds, b.stream, (const Rep *)b.d_reps,
+  hipLaunchKernelGGL(HIP_KERNEL_NAME(k_b_pass1<PREC, EPI_ITO1>), gpass, blk, b.lds[0], b.stream, (const Rep *)b.d_reps,
                      (const int *)b.seg_rep, (const int *)b.start, b.t, (const int *)b.slot_h,
                      (const int *)b.slot_id, (const double *)b.gx, (const double *)b.gy, (const double *)b.gp, e1, k,
                      ap);
-  hipLaunchKernelGGL(k_b_pass2_srk<PREC>, gpass, blk, b.lds, b.stream, (const Rep *)b.d_reps, (const int *)b.seg_rep,
+  hipLaunchKernelGGL(k_b_pass2_srk<PREC>, gpass, blk, b.lds[1], b.stream, (const Rep *)b.d_reps, (const int *)b.seg_rep,
                      (const int *)b.start, b.t, (const int *)b.slot_h, (const int *)b.slot_id, (const double *)b.gx,
                      (const double *)b.gy, (const double *)b.gp, es, k, ap);
 }
@@ -628,6 +642,7 @@ spc2_status run_steps(spc2_batch &b, int method, double dt, int64_t nsteps, cons
     B_TRY(balloc(&b.n_slot, n));
     B_TRY(balloc(&b.n2_slot, n));
     B_TRY(balloc(&b.aphi_slot_f, n));
+    B_TRY(balloc(&b.aq, n));
   }
   int64_t kmax = 0, kmin = std::numeric_limits<int64_t>::max();
   for (int r = 0; r < b.count; ++r) {
@@ -651,6 +666,7 @@ spc2_status run_steps(spc2_batch &b, int method, double dt, int64_t nsteps, cons
   e.sa.sqrt3 = std::sqrt(3.0);
   e.aphi_slot = b.aphi_slot;
   e.aphi_slot_f = b.aphi_slot_f;
+  e.aq = b.aq;
   e.n_slot = b.n_slot;
   e.n2_slot = b.n2_slot;
   bool staged = false;
@@ -707,7 +723,7 @@ uint64_t spc2_batch_footprint(const spc2_params *p) {
   const size_t cells = cell_grid(*p, linked, nx, ny) == SPC2_OK ? (size_t)nx * (size_t)ny : 1;
   const size_t tile = p->precision == SPC2_FP32_KAHAN ? 16 + 16 : (p->precision == SPC2_FP64 ? 24 : 40);
   // 11 doubles (state, omega, stage, spare), 11 ints, tiles; 2 ints per cell
-  // (SE stepping; the first SRK step adds 28 B per particle)
+  // (SE stepping; the first SRK step adds 36 B per particle)
   return n * (11 * 8 + 11 * 4 + tile) + cells * 8 + sizeof(Rep) + 64;
 }
 

@@ -184,7 +184,7 @@ __global__ __launch_bounds__(kBlock) void k_place(int n, const int *cell_of, con
 // the reference's ascending push_back order (ChimeraSystem.cpp:335-338).  The
 // same thread gathers the particle's stage data into the cell-sorted tiles.
 template <int PREC>
-__global__ __launch_bounds__(kBlock) void k_rank_tiles(int n, int nx, double hx, double hy, const int *tmp,
+__global__ __launch_bounds__(kBlock) void k_rank_tiles(int n, int nx, int fixed, double hx, double hy, const int *tmp,
                                                        const int *tmpid, const int *cell_of, const int *start,
                                                        const double *gx, const double *gy, const double *gp,
                                                        int *slot_h, int *slot_id, Tiles t) {
@@ -211,7 +211,10 @@ __global__ __launch_bounds__(kBlock) void k_rank_tiles(int n, int nx, double hx,
     int cx = c % nx, cy = c / nx;
     double sn, cs;
     sincos(p, &sn, &cs);
-    t.f4[dst] = make_float4((float)(x - (double)cx * hx), (float)(y - (double)cy * hy), (float)cs, (float)sn);
+    // fixed: cos and sin as the matrix-core passes' packed features
+    t.f4[dst] = make_float4((float)(x - (double)cx * hx), (float)(y - (double)cy * hy),
+                            fixed ? __uint_as_float(pack_fixed(cs)) : (float)cs,
+                            fixed ? __uint_as_float(pack_fixed(sn)) : (float)sn);
     t.x[dst] = x;
     t.y[dst] = y;
   } else {
@@ -266,15 +269,15 @@ void launch_rank_tiles(Sim &s) {
   dim3 g(blocks_for(s.n)), b(kBlock);
   switch (s.prec) {
     case P64:
-      hipLaunchKernelGGL(k_rank_tiles<P64>, g, b, 0, s.stream, s.n, s.nx, s.kp.hx, s.kp.hy, s.tmp, s.tmpid,
+      hipLaunchKernelGGL(k_rank_tiles<P64>, g, b, 0, s.stream, s.n, s.nx, s.kp.mfma, s.kp.hx, s.kp.hy, s.tmp, s.tmpid,
                          s.cell_of, s.start, s.gx, s.gy, s.gp, s.slot_h, s.slot_id, s.t);
       break;
     case P64F:
-      hipLaunchKernelGGL(k_rank_tiles<P64F>, g, b, 0, s.stream, s.n, s.nx, s.kp.hx, s.kp.hy, s.tmp, s.tmpid,
+      hipLaunchKernelGGL(k_rank_tiles<P64F>, g, b, 0, s.stream, s.n, s.nx, s.kp.mfma, s.kp.hx, s.kp.hy, s.tmp, s.tmpid,
                          s.cell_of, s.start, s.gx, s.gy, s.gp, s.slot_h, s.slot_id, s.t);
       break;
     default:
-      hipLaunchKernelGGL(k_rank_tiles<P32K>, g, b, 0, s.stream, s.n, s.nx, s.kp.hx, s.kp.hy, s.tmp, s.tmpid,
+      hipLaunchKernelGGL(k_rank_tiles<P32K>, g, b, 0, s.stream, s.n, s.nx, s.kp.mfma, s.kp.hx, s.kp.hy, s.tmp, s.tmpid,
                          s.cell_of, s.start, s.gx, s.gy, s.gp, s.slot_h, s.slot_id, s.t);
   }
 }

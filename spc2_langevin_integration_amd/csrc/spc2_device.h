@@ -83,6 +83,24 @@ __device__ __forceinline__ int rank_in_cell(const int *a, int cnt, int id) {
   return r;
 }
 
+// ---- fixed-point features of the matrix-core chimera passes ------------------
+// v in [-1, 1] to the nearest multiple of 2^-27, as four signed base-128 digits,
+// the lowest in byte 0 (bytes 0-2 in [-64, 63], byte 3 in [-64, 64]); kFixedOdd
+// for a value that is not finite.
+constexpr double kFixedUnit = 0x1.0p-27;
+constexpr uint32_t kFixedOdd = 0x80000000u;
+__device__ __forceinline__ uint32_t pack_fixed(double v) {
+  if (!(__builtin_fabs(v) <= 1.0)) return kFixedOdd;
+  const int q0 = (int)__builtin_rint(v * (1.0 / kFixedUnit));
+  const int q1 = (q0 + 64) >> 7, q2 = (q1 + 64) >> 7, q3 = (q2 + 64) >> 7;
+  return (uint32_t)((q0 - (q1 << 7)) & 255) | (uint32_t)((q1 - (q2 << 7)) & 255) << 8 |
+         (uint32_t)((q2 - (q3 << 7)) & 255) << 16 | (uint32_t)q3 << 24;
+}
+__device__ __forceinline__ int unpack_fixed(uint32_t p) {
+  const int d0 = (int)(int8_t)p, d1 = (int)(int8_t)(p >> 8), d2 = (int)(int8_t)(p >> 16), d3 = (int)p >> 24;
+  return (((d3 * 128 + d2) * 128 + d1) * 128) + d0;
+}
+
 // ---- Kahan-compensated FP32 sum ----------------------------------------------
 
 struct Kahan {
@@ -241,29 +259,31 @@ __device__ __forceinline__ void uniform_pair(uint64_t seed, uint64_t step, uint3
 
 // Histogram increment with one atomic per distinct cell per wavefront: lanes
 // holding the same cell take consecutive arrival ranks from a single
-// atomicAdd issued by the lowest such lane.  Every lane of the wavefront takes
-// part (valid == false for lanes past the end).
+// atomicAdd issued by the lowest such lane.  The cells are told apart first and
+// the atomics issued together, so that a wavefront waits for one of them and not
+// for each in turn.  Every lane of the wavefront takes part (valid == false for
+// lanes past the end).
 __device__ __forceinline__ int wave_aggregated_rank(int *count, int c, bool valid) {
   const int lane = threadIdx.x & 63;
   const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int leader = lane;               // the lowest lane of this lane's cell
+  unsigned long long mates = 0ull;  // the lanes of its cell
   bool done = !valid;
-  int rank = 0;
   while (true) {
-    unsigned long long pending = __ballot(!done);
+    const unsigned long long pending = __ballot(!done);
     if (pending == 0ull) break;
-    const int leader = __builtin_ctzll(pending);
-    const int lc = __shfl(c, leader, 64);
-    const bool mine = !done && c == lc;
+    const int first = __builtin_ctzll(pending);
+    const bool mine = !done && c == __shfl(c, first, 64);
     const unsigned long long same = __ballot(mine);
-    int base = 0;
-    if (lane == leader) base = atomicAdd(&count[lc], __popcll(same));
-    base = __shfl(base, leader, 64);
     if (mine) {
-      rank = base + __popcll(same & below);
+      leader = first;
+      mates = same;
       done = true;
     }
   }
-  return rank;
+  int base = 0;
+  if (valid && lane == leader) base = atomicAdd(&count[c], __popcll(mates));
+  return __shfl(base, leader, 64) + __popcll(mates & below);
 }
 
 }  // namespace spc2

@@ -56,6 +56,8 @@ struct KParams {
   // row) or, with chunk 0, row segments of seg_w cells; LDS capacity in tile
   // elements per workgroup
   int seg_w, segs, lds_cap, chunk;
+  int mfma;   // dense FP32 chimera cells: the matrix-core passes (spc2_chimera_mfma.h)
+  double aj, raj;  // their scale of pass 2's a_j, a power of two >= |a_j|, and its reciprocal
   int lanes;  // lanes per centre particle of the FP64 cell walks (a power of two; 1 in the FP32 form)
 };
 
@@ -123,6 +125,7 @@ struct Sim {
   // pass-1 results kept per slot for pass 2
   double *aphi_slot = nullptr, *n_slot = nullptr, *n2_slot = nullptr;
   float *aphi_slot_f = nullptr;
+  uint2 *aq = nullptr;  // matrix-core passes: packed a_j cos, a_j sin by slot
   // materialised noise (optional)
   double *noise = nullptr;
   size_t noise_cap = 0;
@@ -228,9 +231,8 @@ void launch_rank_tiles(Sim &s);
 // spc2_pairs.hip
 constexpr double kSegTarget = 256.0;  // default particles per pair workgroup (row chunk or segment)
 constexpr int kLdsBytes = 60 * 1024;  // dynamic LDS of one pair workgroup at most
-int lds_elem_bytes(int prec);
-int lds_near_bytes(int prec);
-void configure_segments_kp(KParams &k, int prec, double target);
+size_t pair_lds_bytes(const KParams &k, int prec, int pass);  // of one linked pair workgroup
+void configure_segments_kp(KParams &k, int prec, int system, double target);
 void configure_segments(Sim &s);
 void launch_pass1(Sim &s, int epi, double *ox, double *oy, double *op, const StepArgs &sa, double *const k1[3],
                   double *const k2[3], double *const k3[3]);

@@ -454,8 +454,7 @@ template <class Acc, int PREC, int EPI>
 __device__ __forceinline__ void pass1_segment(const KParams &P, const int *__restrict__ start, const Tiles &t,
                                               const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                               const double *gp, const EpiCtx &e, unsigned long long *counts, int seg,
-                                              void *dyn_lds) {
-  __shared__ SegShared sh;
+                                              SegShared &sh, void *dyn_lds) {
   Block b;
   if (!block_range(P, start, t, seg, b)) return;  // the whole workgroup
   const bool fits = b.W <= kMaxSegW;
@@ -522,8 +521,7 @@ __device__ __forceinline__ void pass1_segment(const KParams &P, const int *__res
 template <class Acc, int PREC, int EPI>
 __device__ __forceinline__ void pass2_segment(const KParams &P, const int *__restrict__ start, const Tiles &t,
                                               const int *__restrict__ slot_h, const int *__restrict__ slot_id,
-                                              const double *gp, const EpiCtx &e, int seg, void *dyn_lds) {
-  __shared__ SegShared sh;
+                                              const double *gp, const EpiCtx &e, int seg, SegShared &sh, void *dyn_lds) {
   Block b;
   if (!block_range(P, start, t, seg, b)) return;
   const bool fits = b.W <= kMaxSegW;

@@ -1313,6 +1313,7 @@ struct EpiCtx {
   double *aphi_slot, *n_slot;     // pass-1 results by slot (pass-2 inputs)
   double *n2_slot;                // vortex cohesion partner counts by slot
   float *aphi_slot_f;
+  uint2 *aq;                      // matrix-core passes: pass 2's features a_j cos, a_j sin by slot (packed)
   double *a0, *a1;                // additional by particle (in/out)
   StepArgs sa;
   // Verlet passes: the next stage's tiles, written by the pass-1 epilogue
@@ -1569,6 +1570,7 @@ inline EpiCtx make_ctx(Sim &s, double *ox, double *oy, double *op, const StepArg
   e.n_slot = s.n_slot;
   e.n2_slot = s.n2_slot;
   e.aphi_slot_f = s.aphi_slot_f;
+  e.aq = s.aq;
   e.a0 = s.add[0];
   e.a1 = s.add[1];
   e.sa = sa;

@@ -5,10 +5,12 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "spc2_device.h"
 #include "spc2_internal.h"
+#include "spc2_chimera_mfma.h"
 #include "spc2_lds_stencil.h"
 
 namespace spc2 {
@@ -28,8 +30,9 @@ __global__ __launch_bounds__(kBlock) void k_pass1_lds(KParams P, const int *__re
                                                       const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                                       const double *gp, EpiCtx e, unsigned long long *counts) {
   extern __shared__ float4 dyn_lds[];
+  __shared__ SegShared sh;
   pass1_segment<Acc, PREC, EPI>(P, start, t, slot_h, slot_id, gp, e, counts, xcd_segment(blockIdx.x, gridDim.x),
-                                dyn_lds);
+                                sh, dyn_lds);
 }
 
 template <class Acc, int PREC, int EPI>
@@ -37,7 +40,27 @@ __global__ __launch_bounds__(kBlock) void k_pass2_lds(KParams P, const int *__re
                                                       const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                                       const double *gp, EpiCtx e) {
   extern __shared__ float4 dyn_lds[];
-  pass2_segment<Acc, PREC, EPI>(P, start, t, slot_h, slot_id, gp, e, xcd_segment(blockIdx.x, gridDim.x), dyn_lds);
+  __shared__ SegShared sh;
+  pass2_segment<Acc, PREC, EPI>(P, start, t, slot_h, slot_id, gp, e, xcd_segment(blockIdx.x, gridDim.x), sh, dyn_lds);
+}
+
+// The matrix-core passes of dense FP32 chimera cells.
+template <int EPI>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_pass1_mfma(KParams P, const int *__restrict__ start, Tiles t,
+                                                       const int *__restrict__ slot_h, const int *__restrict__ slot_id,
+                                                       const double *gp, EpiCtx e, unsigned long long *counts) {
+  extern __shared__ float4 dyn_lds[];
+  __shared__ SegShared sh;
+  mfma_segment<1, EPI>(P, start, t, slot_h, slot_id, gp, e, counts, xcd_segment(blockIdx.x, gridDim.x), sh, dyn_lds);
+}
+
+template <int EPI>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_pass2_mfma(KParams P, const int *__restrict__ start, Tiles t,
+                                                       const int *__restrict__ slot_h, const int *__restrict__ slot_id,
+                                                       const double *gp, EpiCtx e) {
+  extern __shared__ float4 dyn_lds[];
+  __shared__ SegShared sh;
+  mfma_segment<2, EPI>(P, start, t, slot_h, slot_id, gp, e, nullptr, xcd_segment(blockIdx.x, gridDim.x), sh, dyn_lds);
 }
 
 // =============================================================================
@@ -74,17 +97,19 @@ __global__ __launch_bounds__(kBlock) void k_pass2_allpairs(KParams P, const doub
 // dispatch
 // =============================================================================
 
-template <int PREC, int PASS>
-size_t lds_bytes(const Sim &s) {
-  return (size_t)s.kp.lds_cap * LdsTile<PREC, PASS>::bytes + lds_near_bytes(PREC);
-}
-
 template <int PREC, int SYS, int EPI>
 void pass1_typed(Sim &s, const EpiCtx &e) {
   unsigned long long *cnt = s.counting ? s.counts : nullptr;
   if (s.linked) {
     const dim3 grid(s.ny * s.kp.segs), blk(kBlock);
-    const size_t sh = lds_bytes<PREC, 1>(s);
+    const size_t sh = pair_lds_bytes(s.kp, PREC, 1);
+    if constexpr (PREC == P32K && SYS == SPC2_CHIMERA) {
+      if (s.kp.mfma) {
+        launch_pair(s, k_pass1_mfma<EPI>, grid, blk, sh, s.kp, (const int *)s.start, s.t, (const int *)s.slot_h,
+                    (const int *)s.slot_id, (const double *)s.gp, e, cnt);
+        return;
+      }
+    }
     if (SYS == SPC2_CHIMERA)
       launch_pair(s, k_pass1_lds<ChimAcc<PREC>, PREC, EPI>, grid, blk, sh, s.kp, (const int *)s.start, s.t,
                   (const int *)s.slot_h, (const int *)s.slot_id, (const double *)s.gp, e, cnt);
@@ -121,8 +146,15 @@ void pass1_sys(Sim &s, int epi, const EpiCtx &e) {
 template <int PREC, int SYS, int EPI>
 void pass2_typed(Sim &s, const EpiCtx &e) {
   if (s.linked) {
-    const size_t sh = lds_bytes<PREC, 2>(s);
+    const size_t sh = pair_lds_bytes(s.kp, PREC, 2);
     const dim3 grid(s.ny * s.kp.segs), blk(kBlock);
+    if constexpr (PREC == P32K && SYS == SPC2_CHIMERA) {
+      if (s.kp.mfma) {
+        launch_pair(s, k_pass2_mfma<EPI>, grid, blk, sh, s.kp, (const int *)s.start, s.t, (const int *)s.slot_h,
+                    (const int *)s.slot_id, (const double *)s.gp, e);
+        return;
+      }
+    }
     if (SYS == SPC2_CHIMERA)
       launch_pair(s, k_pass2_lds<Chim2Acc<PREC>, PREC, EPI>, grid, blk, sh, s.kp, (const int *)s.start, s.t,
                   (const int *)s.slot_h, (const int *)s.slot_id, (const double *)s.gp, e);
@@ -153,6 +185,18 @@ void pass2_sys(Sim &s, int epi, const EpiCtx &e) {
 
 constexpr int kLanes64 = 2;
 constexpr long long kLanesFill = 131072;
+constexpr double kMfmaPerCell = 12.0;
+
+int lds_near_bytes(int prec) { return prec == P64 ? (int)sizeof(NearWords) : 0; }
+
+// bytes per staged candidate of the larger pass
+int lds_elem_bytes(int prec) {
+  switch (prec) {
+    case P32K: return LdsTile<P32K, 2>::bytes;
+    case P64: return LdsTile<P64, 2>::bytes;
+    default: return LdsTile<P64F, 2>::bytes;
+  }
+}
 
 }  // namespace
 
@@ -172,9 +216,13 @@ constexpr long long kLanesFill = 131072;
 //   particle counts follow the cells.
 // The LDS capacity is the mean halo with a margin, within 60 KB; a workgroup
 // whose halo exceeds it reads the same tiles from global memory.
-void configure_segments_kp(KParams &k, int prec, double target) {
+// * The FP32 chimera form of rows with at least kMfmaPerCell particles per cell
+//   takes the matrix-core passes, whose LDS holds whole tiles.
+void configure_segments_kp(KParams &k, int prec, int system, double target) {
   k.chunk = 0;
   k.lanes = 1;
+  k.mfma = 0;
+  k.aj = k.raj = 1.0;
   if (!k.linked) {
     k.seg_w = k.segs = 1;
     k.lds_cap = 0;
@@ -197,6 +245,14 @@ void configure_segments_kp(KParams &k, int prec, double target) {
     k.segs = std::max(1, (int)std::ceil((row + 4.0 * std::sqrt(row) + 8.0) / chunk));
     k.seg_w = std::min(k.nx, (int)std::ceil(chunk / per_cell) + 1);
     halo = 1.25 * 3.0 * (chunk + 3.0 * per_cell);  // chunk's cells, a partial cell at each end, and the sides
+    if (prec == P32K && system == SPC2_CHIMERA && per_cell >= kMfmaPerCell) {
+      k.mfma = 1;
+      k.chunk = std::min(chunk, kMfmaWindow);
+      k.segs = std::max(1, (int)std::ceil((row + 4.0 * std::sqrt(row) + 8.0) / k.chunk));
+      // |a_j| <= |sigma|: sigma times a mean of sines
+      k.aj = std::exp2(std::ceil(std::log2(std::max(std::fabs(k.sigma) * 1.0001, 1e-200))));
+      k.raj = 1.0 / k.aj;
+    }
   } else {
     int w = (int)std::floor(target / std::max(per_cell, 1e-9));
     w = std::max(1, std::min({w, kMaxSegW, k.nx}));
@@ -204,23 +260,31 @@ void configure_segments_kp(KParams &k, int prec, double target) {
     k.segs = (k.nx + w - 1) / w;
     halo = 1.6 * 3.0 * (w + 2) * per_cell;
   }
-  int cap = (int)std::ceil((halo + 160.0) / 64.0) * 64;
-  cap = std::min(cap, (kLdsBytes - lds_near_bytes(prec)) / lds_elem_bytes(prec));
-  if (const char *env = std::getenv("SPC2_LDS_CAP")) cap = std::max(0, std::min(cap, std::atoi(env)));
-  k.lds_cap = cap;
-}
-
-int lds_near_bytes(int prec) { return prec == P64 ? (int)sizeof(NearWords) : 0; }
-
-int lds_elem_bytes(int prec) {
-  switch (prec) {
-    case P32K: return LdsTile<P32K, 2>::bytes;
-    case P64: return LdsTile<P64, 2>::bytes;
-    default: return LdsTile<P64F, 2>::bytes;
+  int cap;
+  if (k.mfma) {
+    cap = (int)std::ceil((halo + 128.0) / kMfmaTile) * kMfmaTile;  // the rows' padding and the far tile
+    cap = std::min(cap, (kLdsBytes - MfmaLds<2>::tail_bytes) / MfmaLds<2>::tile_bytes * kMfmaTile);
+  } else {
+    cap = (int)std::ceil((halo + 160.0) / 64.0) * 64;
+    cap = std::min(cap, (kLdsBytes - lds_near_bytes(prec)) / lds_elem_bytes(prec));
   }
+  if (const char *env = std::getenv("SPC2_LDS_CAP")) cap = std::max(0, std::min(cap, std::atoi(env)));
+  k.lds_cap = k.mfma ? cap / kMfmaTile * kMfmaTile : cap;
 }
 
-void configure_segments(Sim &s) { configure_segments_kp(s.kp, s.prec, kSegTarget); }
+size_t pair_lds_bytes(const KParams &k, int prec, int pass) {
+  if (!k.linked) return 0;
+  if (k.mfma) return (size_t)(pass == 1 ? MfmaLds<1>::bytes(k.lds_cap) : MfmaLds<2>::bytes(k.lds_cap));
+  int elem;
+  switch (prec) {
+    case P32K: elem = pass == 1 ? LdsTile<P32K, 1>::bytes : LdsTile<P32K, 2>::bytes; break;
+    case P64: elem = pass == 1 ? LdsTile<P64, 1>::bytes : LdsTile<P64, 2>::bytes; break;
+    default: elem = pass == 1 ? LdsTile<P64F, 1>::bytes : LdsTile<P64F, 2>::bytes;
+  }
+  return (size_t)k.lds_cap * (size_t)elem + (size_t)lds_near_bytes(prec);
+}
+
+void configure_segments(Sim &s) { configure_segments_kp(s.kp, s.prec, s.P.system, kSegTarget); }
 
 void launch_pass1(Sim &s, int epi, double *ox, double *oy, double *op, const StepArgs &sa, double *const k1[3],
                   double *const k2[3], double *const k3[3]) {
