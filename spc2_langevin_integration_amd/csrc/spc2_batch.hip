@@ -59,7 +59,7 @@ struct Rep {
 // K1: stage (the state itself for SE) and binning into the replica's cells.
 __global__ __launch_bounds__(kB) void k_b_stage_bin(int n, const Rep *reps, const int *rep_of, const double *sx,
                                                     const double *sy, const double *sp, double *gx, double *gy,
-                                                    double *gp, int *cell_of, int *count, int *local) {
+                                                    double *gp, Bins bins) {
   const int h = blockIdx.x * kB + threadIdx.x;
   const bool valid = h < n;
   int c = 0;
@@ -73,13 +73,12 @@ __global__ __launch_bounds__(kB) void k_b_stage_bin(int n, const Rep *reps, cons
       lc = cell_coord(y, b.Ly, R.kp.ny) * R.kp.nx + cell_coord(x, b.Lx, R.kp.nx);
     }
     c = R.coff + lc;
-    cell_of[h] = c;
+    bins.cell_of[h] = c;
     gx[h] = x;
     gy[h] = y;
     gp[h] = sp[h];
   }
-  const int r = wave_aggregated_rank(count, c, valid);
-  if (valid) local[h] = r;
+  bin_particle(bins, c, 0, h, 0, valid);
 }
 
 // K3b: stable counting sort (rank by particle id inside the cell) and the
@@ -410,8 +409,10 @@ struct spc2_batch {
   float *snap = nullptr;
   hipEvent_t snap_ev = nullptr;
   bool snap_pending = false;
+  Bins bins() const { return Bins{cell_of, count_, nullptr, nullptr, local}; }
   size_t lds[2] = {};  // dynamic LDS of the pass-1 and pass-2 launches
   int since_rehome = 0;
+  bool fresh = true;  // a state came in since the last re-homing
 };
 
 namespace {
@@ -572,7 +573,7 @@ void launch_step_kernels(spc2_batch &b, const EpiCtx &e, int k, bool srk, bool s
   if (!staged)
     hipLaunchKernelGGL(k_b_stage_bin, g, blk, 0, b.stream, b.nt, (const Rep *)b.d_reps, (const int *)b.rep_of,
                        (const double *)b.sx, (const double *)b.sy, (const double *)b.sp, b.gx, b.gy, b.gp,
-                       b.cell_of, b.count_, b.local);
+                       b.bins());
   launch_scan_raw(b.stream, b.bsum, b.count_, b.nct, b.start);
   launch_place_raw(b.stream, b.nt, b.cell_of, b.local, b.start, b.hid, b.tmp, b.tmpid);
   hipLaunchKernelGGL(k_b_rank_tiles<PREC>, g, blk, 0, b.stream, b.nt, (const Rep *)b.d_reps, (const int *)b.rep_of,
@@ -586,9 +587,7 @@ void launch_step_kernels(spc2_batch &b, const EpiCtx &e, int k, bool srk, bool s
     es.bgx = b.spare[0];
     es.bgy = b.spare[1];
     es.bgp = b.spare[2];
-    es.bcell = b.cell_of;
-    es.bcount = b.count_;
-    es.blocal = b.local;
+    es.bins = b.bins();
   }
   if (!srk) {
     if (b.napv)
@@ -675,9 +674,14 @@ spc2_status run_steps(spc2_batch &b, int method, double dt, int64_t nsteps, cons
     e.sy = b.sy;
     e.sp = b.sp;
     e.sa.omega = b.omega;
+    // a re-homing: every kRehomeEvery steps, and after the first of several steps
+    // from a new state, whose homes are in id order (at 3.86M particles in random
+    // order the placing and the sort take 240 us a step and in cell order 103, the
+    // pair kernel 690 and 630; a re-homing takes 197)
+    const bool rehome = b.since_rehome + 1 >= kRehomeEvery || (b.fresh && k + 1 < kmax);
     // the next step's stage and bins come from this step's state-writing pass
     // when every replica takes that step and no re-homing comes between
-    const bool fuse = k + 1 < kmin && b.since_rehome + 1 < kRehomeEvery && b.nap + b.napv + b.nseg > 0;
+    const bool fuse = k + 1 < kmin && !rehome && b.nap + b.napv + b.nseg > 0;
     switch (b.prec) {
       case P64: launch_step_kernels<P64>(b, e, (int)k, srk, staged, fuse); break;
       case P64F: launch_step_kernels<P64F>(b, e, (int)k, srk, staged, fuse); break;
@@ -689,7 +693,9 @@ spc2_status run_steps(spc2_batch &b, int method, double dt, int64_t nsteps, cons
       std::swap(b.gp, b.spare[2]);
     }
     staged = fuse;
-    if (++b.since_rehome >= kRehomeEvery) {
+    ++b.since_rehome;
+    if (rehome) {
+      b.fresh = false;
       launch_rehome(b);
       b.since_rehome = 0;
     }
@@ -844,6 +850,7 @@ spc2_status spc2_batch_init_random_state(spc2_batch_t b, double omega_std) {
                      (const int *)b->rep_of, (const int *)b->hid, omega_std, (const int *)nullptr, b->sx, b->sy,
                      b->sp, b->omega);
   if (spc2_status st = check_launch("batch init state")) return st;
+  b->fresh = true;
   B_TRY(hipStreamSynchronize(b->stream));
   return SPC2_OK;
 }
@@ -852,6 +859,7 @@ spc2_status spc2_batch_set_state(spc2_batch_t b, int32_t r, const double *state)
   if (check_replica(b, r) || !state) return set_error(SPC2_ERR_INVALID, "bad replica or null state");
   const Rep &R = b->reps[r];
   if (spc2_status st = ensure_io(*b, (size_t)R.n)) return st;
+  b->fresh = true;
   std::vector<double> buf((size_t)R.n);
   double *dst[3] = {b->sx, b->sy, b->sp};
   for (int c = 0; c < 3; ++c) {

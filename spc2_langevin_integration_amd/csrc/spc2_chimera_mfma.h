@@ -448,6 +448,7 @@ __device__ __forceinline__ void mfma_segment(const KParams &P, const int *__rest
         r.written = r.n != 0;
         r.aphi = r.n != 0 ? P.sigma * A / (double)r.n : 0.0;
         const EpiState st = epilogue1<EPI>(P, e, h, id, k, r);
+        bin_stage<EPI>(P, e, h, id, st);
         if constexpr (EPI == EPI_ITO1) {  // pass 2's features
           const double a = st.ap * P.raj;
           const Fixed<1> own(t.f4[k], nullptr, k);

@@ -9,6 +9,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "spc2_internal.h"
+
 namespace spc2 {
 
 // ---- geometry (PeriodicBoundaryConditions.cpp) -----------------------------
@@ -54,7 +56,7 @@ __device__ __forceinline__ int cell_coord(double x, double L, int n) {
   return (int)f;
 }
 
-// ---- stable rank inside a cell ----------------------------------------------
+// ---- stable rank inside a cell, by slot ------------------------------------
 // The counting sort places a workgroup's slots in cells of increasing index, so
 // their cells span [start of the first slot's cell, end of the last slot's
 // cell).  stage_cell_ids copies the placed ids of that span to LDS when it holds
@@ -284,6 +286,47 @@ __device__ __forceinline__ int wave_aggregated_rank(int *count, int c, bool vali
   int base = 0;
   if (valid && lane == leader) base = atomicAdd(&count[c], __popcll(mates));
   return __shfl(base, leader, 64) + __popcll(mates & below);
+}
+
+// ---- binning --------------------------------------------------------------------
+// Bins home h (particle `id`) into cell c and keeps, for the stable sort by id,
+// either its arrival rank (cap 0: next[h], which k_place orders the particles by) or
+// its id in the cell's list of `cap` entries, whose smaller ids are its rank, read
+// by a thread per home without a placing pass.  Arrivals past cap are chained:
+// chain[c] the last one's home + 1, next[home] the one before.  Every lane of the
+// wavefront that reaches the call takes part.
+__device__ __forceinline__ void bin_particle(const Bins &b, int c, int cap, int h, int id, bool valid) {
+  const int r = wave_aggregated_rank(b.count, c, valid);
+  if (!valid) return;
+  if (cap == 0)
+    b.next[h] = r;
+  else if (r < cap)
+    b.list[(size_t)c * (size_t)cap + r] = id;
+  else
+    b.next[h] = atomicExch(&b.chain[c], h + 1);
+}
+
+// The number of cell c's cnt particles with an id below `id`, from its list.
+__device__ __forceinline__ int rank_in_bin(const Bins &b, int c, int cap, int cnt, const int *hid, int id) {
+  const int4 *list = (const int4 *)(b.list + (size_t)c * (size_t)cap);  // cap is a multiple of four
+  const int m = min(cnt, cap);
+  int r = 0;
+  for (int q = 0; 4 * q < m; q += 4) {  // four requests under way (within the list: few of them are for nothing)
+    int4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = list[min(q + u, cap / 4 - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = 4 * (q + u);
+      r += k < m && v[u].x < id;
+      r += k + 1 < m && v[u].y < id;
+      r += k + 2 < m && v[u].z < id;
+      r += k + 3 < m && v[u].w < id;
+    }
+  }
+  if (cnt > cap)
+    for (int k = b.chain[c]; k; k = b.next[k - 1]) r += hid[k - 1] < id;
+  return r;
 }
 
 }  // namespace spc2

@@ -58,6 +58,7 @@ struct KParams {
   int seg_w, segs, lds_cap, chunk;
   int mfma;   // dense FP32 chimera cells: the matrix-core passes (spc2_chimera_mfma.h)
   double aj, raj;  // their scale of pass 2's a_j, a power of two >= |a_j|, and its reciprocal
+  int bin_cap;  // entries of a cell's list (see Bins), a multiple of 4; 0: no lists
   int lanes;  // lanes per centre particle of the FP64 cell walks (a power of two; 1 in the FP32 form)
 };
 
@@ -66,6 +67,13 @@ struct Tiles {
   double *x, *y, *p, *c, *s;  // FP64 forms: wrapped stage position, stage phase, cos/sin
   float4 *f4;                 // FP32 form: cell-local x, y and cos, sin of the phase
   int *cell;                  // cell of each slot
+};
+
+// One binning (bin_particle): cell of each home, count of each cell, and either the
+// arrival ranks by home (next) or the cells' lists of particle ids with their
+// overflow chains (links in next).
+struct Bins {
+  int *cell_of, *count, *chain, *list, *next;
 };
 
 struct StepArgs {
@@ -104,10 +112,17 @@ struct Sim {
   int *hid = nullptr, *hpos = nullptr;
   bool hpos_stale = false;
   // cell list (per home: cell_of, local; per slot: tmp/tmpid while placing,
-  // then slot_h / slot_id = home / id of the particle in each cell-sorted slot)
-  int *cell_of = nullptr, *count = nullptr, *local = nullptr, *start = nullptr, *tmp = nullptr,
-      *tmpid = nullptr, *slot_h = nullptr, *slot_id = nullptr;
+  // then slot_h / slot_id = home / id of the particle in each cell-sorted slot);
+  // with lists (bin_cap > 0) count holds two sets of count_stride counts and as many
+  // chains, of which bin_set takes the next binning, else one set of counts
+  int *cell_of = nullptr, *count = nullptr, *local = nullptr, *start = nullptr, *tmp = nullptr, *tmpid = nullptr,
+      *bin_list = nullptr, *slot_h = nullptr, *slot_id = nullptr;
+  int bin_set = 0, count_stride = 0;  // counts of a set, padded
   bool built = false;  // slot_h holds the cell order of the current homes
+  Bins bins() const {
+    int *c = count + (size_t)bin_set * 2 * (size_t)count_stride;
+    return Bins{cell_of, c, c + count_stride, bin_list, local};
+  }
   int rehome_every = 16, steps_since_rehome = 0;
   // re-homing double buffers (state x, y, phi, omega, k_1..k_4) and id-order
   // transfer scratch for the ABI's host arrays
@@ -115,13 +130,16 @@ struct Sim {
   int *spare_i = nullptr;
   double *io[3] = {};
   Tiles t{};
-  // Verlet: the next stage's tiles and phases, written by a pass-1 epilogue
-  // (t2.cell aliases t.cell); swapped with t / gp after that launch
+  // The next stage, written by a pass's epilogue.  Verlet: its tiles and phases
+  // (t2.cell aliases t.cell), swapped with t / gp after that launch.  All pairs:
+  // gx2, gy2, gp2 and the FP32 tiles t2.f4, swapped likewise.  Linked cells: gx, gy,
+  // gp in place (a pass reads its own particle's gp only) and the bins.
   Tiles t2{};
-  double *gp2 = nullptr;
+  double *gx2 = nullptr, *gy2 = nullptr, *gp2 = nullptr;
   int vnext = 0;            // next launch's stage write: 0 none, 1 s + vnext_kcdt k, 2 the new state
   double vnext_kcdt = 0.0;
-  bool tile_fresh = false;  // t / gp hold the tiles of the current state
+  bool tile_fresh = false;  // Verlet: t / gp hold the tiles of the current state
+  bool staged = false;      // cells, all pairs: the next build finds its stage (and bins) written
   // pass-1 results kept per slot for pass 2
   double *aphi_slot = nullptr, *n_slot = nullptr, *n2_slot = nullptr;
   float *aphi_slot_f = nullptr;
@@ -221,13 +239,12 @@ void fill_kparams_from(KParams &k, const spc2_params &P, int n, int nx, int ny, 
 // spc2_cells.hip
 void launch_stage_bin(Sim &s, const double *kx, const double *ky, const double *kp, double kcdt);
 int scan_blocks(int nc);
-void launch_scan(Sim &s);
 void launch_scan_array(Sim &s, int *count, int m, int *out);
 void launch_scan_raw(hipStream_t st, int *bsum, int *count, int m, int *out);
 void launch_place_raw(hipStream_t st, int n, const int *cell_of, const int *local, const int *start, const int *hid,
                       int *tmp, int *tmpid);
-void launch_place(Sim &s);
-void launch_rank_tiles(Sim &s);
+void launch_cells(Sim &s);
+void configure_bins(Sim &s);
 // spc2_pairs.hip
 constexpr double kSegTarget = 256.0;  // default particles per pair workgroup (row chunk or segment)
 constexpr int kLdsBytes = 60 * 1024;  // dynamic LDS of one pair workgroup at most

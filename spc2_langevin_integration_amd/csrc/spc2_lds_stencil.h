@@ -510,7 +510,7 @@ __device__ __forceinline__ void pass1_segment(const KParams &P, const int *__res
     const int h = slot_h[k], id = slot_id[k];
     Pass1Out o{};
     acc.finish(P, PREC == P32K ? gp[h] : 0.0, o);
-    epilogue1<EPI>(P, e, h, id, k, o);
+    bin_stage<EPI>(P, e, h, id, epilogue1<EPI>(P, e, h, id, k, o));
     cand_sum += cand;
     n_sum += o.n;
     n2_sum += o.n2;

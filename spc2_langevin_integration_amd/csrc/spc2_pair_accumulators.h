@@ -1322,12 +1322,13 @@ struct EpiCtx {
   double *gpn;
   double kcdt_n;
   int next;
-  // Batch steps: the state-writing epilogue (SE, SRK) also stages and bins the
-  // new state for the next step (stage arrays bgx/bgy/bgp by particle, its
-  // cell, its rank among the cell's count); null bcell: a separate launch does
-  // that at the next step.  bcoff: the replica's first cell.
+  // Steps over linked cells and batch steps: the epilogue also stages and bins
+  // what the next build takes (linked single handles: next and kcdt_n as above;
+  // the batch: the new state), into bgx/bgy/bgp by particle and `bins`; null
+  // bins.cell_of: a separate launch does that.  bcoff: the replica's first cell.
+  // All-pairs single handles: bgx/bgy/bgp and tn.f4 without bins.
   double *bgx, *bgy, *bgp;
-  int *bcell, *bcount, *blocal;
+  Bins bins;
   int bcoff;
 };
 
@@ -1343,11 +1344,11 @@ __device__ __forceinline__ void wrap_state(const KParams &P, double &x, double &
   y = y - floor(y * P.rLy) * P.Ly;
 }
 
-// The new state (x, y, p) of particle h staged for the next step as the
-// batch's stage-and-bin launch stages it: the conditional wrap, the cell of the
-// wrapped position (the replica's one cell on the all-pairs path) and a rank
-// among that cell's particles from a wave-aggregated atomic on its count.
-__device__ __forceinline__ void bin_next(const KParams &P, const EpiCtx &e, int h, double x, double y, double p) {
+// The next stage (x, y, p) of particle h as the stage-and-bin launch writes it:
+// the conditional wrap, the cell of the wrapped position (a replica's one cell on
+// the all-pairs path) and its bin.
+__device__ __forceinline__ void bin_next(const KParams &P, const EpiCtx &e, int h, int id, double x, double y,
+                                         double p) {
   int lc = 0;
   if (P.linked) {
     const Box b{P.Lx, P.Ly, P.rLx, P.rLy};
@@ -1355,11 +1356,41 @@ __device__ __forceinline__ void bin_next(const KParams &P, const EpiCtx &e, int 
     lc = cell_coord(y, b.Ly, P.ny) * P.nx + cell_coord(x, b.Lx, P.nx);
   }
   const int c = e.bcoff + lc;
-  e.bcell[h] = c;
+  e.bins.cell_of[h] = c;
   e.bgx[h] = x;
   e.bgy[h] = y;
   e.bgp[h] = p;
-  e.blocal[h] = wave_aggregated_rank(e.bcount, c, true);
+  bin_particle(e.bins, c, P.bin_cap, h, id, true);
+}
+
+// Linked cells, the passes that leave the state alone (EPI_K) or combine it
+// (RK4's last): the next stage of particle h from what epilogue1 returned.
+template <int EPI>
+__device__ __forceinline__ void bin_stage(const KParams &P, const EpiCtx &e, int h, int id, const EpiState &r) {
+  if (EPI == EPI_K && e.bins.cell_of)
+    bin_next(P, e, h, id, e.sx[h] + e.kcdt_n * r.ax, e.sy[h] + e.kcdt_n * r.ay, e.sp[h] + e.kcdt_n * r.ap);
+  if (EPI == EPI_RK4_FINAL && e.bins.cell_of) bin_next(P, e, h, id, r.x, r.y, r.p);
+}
+
+// All pairs, single handles: the next stage of particle h (double-buffered: other
+// particles still read this one) and its FP32 tile, as the stage launch writes them.
+template <int EPI>
+__device__ __forceinline__ void stage_next(const EpiCtx &e, int h, const EpiState &r) {
+  if (EPI == EPI_ITO1 || EPI == EPI_ITO2 || !e.next) return;
+  double x = r.x, y = r.y, p = r.p;
+  if (EPI == EPI_K) {
+    x = e.sx[h] + e.kcdt_n * r.ax;
+    y = e.sy[h] + e.kcdt_n * r.ay;
+    p = e.sp[h] + e.kcdt_n * r.ap;
+  }
+  e.bgx[h] = x;
+  e.bgy[h] = y;
+  e.bgp[h] = p;
+  if (e.tn.f4) {
+    double sn, cs;
+    sincos(p, &sn, &cs);
+    e.tn.f4[h] = make_float4((float)x, (float)y, (float)cs, (float)sn);
+  }
 }
 
 // Final phi derivative given the in/out value (k_next or derivative entry
@@ -1457,7 +1488,7 @@ __device__ __forceinline__ EpiState epilogue1(const KParams &P, const EpiCtx &e,
     e.sx[h] = x;
     e.sy[h] = y;
     e.sp[h] = p;
-    if (e.bcell) bin_next(P, e, h, x, y, p);
+    if (e.bins.cell_of) bin_next(P, e, h, id, x, y, p);
     r.ap = ap;
     r.x = x;
     r.y = y;
@@ -1496,7 +1527,7 @@ __device__ __forceinline__ EpiState epilogue2(const KParams &P, const EpiCtx &e,
     e.sx[h] = x;
     e.sy[h] = y;
     e.sp[h] = p;
-    if (e.bcell) bin_next(P, e, h, x, y, p);
+    if (e.bins.cell_of) bin_next(P, e, h, id, x, y, p);
     r.x = x;
     r.y = y;
     r.p = p;

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(kBlock) void k_pass1_allpairs(KParams P, const doub
   Pass1Out o{};
   if (active) {
     allpairs_pass1<PREC, SYS>(P, i, g, gx, gy, gp, tiles, o);
-    if (lead) epilogue1<EPI>(P, e, i, i, i, o);  // all pairs: home order is the id order
+    if (lead) stage_next<EPI>(e, i, epilogue1<EPI>(P, e, i, i, i, o));  // all pairs: home order is the id order
   }
   if (counts) count_add(counts, lead ? P.n - 1 : 0, lead ? o.n : 0, lead ? o.n2 : 0);
 }
@@ -90,12 +90,43 @@ __global__ __launch_bounds__(kBlock) void k_pass2_allpairs(KParams P, const doub
   Pass2Out o;
   const double in0 = EPI == EPI_ITO2 ? e.a0[i] : 0.0, in1 = EPI == EPI_ITO2 ? e.a1[i] : 0.0;
   allpairs_pass2<SYS>(P, i, g, gx, gy, gp, e.aphi_slot, e.n_slot, e.n2_slot, in0, in1, o);
-  if (g == 0) epilogue2<EPI>(P, e, i, i, o);
+  if (g == 0) stage_next<EPI>(e, i, epilogue2<EPI>(P, e, i, i, o));
 }
 
 // =============================================================================
 // dispatch
 // =============================================================================
+
+// Has the launch write the next stage (s.vnext, consumed here): the bins of linked
+// cells, or the all-pairs path's second stage arrays.
+bool take_next(Sim &s, EpiCtx &e) {
+  if (!s.vnext) return false;
+  e.next = s.vnext;
+  e.kcdt_n = s.vnext_kcdt;
+  s.vnext = 0;
+  if (s.linked) {
+    e.bgx = s.gx;
+    e.bgy = s.gy;
+    e.bgp = s.gp;
+    e.bins = s.bins();
+  } else {
+    e.bgx = s.gx2;
+    e.bgy = s.gy2;
+    e.bgp = s.gp2;
+    e.tn.f4 = s.t2.f4;
+  }
+  return true;
+}
+
+void next_taken(Sim &s) {
+  if (!s.linked) {
+    std::swap(s.gx, s.gx2);
+    std::swap(s.gy, s.gy2);
+    std::swap(s.gp, s.gp2);
+    std::swap(s.t.f4, s.t2.f4);
+  }
+  s.staged = true;
+}
 
 template <int PREC, int SYS, int EPI>
 void pass1_typed(Sim &s, const EpiCtx &e) {
@@ -223,6 +254,7 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
   k.lanes = 1;
   k.mfma = 0;
   k.aj = k.raj = 1.0;
+  k.bin_cap = 0;
   if (!k.linked) {
     k.seg_w = k.segs = 1;
     k.lds_cap = 0;
@@ -289,22 +321,26 @@ void configure_segments(Sim &s) { configure_segments_kp(s.kp, s.prec, s.P.system
 void launch_pass1(Sim &s, int epi, double *ox, double *oy, double *op, const StepArgs &sa, double *const k1[3],
                   double *const k2[3], double *const k3[3]) {
   EpiCtx e = make_ctx(s, ox, oy, op, sa, k1, k2, k3);
+  const bool next = take_next(s, e);
   switch (s.prec) {
     case P64: pass1_sys<P64>(s, epi, e); break;
     case P64F: pass1_sys<P64F>(s, epi, e); break;
     default: pass1_sys<P32K>(s, epi, e);
   }
+  if (next) next_taken(s);
 }
 
 void launch_pass2(Sim &s, int epi, double *a0, double *a1, const StepArgs &sa) {
   EpiCtx e = make_ctx(s, nullptr, nullptr, nullptr, sa, nullptr, nullptr, nullptr);
   e.a0 = a0;
   e.a1 = a1;
+  const bool next = take_next(s, e);
   switch (s.prec) {
     case P64: pass2_sys<P64>(s, epi, e); break;
     case P64F: pass2_sys<P64F>(s, epi, e); break;
     default: pass2_sys<P32K>(s, epi, e);
   }
+  if (next) next_taken(s);
 }
 
 }  // namespace spc2
