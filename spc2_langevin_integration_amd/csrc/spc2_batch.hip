@@ -235,7 +235,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(PREC == P32K
   const EpiCtx c = rep_ctx(e, R, k);
   if constexpr (PREC == P32K) {
     if (P.mfma) {
-      mfma_segment<1, EPI>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
+      mfma_segment<1, EPI, false>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
       return;
     }
   }
@@ -264,7 +264,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(PREC == P32K
   const EpiCtx c = rep_ctx(e, R, k);
   if constexpr (PREC == P32K) {
     if (P.mfma) {
-      mfma_segment<2, EPI_SRK>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
+      mfma_segment<2, EPI_SRK, false>(P, start + R.coff, t, slot_h, slot_id, gp, c, nullptr, sg - R.soff, sh, dyn_lds);
       return;
     }
   }

@@ -57,6 +57,7 @@ namespace {
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 
+constexpr int kMfmaShort = 64;         // slots of a short chunk (configure_segments)
 constexpr int kMfmaTile = 16;          // candidates per tile, centres per group
 constexpr int kMfmaWindow = kPairBlock;  // centres of a workgroup at most
 constexpr float kMfmaFar = 1.0e6f;     // x and y of the padding candidates
@@ -301,7 +302,10 @@ __device__ __forceinline__ void mfma_cell(const KParams &P, const Tiles &t, cons
 }
 
 // One pair workgroup: pass1_segment / pass2_segment of a dense FP32 chimera system.
-template <int PASS, int EPI>
+// SHORT: for chunks of at most kMfmaShort slots, of fewer cells than wavefronts,
+// whose groups of centres then go to a wavefront each (an instance of its own: in
+// one kernel the two walks' registers cost a batch's pass 13%).
+template <int PASS, int EPI, bool SHORT>
 __device__ __forceinline__ void mfma_segment(const KParams &P, const int *__restrict__ start, const Tiles &t,
                                              const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                              const double *gp, const EpiCtx &e, unsigned long long *counts, int seg,
@@ -399,16 +403,25 @@ __device__ __forceinline__ void mfma_segment(const KParams &P, const int *__rest
   if (staged) {
     const int wave = threadIdx.x >> 6, c1 = c0 + ncen;
     int unit = 0;
-    for (int q = 1; q <= g.W; ++q) {
-      int a = __builtin_amdgcn_readfirstlane(max(c0, rows.at(1, sh.off[g.ncol + q])));
-      const int z = __builtin_amdgcn_readfirstlane(min(c1, rows.at(1, sh.off[g.ncol + q + 1])));
-      if (a >= z || (unit++ & 3) != wave) continue;
-      while (a < z) {  // at most three groups at a time (registers), four as two and two
-        const int left = (z - a + 15) >> 4, groups = left == 4 ? 2 : min(3, left), ce = min(z, a + 16 * groups);
-        if (groups == 3) mfma_cell<PASS, 3>(P, t, sh, g, rows, lds, q, a, ce, c0, b.k0, band);
-        else if (groups == 2) mfma_cell<PASS, 2>(P, t, sh, g, rows, lds, q, a, ce, c0, b.k0, band);
-        else mfma_cell<PASS, 1>(P, t, sh, g, rows, lds, q, a, ce, c0, b.k0, band);
-        a = ce;
+    if (SHORT) {
+      for (int q = 1; q <= g.W; ++q) {
+        int a = __builtin_amdgcn_readfirstlane(max(c0, rows.at(1, sh.off[g.ncol + q])));
+        const int z = __builtin_amdgcn_readfirstlane(min(c1, rows.at(1, sh.off[g.ncol + q + 1])));
+        for (; a < z; a += 16, ++unit)
+          if ((unit & 3) == wave) mfma_cell<PASS, 1>(P, t, sh, g, rows, lds, q, a, min(z, a + 16), c0, b.k0, band);
+      }
+    } else {
+      for (int q = 1; q <= g.W; ++q) {
+        int a = __builtin_amdgcn_readfirstlane(max(c0, rows.at(1, sh.off[g.ncol + q])));
+        const int z = __builtin_amdgcn_readfirstlane(min(c1, rows.at(1, sh.off[g.ncol + q + 1])));
+        if (a >= z || (unit++ & 3) != wave) continue;
+        while (a < z) {  // at most three groups at a time (registers), four as two and two
+          const int left = (z - a + 15) >> 4, groups = left == 4 ? 2 : min(3, left), ce = min(z, a + 16 * groups);
+          if (groups == 3) mfma_cell<PASS, 3>(P, t, sh, g, rows, lds, q, a, ce, c0, b.k0, band);
+          else if (groups == 2) mfma_cell<PASS, 2>(P, t, sh, g, rows, lds, q, a, ce, c0, b.k0, band);
+          else mfma_cell<PASS, 1>(P, t, sh, g, rows, lds, q, a, ce, c0, b.k0, band);
+          a = ce;
+        }
       }
     }
     __syncthreads();

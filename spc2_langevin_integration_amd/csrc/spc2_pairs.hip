@@ -45,22 +45,22 @@ __global__ __launch_bounds__(kBlock) void k_pass2_lds(KParams P, const int *__re
 }
 
 // The matrix-core passes of dense FP32 chimera cells.
-template <int EPI>
+template <int EPI, bool SHORT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_pass1_mfma(KParams P, const int *__restrict__ start, Tiles t,
                                                        const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                                        const double *gp, EpiCtx e, unsigned long long *counts) {
   extern __shared__ float4 dyn_lds[];
   __shared__ SegShared sh;
-  mfma_segment<1, EPI>(P, start, t, slot_h, slot_id, gp, e, counts, xcd_segment(blockIdx.x, gridDim.x), sh, dyn_lds);
+  mfma_segment<1, EPI, SHORT>(P, start, t, slot_h, slot_id, gp, e, counts, xcd_segment(blockIdx.x, gridDim.x), sh, dyn_lds);
 }
 
-template <int EPI>
+template <int EPI, bool SHORT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_pass2_mfma(KParams P, const int *__restrict__ start, Tiles t,
                                                        const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                                        const double *gp, EpiCtx e) {
   extern __shared__ float4 dyn_lds[];
   __shared__ SegShared sh;
-  mfma_segment<2, EPI>(P, start, t, slot_h, slot_id, gp, e, nullptr, xcd_segment(blockIdx.x, gridDim.x), sh, dyn_lds);
+  mfma_segment<2, EPI, SHORT>(P, start, t, slot_h, slot_id, gp, e, nullptr, xcd_segment(blockIdx.x, gridDim.x), sh, dyn_lds);
 }
 
 // =============================================================================
@@ -136,7 +136,7 @@ void pass1_typed(Sim &s, const EpiCtx &e) {
     const size_t sh = pair_lds_bytes(s.kp, PREC, 1);
     if constexpr (PREC == P32K && SYS == SPC2_CHIMERA) {
       if (s.kp.mfma) {
-        launch_pair(s, k_pass1_mfma<EPI>, grid, blk, sh, s.kp, (const int *)s.start, s.t, (const int *)s.slot_h,
+        launch_pair(s, s.kp.chunk <= kMfmaShort ? k_pass1_mfma<EPI, true> : k_pass1_mfma<EPI, false>, grid, blk, sh, s.kp, (const int *)s.start, s.t, (const int *)s.slot_h,
                     (const int *)s.slot_id, (const double *)s.gp, e, cnt);
         return;
       }
@@ -181,7 +181,7 @@ void pass2_typed(Sim &s, const EpiCtx &e) {
     const dim3 grid(s.ny * s.kp.segs), blk(kBlock);
     if constexpr (PREC == P32K && SYS == SPC2_CHIMERA) {
       if (s.kp.mfma) {
-        launch_pair(s, k_pass2_mfma<EPI>, grid, blk, sh, s.kp, (const int *)s.start, s.t, (const int *)s.slot_h,
+        launch_pair(s, s.kp.chunk <= kMfmaShort ? k_pass2_mfma<EPI, true> : k_pass2_mfma<EPI, false>, grid, blk, sh, s.kp, (const int *)s.start, s.t, (const int *)s.slot_h,
                     (const int *)s.slot_id, (const double *)s.gp, e);
         return;
       }
@@ -231,6 +231,12 @@ int lds_elem_bytes(int prec) {
 
 }  // namespace
 
+// a row's mean count and four standard deviations, in chunks
+static int chunks_per_row(const KParams &k) {
+  const double row = (double)k.n / (double)k.ny;
+  return std::max(1, (int)std::ceil((row + 4.0 * std::sqrt(row) + 8.0) / k.chunk));
+}
+
 // The pair workgroups of a linked system: about `target` lanes each and an LDS
 // capacity for their halo.
 // * The FP64 forms split each particle's candidates over `lanes` lanes: enough
@@ -272,15 +278,14 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
     int chunk = unit * std::max(1, (int)std::lround(target / unit));
     // at most kMaxSegW - 3 cells' worth, so a chunk's columns fit the halo tables
     chunk = std::min(chunk, unit * std::max(1, (int)std::floor((kMaxSegW - 3) * per_cell / unit)));
-    const double row = (double)k.n / (double)k.ny;
     k.chunk = chunk;
-    k.segs = std::max(1, (int)std::ceil((row + 4.0 * std::sqrt(row) + 8.0) / chunk));
+    k.segs = chunks_per_row(k);
     k.seg_w = std::min(k.nx, (int)std::ceil(chunk / per_cell) + 1);
     halo = 1.25 * 3.0 * (chunk + 3.0 * per_cell);  // chunk's cells, a partial cell at each end, and the sides
     if (prec == P32K && system == SPC2_CHIMERA && per_cell >= kMfmaPerCell) {
       k.mfma = 1;
       k.chunk = std::min(chunk, kMfmaWindow);
-      k.segs = std::max(1, (int)std::ceil((row + 4.0 * std::sqrt(row) + 8.0) / k.chunk));
+      k.segs = chunks_per_row(k);
       // |a_j| <= |sigma|: sigma times a mean of sines
       k.aj = std::exp2(std::ceil(std::log2(std::max(std::fabs(k.sigma) * 1.0001, 1e-200))));
       k.raj = 1.0 / k.aj;
@@ -316,7 +321,20 @@ size_t pair_lds_bytes(const KParams &k, int prec, int pass) {
   return (size_t)k.lds_cap * (size_t)elem + (size_t)lds_near_bytes(prec);
 }
 
-void configure_segments(Sim &s) { configure_segments_kp(s.kp, s.prec, s.P.system, kSegTarget); }
+// A single handle's pair workgroups.  The matrix-core passes of a small system are
+// bound by the latency of one workgroup's phases, so its chunks are halved while
+// twice the workgroups still fit the device at once (four on each of 256 CUs), to 32
+// slots at the least (two groups of centres).  Pass 1 of SE at N = 8191: 24.7 us with
+// 256 slots, 18.7 with 128, 16.7 with 64, 14.3 with 32, 14.5 with 16; both SRK passes
+// at N = 40,000: 51, 42, 39 and, past one fill, 51 with 32; at N = 120,000: 71, 67 and
+// 86 with 64.  (The sums are whole numbers: no result depends on the chunk.)
+void configure_segments(Sim &s) {
+  KParams &k = s.kp;
+  configure_segments_kp(k, s.prec, s.P.system, kSegTarget);
+  if (!k.mfma) return;
+  while (k.chunk > 32 && 2LL * k.n <= 1024LL * k.chunk) k.chunk /= 2;
+  k.segs = chunks_per_row(k);
+}
 
 void launch_pass1(Sim &s, int epi, double *ox, double *oy, double *op, const StepArgs &sa, double *const k1[3],
                   double *const k2[3], double *const k3[3]) {

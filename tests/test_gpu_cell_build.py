@@ -90,3 +90,20 @@ def test_clustered_replicas_are_single_handles(prec, method):
             s.set_state(st)
             s.step(method, 0.01, 0, STEPS)
             assert np.array_equal(got[r], s.get_state()), f"replica {r}"
+
+
+# both sides of the chunk lengths of the matrix-core passes (32, 64, 128, 256 slots); a batch's are 256
+@pytest.mark.parametrize("method", ["se", "srk"])
+@pytest.mark.parametrize("n", [16384, 16385, 32769, 65537, 131073])
+def test_chunk_length_leaves_the_bits(n, method):
+    L = float(np.sqrt(n / 4000.0))
+    p = spc2.params("chimera", "fp32k", "auto", n=n, L=L, rho=0.1, v0=0.01, sigma=1.0, alpha=1.45, D=0.01, seed=3)
+    st = state_of(n, None)
+    st[0::3] *= L
+    st[1::3] *= L
+    with spc2.Batch([p]) as b, spc2.Sim(p) as s:
+        b.set_state(0, st)
+        b.step(0.01, 3, method=method)
+        s.set_state(st)
+        s.step(method, 0.01, 0, 3)
+        assert np.array_equal(b.get_state(0), s.get_state())
