@@ -313,14 +313,27 @@ __global__ __launch_bounds__(kB) void k_b_init_state(int n, const Rep *reps, con
 }
 
 // id order <-> home order for one replica
-__global__ __launch_bounds__(kB) void k_b_to_home(int n, int off, const int *hpos, const double *src, double *dst) {
+// One replica's AoS array by id, comps (1 or 3) components, to home order and back.
+__global__ __launch_bounds__(kB) void k_b_to_home(int n, int off, int comps, const int *hpos, const double *aos,
+                                                  double *d0, double *d1, double *d2) {
   const int i = blockIdx.x * kB + threadIdx.x;
-  if (i < n) dst[hpos[off + i]] = src[i];
+  if (i >= n) return;
+  const int h = hpos[off + i];
+  d0[h] = aos[(size_t)comps * i];
+  if (comps == 3) {
+    d1[h] = aos[(size_t)3 * i + 1];
+    d2[h] = aos[(size_t)3 * i + 2];
+  }
 }
 
-__global__ __launch_bounds__(kB) void k_b_from_home(int n, int off, const int *hpos, const double *src, double *dst) {
+__global__ __launch_bounds__(kB) void k_b_from_home(int n, int off, const int *hpos, const double *sx,
+                                                    const double *sy, const double *sp, double *aos) {
   const int i = blockIdx.x * kB + threadIdx.x;
-  if (i < n) dst[i] = src[hpos[off + i]];
+  if (i >= n) return;
+  const int h = hpos[off + i];
+  aos[3 * (size_t)i] = sx[h];
+  aos[3 * (size_t)i + 1] = sy[h];
+  aos[3 * (size_t)i + 2] = sp[h];
 }
 
 // Carries n values of one replica from another batch (home order there, id
@@ -858,33 +871,25 @@ spc2_status spc2_batch_init_random_state(spc2_batch_t b, double omega_std) {
 spc2_status spc2_batch_set_state(spc2_batch_t b, int32_t r, const double *state) {
   if (check_replica(b, r) || !state) return set_error(SPC2_ERR_INVALID, "bad replica or null state");
   const Rep &R = b->reps[r];
-  if (spc2_status st = ensure_io(*b, (size_t)R.n)) return st;
+  const size_t bytes = sizeof(double) * 3 * (size_t)R.n;
+  if (spc2_status st = ensure_io(*b, 3 * (size_t)R.n)) return st;
   b->fresh = true;
-  std::vector<double> buf((size_t)R.n);
-  double *dst[3] = {b->sx, b->sy, b->sp};
-  for (int c = 0; c < 3; ++c) {
-    for (int i = 0; i < R.n; ++i) buf[i] = state[3 * (size_t)i + c];
-    B_TRY(hipMemcpyAsync(b->io, buf.data(), sizeof(double) * R.n, hipMemcpyHostToDevice, b->stream));
-    hipLaunchKernelGGL(k_b_to_home, dim3(bfor(R.n)), dim3(kB), 0, b->stream, R.n, R.poff, (const int *)b->hpos,
-                       (const double *)b->io, dst[c]);
-    B_TRY(hipStreamSynchronize(b->stream));
-  }
+  B_TRY(hipMemcpyAsync(b->io, state, bytes, hipMemcpyHostToDevice, b->stream));
+  hipLaunchKernelGGL(k_b_to_home, dim3(bfor(R.n)), dim3(kB), 0, b->stream, R.n, R.poff, 3, (const int *)b->hpos,
+                     (const double *)b->io, b->sx, b->sy, b->sp);
+  B_TRY(hipStreamSynchronize(b->stream));
   return check_launch("batch set state");
 }
 
 spc2_status spc2_batch_get_state(spc2_batch_t b, int32_t r, double *state) {
   if (check_replica(b, r) || !state) return set_error(SPC2_ERR_INVALID, "bad replica or null state");
   const Rep &R = b->reps[r];
-  if (spc2_status st = ensure_io(*b, (size_t)R.n)) return st;
-  std::vector<double> buf((size_t)R.n);
-  const double *src[3] = {b->sx, b->sy, b->sp};
-  for (int c = 0; c < 3; ++c) {
-    hipLaunchKernelGGL(k_b_from_home, dim3(bfor(R.n)), dim3(kB), 0, b->stream, R.n, R.poff, (const int *)b->hpos,
-                       src[c], b->io);
-    B_TRY(hipMemcpyAsync(buf.data(), b->io, sizeof(double) * R.n, hipMemcpyDeviceToHost, b->stream));
-    B_TRY(hipStreamSynchronize(b->stream));
-    for (int i = 0; i < R.n; ++i) state[3 * (size_t)i + c] = buf[i];
-  }
+  const size_t bytes = sizeof(double) * 3 * (size_t)R.n;
+  if (spc2_status st = ensure_io(*b, 3 * (size_t)R.n)) return st;
+  hipLaunchKernelGGL(k_b_from_home, dim3(bfor(R.n)), dim3(kB), 0, b->stream, R.n, R.poff, (const int *)b->hpos,
+                     (const double *)b->sx, (const double *)b->sy, (const double *)b->sp, b->io);
+  B_TRY(hipMemcpyAsync(state, b->io, bytes, hipMemcpyDeviceToHost, b->stream));
+  B_TRY(hipStreamSynchronize(b->stream));
   return check_launch("batch get state");
 }
 
@@ -893,8 +898,8 @@ spc2_status spc2_batch_set_omega(spc2_batch_t b, int32_t r, const double *omega)
   const Rep &R = b->reps[r];
   if (spc2_status st = ensure_io(*b, (size_t)R.n)) return st;
   B_TRY(hipMemcpyAsync(b->io, omega, sizeof(double) * R.n, hipMemcpyHostToDevice, b->stream));
-  hipLaunchKernelGGL(k_b_to_home, dim3(bfor(R.n)), dim3(kB), 0, b->stream, R.n, R.poff, (const int *)b->hpos,
-                     (const double *)b->io, b->omega);
+  hipLaunchKernelGGL(k_b_to_home, dim3(bfor(R.n)), dim3(kB), 0, b->stream, R.n, R.poff, 1, (const int *)b->hpos,
+                     (const double *)b->io, b->omega, nullptr, nullptr);
   B_TRY(hipStreamSynchronize(b->stream));
   return check_launch("batch set omega");
 }

@@ -128,7 +128,7 @@ struct Sim {
   // transfer scratch for the ABI's host arrays
   double *spare[16] = {};
   int *spare_i = nullptr;
-  double *io[3] = {};
+  double *io = nullptr;  // 3 n
   Tiles t{};
   // The next stage, written by a pass's epilogue.  Verlet: its tiles and phases
   // (t2.cell aliases t.cell), swapped with t / gp after that launch.  All pairs:
@@ -274,8 +274,8 @@ void launch_verlet_pass1(Sim &s, int epi, double *ox, double *oy, double *op, co
 void launch_verlet_pass2(Sim &s, int epi, double *a0, double *a1, const StepArgs &sa);
 void launch_drift(Sim &s, double *out);
 // spc2_misc.hip
-void launch_to_home(Sim &s, const double *src_id, double *dst_home);
-void launch_from_home(Sim &s, const double *src_home, double *dst_id);
+void launch_to_home(Sim &s, const double *aos, double *const *dst, int comps);
+void launch_from_home(Sim &s, double *const *src, int comps, double *aos);
 void launch_from_home_int(Sim &s, const int *src_home, int *dst_id);
 void launch_slot_to_id(Sim &s, const int *id_of_slot, const double *src_slot, double *dst_id);
 void launch_identity_homes(Sim &s);

@@ -91,14 +91,23 @@ __global__ __launch_bounds__(kBlock) void k_init_state(int n, double Lx, double 
 }
 
 // id-ordered host arrays <-> home-ordered device arrays
-__global__ __launch_bounds__(kBlock) void k_to_home(int n, const int *hpos, const double *src_id, double *dst_home) {
-  int id = blockIdx.x * blockDim.x + threadIdx.x;
-  if (id < n) dst_home[hpos[id]] = src_id[id];
+// AoS array by particle id, comps (1 to 3) components, to home-ordered arrays and
+// back, a thread per home.
+struct Comps {
+  double *p[3];
+};
+__global__ __launch_bounds__(kBlock) void k_to_home(int n, int comps, const int *hid, const double *aos, Comps dst) {
+  const int h = blockIdx.x * blockDim.x + threadIdx.x;
+  if (h >= n) return;
+  const double *src = aos + (size_t)hid[h] * comps;
+  for (int c = 0; c < comps; ++c) dst.p[c][h] = src[c];
 }
 
-__global__ __launch_bounds__(kBlock) void k_from_home(int n, const int *hpos, const double *src_home, double *dst_id) {
-  int id = blockIdx.x * blockDim.x + threadIdx.x;
-  if (id < n) dst_id[id] = src_home[hpos[id]];
+__global__ __launch_bounds__(kBlock) void k_from_home(int n, int comps, const int *hid, Comps src, double *aos) {
+  const int h = blockIdx.x * blockDim.x + threadIdx.x;
+  if (h >= n) return;
+  double *dst = aos + (size_t)hid[h] * comps;
+  for (int c = 0; c < comps; ++c) dst[c] = src.p[c][h];
 }
 
 // Per-slot values to particle-id order through a slot -> id map.
@@ -200,14 +209,18 @@ void launch_order_param(Sim &s, double *out2) {
   hipLaunchKernelGGL(k_order_final, dim3(1), dim3(kBlock), 0, s.stream, nb, (const double *)s.red, out2);
 }
 
-void launch_to_home(Sim &s, const double *src_id, double *dst_home) {
-  ensure_hpos(s);
-  hipLaunchKernelGGL(k_to_home, dim3(blocks_for(s.n)), dim3(kBlock), 0, s.stream, s.n, s.hpos, src_id, dst_home);
+void launch_to_home(Sim &s, const double *aos, double *const *dst, int comps) {
+  Comps c{};
+  std::copy(dst, dst + comps, c.p);
+  hipLaunchKernelGGL(k_to_home, dim3(blocks_for(s.n)), dim3(kBlock), 0, s.stream, s.n, comps, (const int *)s.hid, aos,
+                     c);
 }
 
-void launch_from_home(Sim &s, const double *src_home, double *dst_id) {
-  ensure_hpos(s);
-  hipLaunchKernelGGL(k_from_home, dim3(blocks_for(s.n)), dim3(kBlock), 0, s.stream, s.n, s.hpos, src_home, dst_id);
+void launch_from_home(Sim &s, double *const *src, int comps, double *aos) {
+  Comps c{};
+  std::copy(src, src + comps, c.p);
+  hipLaunchKernelGGL(k_from_home, dim3(blocks_for(s.n)), dim3(kBlock), 0, s.stream, s.n, comps, (const int *)s.hid, c,
+                     aos);
 }
 
 void launch_slot_to_id(Sim &s, const int *id_of_slot, const double *src_slot, double *dst_id) {

@@ -107,3 +107,15 @@ def test_chunk_length_leaves_the_bits(n, method):
         s.set_state(st)
         s.step(method, 0.01, 0, 3)
         assert np.array_equal(b.get_state(0), s.get_state())
+
+
+@pytest.mark.parametrize("n", [1, 255, 257, 5003])
+@pytest.mark.parametrize("path", ["cells", "all_pairs", "verlet"])
+def test_state_goes_up_and_comes_back(path, n):
+    st = state_of(n, None, seed=n)
+    with spc2.Sim(model("chimera", "fp64", n, path)) as s:
+        s.set_state(st)
+        assert np.array_equal(s.get_state(), st)
+    with spc2.Batch([model("chimera", "fp64", n, "auto"), model("vortex", "fp64", 7, "auto")]) as b:
+        b.set_state(0, st)
+        assert np.array_equal(b.get_state(0), st)
