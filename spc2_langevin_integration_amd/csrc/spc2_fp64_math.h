@@ -19,12 +19,14 @@ constexpr double kPiHi = 0x1.921fb54442d18p+1, kPiLo = 0x1.1a62633145c07p-53, kI
 constexpr double kRound = 0x1.8p+52;
 constexpr double kTrigMax = 0x1p+45;  // larger arguments, infinities and NaN take the library functions
 
-// a * b + c with c in its own registers.  The compiler forms an accumulating
-// v_fmac for these and copies each coefficient into its destination first, 7
-// more instructions per sine.
+// a * b + c, c a constant in scalar registers.  The compiler forms an accumulating
+// v_fmac for these and copies each coefficient into its destination first, 7 more
+// instructions per sine; in vector registers the coefficients, hoisted out of the
+// walks, took 14 of them (a wavefront per SIMD less in the chimera cell walks: 143
+// against 134 us in pass 1 at N = 262,144, 168 against 160 in pass 2).
 __device__ __forceinline__ double fma3(double a, double b, double c) {
   double d;
-  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "s"(c));
   return d;
 }
 

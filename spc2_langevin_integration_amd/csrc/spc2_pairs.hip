@@ -25,8 +25,12 @@ inline int blocks_for(long long n, int b = kBlock) { return (int)((n + b - 1) / 
 // Pass-1 and pass-2 kernels over linked cells
 // =============================================================================
 
+// (FP64: three wavefronts per SIMD at the least, for which the vortex passes keep 4 to
+// 33 registers in scratch.  With two, N = 160,000: 86 us for 76 of RK4's pass; N =
+// 100,000, SRK: 50 for 52 and 91 for 89.)
 template <class Acc, int PREC, int EPI>
-__global__ __launch_bounds__(kBlock) void k_pass1_lds(KParams P, const int *__restrict__ start, Tiles t,
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(PREC == P64 ? 3 : 1))) void k_pass1_lds(KParams P, const int *__restrict__ start, Tiles t,
                                                       const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                                       const double *gp, EpiCtx e, unsigned long long *counts) {
   extern __shared__ float4 dyn_lds[];
@@ -36,7 +40,8 @@ __global__ __launch_bounds__(kBlock) void k_pass1_lds(KParams P, const int *__re
 }
 
 template <class Acc, int PREC, int EPI>
-__global__ __launch_bounds__(kBlock) void k_pass2_lds(KParams P, const int *__restrict__ start, Tiles t,
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(PREC == P64 ? 3 : 1))) void k_pass2_lds(KParams P, const int *__restrict__ start, Tiles t,
                                                       const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                                       const double *gp, EpiCtx e) {
   extern __shared__ float4 dyn_lds[];
