@@ -391,6 +391,113 @@ __device__ __forceinline__ int visit_lds64(Acc &acc, const Src64 &src, const Seg
   return cand - 1;
 }
 
+// The FP32 vortex pass 2: as visit_lds64, one lane to a particle.  Its term (60
+// instructions, and the cohesion's) stood behind the distance test, where nearly
+// every candidate of a wavefront ran it for the third of the lanes that needed it;
+// the partners' terms, and their order in each sum, are visit_lds's.  Two partners'
+// terms are formed together: at the sizes of one replica a SIMD holds one wavefront,
+// and the chain of operations bounds it.  N = 1000: 48 -> 33
+// us, N = 50,000: 51 -> 39, N = 400,000: 118 -> 109.
+template <class Acc>
+__device__ __forceinline__ void visit_near32(Acc &acc, const Src32 &src, const SegShared &sh, int ncol, int qi, int ei,
+                                             NearWords *near, const KParams &P) {
+  const int me = threadIdx.x;
+  const float lim = fmaxf(P.rho2f_hi, P.xr2f_hi);  // beyond it no decision finds a partner
+  const float ol = acc.co.col(-1), oc = acc.co.col(0), orr = acc.co.col(1);
+  struct Row {  // a stencil row's columns and offset, for the candidates from `first` on
+    int b1, b2;
+    float oy;
+  };
+  const auto row = [&](int r) {
+    return Row{sh.off[r * ncol + qi], sh.off[r * ncol + qi + 1], (float)(r - 1) * P.hyf - acc.yl};
+  };
+  const auto row_of = [&](int m) { return row((m >= sh.off[ncol]) + (m >= sh.off[2 * ncol])); };
+  const auto ox = [&](const Row &w, int m) { return m < w.b1 ? ol : (m >= w.b2 ? orr : oc); };
+  CohQueue64 cq;
+  int r = 0, m0 = sh.off[qi - 1], hi = sh.off[qi + 2];
+  Row at = row(0);
+  bool more = true;
+  while (more) {
+    int words = 0;
+    while (words < kNearWords) {
+      while (m0 >= hi && r < 2) {
+        ++r;
+        m0 = sh.off[r * ncol + qi - 1];
+        hi = sh.off[r * ncol + qi + 2];
+        at = row(r);
+      }
+      if (m0 >= hi) break;
+      const int cnt = min(32, hi - m0);
+      uint32_t word = 0;
+      for (int u = 0; u < cnt; u += 4) {  // those past the run are masked off
+        uint32_t b = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float2 v = *(const float2 *)(src.f4 + m0 + u + k);
+          const float dx = v.x + ox(at, m0 + u + k), dy = v.y + at.oy;
+          b |= __builtin_fmaf(dx, dx, dy * dy) <= lim ? 1u << k : 0u;
+        }
+        word |= b << u;
+      }
+      if (cnt < 32) word &= (1u << cnt) - 1u;
+      if ((unsigned)(ei - m0) < 32u) word &= ~(1u << (ei - m0));  // not the particle itself
+      near->bits[words][me] = word;
+      near->first[words][me] = (uint16_t)m0;
+      ++words;
+      m0 += 32;
+    }
+    more = __any(m0 < hi || r < 2);
+    uint32_t m = 0;
+    int w = 0, first = 0;
+    Row in = at;
+    bool left = true;
+    while (left) {
+      if (m == 0 && w < words) {
+        m = near->bits[w][me];
+        first = near->first[w][me];
+        in = row_of(first);
+        ++w;
+      }
+      if (m != 0) {
+        const int c0 = first + __builtin_ctz(m);
+        m &= m - 1u;
+        const bool two = m != 0;
+        const int c1 = two ? first + __builtin_ctz(m) : c0;
+        m &= m - 1u;  // (0 stays 0)
+        const float4 v0 = src.f4[c0], v1 = src.f4[c1];
+        const float a0 = src.aj[c0], a1 = src.aj[c1];
+        const float dx0 = v0.x + ox(in, c0), dy0 = v0.y + in.oy, dx1 = v1.x + ox(in, c1), dy1 = v1.y + in.oy;
+        const float s0 = __builtin_fmaf(dx0, dx0, dy0 * dy0), s1 = __builtin_fmaf(dx1, dx1, dy1 * dy1);
+        bool inr0, inc0, inn0, inr1, inc1, inn1;
+        acc.decide(src, c0, s0, inr0, inc0, inn0, P);
+        acc.decide(src, c1, s1, inr1, inc1, inn1, P);
+        const auto t0 = acc.align(v0, dx0, dy0, s0, inn0, a0, P), t1 = acc.align(v1, dx1, dy1, s1, inn1, a1, P);
+        if (inr0) {
+          acc.A0.add_prod(t0.w, t0.cph);
+          acc.A1.add(t0.t);
+        }
+        if (inr1 & two) {
+          acc.A0.add_prod(t1.w, t1.cph);
+          acc.A1.add(t1.t);
+        }
+        if (inc0) cq.push(c0);
+        if (inc1 & two) cq.push(c1);
+      }
+      left = __any(m != 0 || w < words);
+      if (!left || __any(cq.n > CohQueue64::kFull - 2)) {
+        while (cq.n > 0) {
+          --cq.n;
+          const int c = (int)((cq.q >> (16 * cq.n)) & 0xffffu);
+          const Row z = row_of(c);
+          const float4 v = src.f4[c];
+          const float dx = v.x + ox(z, c), dy = v.y + z.oy;
+          acc.cohesion(src, c, v, dx, dy, __builtin_fmaf(dx, dx, dy * dy), P);
+        }
+      }
+    }
+  }
+}
+
 // Same visit over the global tiles, cell by cell (slot k in cell c); the FP64
 // forms' lane g takes the run of each stencil row that visit_lds64 gives it.
 template <class Acc, class S>
@@ -440,7 +547,7 @@ __device__ __forceinline__ bool wraps(const KParams &P, const Seg &g) {
   return g.cx0 < 1 || g.cx0 + g.W >= P.nx || g.cy < 1 || g.cy + 1 >= P.ny;
 }
 
-// The plain FP64 form's words, after the staged tiles.
+// The words of the walks that find the near partners first, after the staged tiles.
 template <int PREC, int PASS>
 __device__ __forceinline__ NearWords *near_words(void *dyn_lds, const KParams &P) {
   return (NearWords *)((char *)dyn_lds + (size_t)P.lds_cap * LdsTile<PREC, PASS>::bytes);
@@ -562,7 +669,9 @@ __device__ __forceinline__ void pass2_segment(const KParams &P, const int *__res
         else hi = mid - 1;
       }
       acc.init(lt.src(), ei, k, t, P, in);
-      if constexpr (PREC == P32K)
+      if constexpr (HasNear32<Acc>::value)
+        visit_near32(acc, lt.src(), sh, g.ncol, lo, ei, near_words<PREC, 2>(dyn_lds, P), P);
+      else if constexpr (PREC == P32K)
         visit_lds(acc, lt.src(), sh, g.ncol, lo, ei, P);
       else
         visit_lds64(acc, lt.src(), sh, g.ncol, lo, ei, gl, wraps(P, g), near_words<PREC, 2>(dyn_lds, P), P);

@@ -223,8 +223,6 @@ constexpr int kLanes64 = 2;
 constexpr long long kLanesFill = 131072;
 constexpr double kMfmaPerCell = 12.0;
 
-int lds_near_bytes(int prec) { return prec == P64 ? (int)sizeof(NearWords) : 0; }
-
 // bytes per staged candidate of the larger pass
 int lds_elem_bytes(int prec) {
   switch (prec) {
@@ -266,6 +264,8 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
   k.mfma = 0;
   k.aj = k.raj = 1.0;
   k.bin_cap = 0;
+  k.near[0] = prec == P64 ? (int)sizeof(NearWords) : 0;
+  k.near[1] = prec == P64 || (prec == P32K && system == SPC2_VORTEX) ? (int)sizeof(NearWords) : 0;
   if (!k.linked) {
     k.seg_w = k.segs = 1;
     k.lds_cap = 0;
@@ -308,7 +308,7 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
     cap = std::min(cap, (kLdsBytes - MfmaLds<2>::tail_bytes) / MfmaLds<2>::tile_bytes * kMfmaTile);
   } else {
     cap = (int)std::ceil((halo + 160.0) / 64.0) * 64;
-    cap = std::min(cap, (kLdsBytes - lds_near_bytes(prec)) / lds_elem_bytes(prec));
+    cap = std::min(cap, (kLdsBytes - k.near[1]) / lds_elem_bytes(prec));
   }
   if (const char *env = std::getenv("SPC2_LDS_CAP")) cap = std::max(0, std::min(cap, std::atoi(env)));
   k.lds_cap = k.mfma ? cap / kMfmaTile * kMfmaTile : cap;
@@ -323,7 +323,7 @@ size_t pair_lds_bytes(const KParams &k, int prec, int pass) {
     case P64: elem = pass == 1 ? LdsTile<P64, 1>::bytes : LdsTile<P64, 2>::bytes; break;
     default: elem = pass == 1 ? LdsTile<P64F, 1>::bytes : LdsTile<P64F, 2>::bytes;
   }
-  return (size_t)k.lds_cap * (size_t)elem + (size_t)lds_near_bytes(prec);
+  return (size_t)k.lds_cap * (size_t)elem + (size_t)k.near[pass - 1];
 }
 
 // A single handle's pair workgroups.  The matrix-core passes of a small system are

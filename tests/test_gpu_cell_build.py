@@ -119,3 +119,25 @@ def test_state_goes_up_and_comes_back(path, n):
     with spc2.Batch([model("chimera", "fp64", n, "auto"), model("vortex", "fp64", 7, "auto")]) as b:
         b.set_state(0, st)
         assert np.array_equal(b.get_state(0), st)
+
+
+# the FP32 vortex pass 2 that finds the near partners first, against its walk over the global tiles: no, few and
+# many partners (more words of bits than are kept at once, full cohesion queues), boxes that wrap
+@pytest.mark.parametrize("spread", [None, 0.5, 0.12])
+@pytest.mark.parametrize("n", [1, 65, 700, 2049])
+@pytest.mark.parametrize("rho", [0.24, 0.09])
+def test_near_partners_first_leaves_the_bits(monkeypatch, rho, n, spread):
+    out = []
+    for cap in (None, "0"):
+        if cap is not None:
+            monkeypatch.setenv("SPC2_LDS_CAP", cap)
+        p = spc2.params("vortex", "fp32k", "cells", n=n, L=1.0, rho=rho, D=0.02, seed=5, velocity=0.1, mu_plus=10.0,
+                        mu_minus=8.0, xi_a=0.4 * rho, xi_r=0.3 * rho, kappa=2.0)
+        with spc2.Sim(p) as s:
+            s.set_state(state_of(n, spread))
+            rhs = s.eval_rhs_ito()
+            s.step("srk", 0.005, 0, 2)
+            out.append((*rhs, s.get_state()))
+    for a, b in zip(*out):
+        assert np.isfinite(a).all()
+        assert np.array_equal(a, b)
