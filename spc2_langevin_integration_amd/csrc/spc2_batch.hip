@@ -344,12 +344,15 @@ __global__ __launch_bounds__(kB) void k_b_gather(int n, const int *src_hpos, int
   if (i < n) dst[dst_off + i] = src[src_hpos[src_off + i]];
 }
 
-// Order parameter sums per replica (one workgroup per replica, FP64).
+// Order parameter sums per replica (FP64), in kOrderSplit parts that the caller adds:
+// with one workgroup per replica the largest set the time (290 us for 24 replicas of
+// up to 200,000 particles).
+constexpr int kOrderSplit = 16;
 __global__ __launch_bounds__(kB) void k_b_order(const Rep *reps, const double *sp, double *out) {
   __shared__ double sc[kB], ss[kB];
-  const Rep &R = reps[blockIdx.x];
+  const Rep &R = reps[blockIdx.x / kOrderSplit];
   double c = 0.0, s = 0.0;
-  for (int i = threadIdx.x; i < R.n; i += kB) {
+  for (int i = blockIdx.x % kOrderSplit * kB + threadIdx.x; i < R.n; i += kOrderSplit * kB) {
     double sn, cs;
     sincos(sp[R.poff + i], &sn, &cs);
     c += cs;
@@ -548,7 +551,7 @@ spc2_status alloc_batch(spc2_batch &b) {
       BA(b.t.c, n); BA(b.t.s, n);
     }
   }
-  BA(b.red, 2 * (size_t)b.count);
+  BA(b.red, 2 * (size_t)b.count * kOrderSplit);
 #undef BA
   B_TRY(hipMemsetAsync(b.count_, 0, sizeof(int) * nc, b.stream));
   B_TRY(hipMemsetAsync(b.omega, 0, sizeof(double) * n, b.stream));
@@ -743,7 +746,7 @@ uint64_t spc2_batch_footprint(const spc2_params *p) {
   const size_t tile = p->precision == SPC2_FP32_KAHAN ? 16 + 16 : (p->precision == SPC2_FP64 ? 24 : 40);
   // 11 doubles (state, omega, stage, spare), 11 ints, tiles; 2 ints per cell
   // (SE stepping; the first SRK step adds 36 B per particle)
-  return n * (11 * 8 + 11 * 4 + tile) + cells * 8 + sizeof(Rep) + 64;
+  return n * (11 * 8 + 11 * 4 + tile) + cells * 8 + sizeof(Rep) + 64 + 16 * kOrderSplit;
 }
 
 spc2_status spc2_batch_create_from(const spc2_params *replicas, int32_t count, spc2_batch_t prev,
@@ -920,14 +923,20 @@ spc2_status spc2_batch_steps_done(spc2_batch_t b, int64_t *steps) {
 
 spc2_status spc2_batch_order_parameters(spc2_batch_t b, double *R, double *psi) {
   if (check_batch(b) || !R || !psi) return set_error(SPC2_ERR_INVALID, "null argument");
-  hipLaunchKernelGGL(k_b_order, dim3(b->count), dim3(kB), 0, b->stream, (const Rep *)b->d_reps, (const double *)b->sp,
+  hipLaunchKernelGGL(k_b_order, dim3(b->count * kOrderSplit), dim3(kB), 0, b->stream, (const Rep *)b->d_reps, (const double *)b->sp,
                      b->red);
   if (spc2_status st = check_launch("batch order parameter")) return st;
-  std::vector<double> s(2 * (size_t)b->count);
+  std::vector<double> s(2 * (size_t)b->count * kOrderSplit);
   B_TRY(hipMemcpyAsync(s.data(), b->red, sizeof(double) * s.size(), hipMemcpyDeviceToHost, b->stream));
   B_TRY(hipStreamSynchronize(b->stream));
   for (int r = 0; r < b->count; ++r) {
-    const double c = s[2 * r] / b->reps[r].n, sn = s[2 * r + 1] / b->reps[r].n;
+    double c = 0.0, sn = 0.0;
+    for (int q = r * kOrderSplit; q < (r + 1) * kOrderSplit; ++q) {
+      c += s[2 * q];
+      sn += s[2 * q + 1];
+    }
+    c /= b->reps[r].n;
+    sn /= b->reps[r].n;
     R[r] = std::sqrt(c * c + sn * sn);
     psi[r] = std::atan2(sn, c);
   }
