@@ -45,8 +45,12 @@
 // 2 160 us).  On the way there: four groups per tile read held 168 registers (3
 // wavefronts, 735 us); the chunk's frame for the products instead of the cell's
 // needs a band 30 times wider, whose FP64 decisions cost more than the shift.
-// Taken from kMfmaPerCell = 12 particles per cell: below that most of a group's 16
-// centres are padding.  Compiled with -ffp-contract=off.
+// Taken from kMfmaPerCell = 20 particles per cell; in sparser cells more of a group's
+// 16 centres are padding.  At N = 200,000, pass 1 and both SRK passes, the scalar
+// walk against this: 24 and 71 against 34 and 75 us at 11 per cell, 27 and 81 against
+// 34 and 74 at 16, 33 and 96 against 33 and 80 at 24.  (A small system alone would
+// gain from 9 on: 20 and 43 against 12 and 27 us at N = 20,000; but the choice is a
+// replica's too, whose batch fills the device.)  Compiled with -ffp-contract=off.
 #pragma once
 
 #include "spc2_lds_stencil.h"

@@ -221,7 +221,7 @@ void pass2_sys(Sim &s, int epi, const EpiCtx &e) {
 
 constexpr int kLanes64 = 2;
 constexpr long long kLanesFill = 131072;
-constexpr double kMfmaPerCell = 12.0;
+constexpr double kMfmaPerCell = 20.0;
 
 // bytes per staged candidate of the larger pass
 int lds_elem_bytes(int prec) {

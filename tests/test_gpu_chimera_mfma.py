@@ -23,7 +23,7 @@ DT, RHO = 0.005, 0.1
 # (cells per side, mean particles per cell): around the least filling that takes
 # the passes, one to several groups of 16 centres, grids whose chunks wrap around
 CASES = [(4, 11.9), (4, 12.1), (4, 40.0), (5, 15.5), (5, 47.0), (7, 49.0), (9, 70.0), (6, 130.0), (23, 13.0),
-         (31, 40.0)]
+         (31, 40.0), (4, 19.9), (4, 20.1), (5, 20.4), (7, 24.0), (23, 21.0)]
 
 
 def system(cells, filling, prec="fp32k", sigma=1.3, seed=5):
