@@ -27,10 +27,12 @@ inline int blocks_for(long long n, int b = kBlock) { return (int)((n + b - 1) / 
 
 // (FP64: three wavefronts per SIMD at the least, for which the vortex passes keep 4 to
 // 33 registers in scratch.  With two, N = 160,000: 86 us for 76 of RK4's pass; N =
-// 100,000, SRK: 50 for 52 and 91 for 89.)
+// 100,000, SRK: 50 for 52 and 91 for 89.  FP32 pass 1: four, which the vortex passes
+// that bin their next stage miss by 3 to 5 registers: 153 for 130 us at N = 1M, where
+// the bin kernel of its own takes 17 and the pass without it 117.)
 template <class Acc, int PREC, int EPI>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(PREC == P64 ? 3 : 1))) void k_pass1_lds(KParams P, const int *__restrict__ start, Tiles t,
+__attribute__((amdgpu_waves_per_eu(PREC == P64 ? 3 : (PREC == P32K ? 4 : 1)))) void k_pass1_lds(KParams P, const int *__restrict__ start, Tiles t,
                                                       const int *__restrict__ slot_h, const int *__restrict__ slot_id,
                                                       const double *gp, EpiCtx e, unsigned long long *counts) {
   extern __shared__ float4 dyn_lds[];
