@@ -863,7 +863,12 @@ spc2_status spc2_step_ex(spc2_sim_t h, int32_t method, double dt, int64_t step0,
         s.drift += (method == SPC2_SRK ? srk_step_reach(s, dt) : std::fabs(s.P.v0) * dt) * (1.0 + 1e-12);
     }
     maybe_rehome(s);
-    if (spc2_status st = check_launch("step")) return st;
+    if (spc2_status st = check_launch("step")) {
+      // the next call stages and bins afresh
+      s.staged = false;
+      (void)hipMemsetAsync(s.count, 0, sizeof(int) * 4 * (size_t)s.count_stride, s.stream);
+      return st;
+    }
   }
   HIP_TRY(hipStreamSynchronize(s.stream));
   return SPC2_OK;
