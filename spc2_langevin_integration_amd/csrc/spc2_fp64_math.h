@@ -89,8 +89,9 @@ __device__ __forceinline__ bool phase_fits(double p) { return __builtin_fabs(p) 
 
 // sqrt(a) of a squared separation: the hardware estimate of 1 / sqrt(a) and two
 // Goldschmidt steps with a residual correction, the correctly rounded root for
-// normal a without the library's scaling of denormals; 0 for a == 0.  For 0 <=
-// a < 1e300 only.
+// normal a without the library's scaling of denormals; 0 for a == 0 and NaN for
+// NaN (a separation that is not finite fails every test of the root, as with the
+// library's).  For 0 <= a < 1e300 and NaN only.
 __device__ __forceinline__ double sqrt_sep(double a) {
   const double y = __builtin_amdgcn_rsq(a);
   double g = a * y, h = 0.5 * y;
@@ -101,7 +102,7 @@ __device__ __forceinline__ double sqrt_sep(double a) {
   g = __builtin_fma(e, h, g);
   e = __builtin_fma(-g, g, a);
   g = __builtin_fma(e, h, g);
-  return a > 0.0 ? g : 0.0;
+  return a > 0.0 ? g : a;
 }
 
 // a / c for a launch constant c with rc = 1 / c rounded: the product and one
