@@ -542,9 +542,12 @@ __device__ __forceinline__ int visit_global(Acc &acc, const S &src, const int *s
 }
 
 // A halo column or row of the workgroup wraps: without one the candidates'
-// separations need no min-image.
+// separations need no min-image.  A candidate is less than two cells away along an
+// axis, so that with four cells or more the plain difference is the nearer image;
+// with three it may lie beyond half the box, and a cutoff wider than a cell (xi_r)
+// then finds its nearer image.
 __device__ __forceinline__ bool wraps(const KParams &P, const Seg &g) {
-  return g.cx0 < 1 || g.cx0 + g.W >= P.nx || g.cy < 1 || g.cy + 1 >= P.ny;
+  return g.cx0 < 1 || g.cx0 + g.W >= P.nx || g.cy < 1 || g.cy + 1 >= P.ny || P.nx < 4 || P.ny < 4;
 }
 
 // The words of the walks that find the near partners first, after the staged tiles.

@@ -1,5 +1,5 @@
 """Positions at the edges of what the passes take, against the oracle: positions
-that are not finite.  Bars: tests/_parity.py."""
+that are not finite, boxes of three cells along an axis.  Bars: tests/_parity.py."""
 import os
 import sys
 
@@ -63,3 +63,26 @@ def test_position_that_is_not_finite_is_no_partner(system, path, prec, bad):
     st = state_of(n)
     st[3 * 17] = bad
     check(p, orc, st, prec, f"{system} {path} {prec} {bad}")
+
+
+# three cells along an axis and partners beyond a cell's side: from the middle cells some lie more than half the box
+# away, so that the nearer image counts although no halo wraps (3 x 3 cells forced, then 4 x 3 as the reference takes)
+@pytest.mark.parametrize("Lx,Ly,rho,xi_r", [(1.0, 1.0, 0.33, 0.45), (1.0, 0.8, 0.25, 0.3), (0.8, 1.0, 0.25, 0.3)])
+@pytest.mark.parametrize("filling", [9, 61])
+@pytest.mark.parametrize("prec", ["fp64", "fp64f"])
+def test_three_cells_along_an_axis(monkeypatch, prec, filling, Lx, Ly, rho, xi_r):
+    n = filling * int(Lx / rho) * int(Ly / rho)
+    p, orc = systems("vortex", prec, "cells", n, Lx, Ly, rho, 0.2 * rho, xi_r)
+    if Lx < Ly:  # the oracle takes all pairs there (rho > Lx / 4): the walks against each other only
+        orc = None
+    st, out = state_of(n, Lx, Ly), []
+    for cap in (None, "0"):
+        if cap is not None:
+            monkeypatch.setenv("SPC2_LDS_CAP", cap)
+        if orc is not None:
+            check(p, orc, st, prec, f"{prec} {Lx} x {Ly}")
+        with spc2.Sim(p) as s:
+            s.set_state(st)
+            out.append((*s.neighbour_counts(), *s.eval_rhs_ito()))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
