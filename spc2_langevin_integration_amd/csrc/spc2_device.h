@@ -23,11 +23,18 @@ struct Box {
 // ClassAEffectiveParticleDistance, PeriodicBoundaryConditions.cpp:22-34:
 // dx = x_j - x_i; dx -= int(dx * 2.0 / L) * L (truncation toward zero).  Three
 // instructions: the truncation stays in FP64, and the fused product rounds as
-// the separate one does, since the count of boxes (0, +-1; +-2 at most for
-// stage positions just outside the box) times L is exact.  r2L = 2 (1 / L), a
-// launch constant: the product is that of d * 2.0 * (1 / L).
+// the separate one does while the count of boxes times L is exact, that is for
+// counts of 0, +-1 and +-2: positions in the box or within half a box of its
+// edge, as the cell and list walks have them (their stages are wrapped).  r2L =
+// 2 (1 / L), a launch constant: the product is that of d * 2.0 * (1 / L).
 __device__ __forceinline__ double min_image(double d, double L, double r2L) {
   return __builtin_fma(-__builtin_trunc(d * r2L), L, d);
+}
+
+// The same for any positions (the all-pairs path never wraps its stages, and a
+// state may lie boxes away): the product of its own that the reference rounds.
+__device__ __forceinline__ double min_image_any(double d, double L, double r2L) {
+  return d - __builtin_trunc(d * r2L) * L;
 }
 
 // Scalar wrap, PeriodicBoundaryConditions.cpp:117-121: x - floor(x / L) * L.

@@ -1718,8 +1718,8 @@ __device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, int g, c
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = PREC == P32K ? 0.0 : gp[j];
       const float4 tj = PREC == P32K ? tiles[j] : float4{};
-      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
+      const double dx = min_image_any(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image_any(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       if ((r2 <= P.rho2) & (j != i)) {
         if constexpr (PREC == P64) {
@@ -1754,8 +1754,8 @@ __device__ __forceinline__ void allpairs_pass1(const KParams &P, int i, int g, c
 #pragma unroll 1
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = gp[j];
-      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
+      const double dx = min_image_any(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image_any(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       // (partners beyond both radii cannot pass the tests of the root below)
       if ((r2 > P.outer2 * 1.000000000001) | (j == i)) continue;
@@ -1818,8 +1818,8 @@ __device__ __forceinline__ void allpairs_pass2(const KParams &P, int i, int g, c
 #pragma unroll 1
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = gp[j], aj = aphi[j];
-      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
+      const double dx = min_image_any(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image_any(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       if ((r2 > P.outer2 * 1.000000000001) | (j == i)) continue;
       const double dr = sqrt_sep(r2);
@@ -1849,8 +1849,8 @@ __device__ __forceinline__ void allpairs_pass2(const KParams &P, int i, int g, c
 #pragma unroll 1
     for (int j = g; j < P.n; j += kApLanes) {
       const double pj = gp[j], aj = aphi[j];
-      const double dx = min_image(gx[j] - xi, P.Lx, P.r2Lx);
-      const double dy = min_image(gy[j] - yi, P.Ly, P.r2Ly);
+      const double dx = min_image_any(gx[j] - xi, P.Lx, P.r2Lx);
+      const double dy = min_image_any(gy[j] - yi, P.Ly, P.r2Ly);
       const double r2 = dx * dx + dy * dy;
       if ((r2 <= P.rho2) & (n != 0) & (j != i)) {
         const double cph = cos_term(pj - pi - P.alpha);

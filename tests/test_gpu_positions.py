@@ -1,5 +1,6 @@
 """Positions at the edges of what the passes take, against the oracle: positions
-that are not finite, boxes of three cells along an axis.  Bars: tests/_parity.py."""
+that are not finite, boxes of three cells along an axis, positions
+several boxes apart.  Bars: tests/_parity.py."""
 import os
 import sys
 
@@ -86,3 +87,17 @@ def test_three_cells_along_an_axis(monkeypatch, prec, filling, Lx, Ly, rho, xi_r
             out.append((*s.neighbour_counts(), *s.eval_rhs_ito()))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+# positions several boxes apart on the all-pairs path, rho the reference's separation itself: its product of the box
+# count (3, 5) and L is rounded, and a fused one puts the partner a hair beyond rho
+@pytest.mark.parametrize("L,d,rho", [(0.7, 1.107265286604193, 0.9927347133958067),
+                                     (1.7, 2.7338815754156287, 2.366118424584371),
+                                     (1.1, 3.213312990181401, 2.286687009818599)])
+@pytest.mark.parametrize("prec", ["fp64", "fp32k", "fp64f"])
+@pytest.mark.parametrize("system", ["chimera", "vortex"])
+def test_all_pairs_several_boxes_apart(system, prec, L, d, rho):
+    p, orc = systems(system, prec, "all_pairs", 2, L, L, rho)
+    st = np.array([0.0, 0.1, 1.0, d, 0.1, 2.5])
+    assert list(O.neighbour_counts(orc, st)[0]) == [1, 1]
+    check(p, orc, st, prec, f"{system} {prec}")
