@@ -249,7 +249,7 @@ spc2_status alloc_all(Sim &s) {
 spc2_status upload_aos(Sim &s, const double *aos, double *const *dst, int comps) {
   HIP_TRY(hipMemcpyAsync(s.io, aos, sizeof(double) * (size_t)comps * (size_t)s.n, hipMemcpyHostToDevice, s.stream));
   launch_to_home(s, s.io, dst, comps);
-  return SPC2_OK;
+  return check_launch("upload");
 }
 
 spc2_status download_aos(Sim &s, double *aos, double *const *src, int comps) {
@@ -257,6 +257,20 @@ spc2_status download_aos(Sim &s, double *aos, double *const *src, int comps) {
   HIP_TRY(hipMemcpyAsync(aos, s.io, sizeof(double) * (size_t)comps * (size_t)s.n, hipMemcpyDeviceToHost, s.stream));
   HIP_TRY(hipStreamSynchronize(s.stream));
   return SPC2_OK;
+}
+
+// check_launch of a call that builds cells or stages ahead.  If a launch failed, a
+// binning may have run without the sort that takes it and clears the other set of
+// counts, and a later build would add to what was left (slots beyond n): the counts
+// are cleared and the next build stages and bins afresh.
+spc2_status check_build(Sim &s, const char *what) {
+  const spc2_status st = check_launch(what);
+  if (st) {
+    s.staged = s.tile_fresh = s.built = false;
+    s.vnext = 0;
+    (void)hipMemsetAsync(s.count, 0, sizeof(int) * 4 * (size_t)s.count_stride, s.stream);
+  }
+  return st;
 }
 
 // Verlet list from the positions s + kcdt * kprev (the state when kprev is
@@ -280,7 +294,7 @@ spc2_status verlet_build(Sim &s, double *const *kprev, double kcdt, bool k_xy_li
   }
   launch_verlet_count(s, try_lds);
   launch_scan_array(s, s.wmax, s.nw, s.wrow);
-  if (spc2_status st = check_launch("verlet count")) return st;
+  if (spc2_status st = check_build(s, "verlet count")) return st;
   // lane slots sorted by list length pay off when lists are long enough for the
   // saved wavefront iterations and list padding to outweigh the epilogue's
   // scattered accesses (measured on the vortex RK4 pass at 45 entries per
@@ -350,7 +364,7 @@ spc2_status verlet_build(Sim &s, double *const *kprev, double kcdt, bool k_xy_li
   else
     launch_verlet_fill(s);
   HIP_TRY(hipMemsetAsync(s.vlist + (size_t)groups * 256, 0, sizeof(int) * 256 * kVerletSpareGroups, s.stream));
-  if (spc2_status st = check_launch("verlet build")) return st;
+  if (spc2_status st = check_build(s, "verlet build")) return st;
   s.vbuilt = true;
   s.built = false;
   s.tile_fresh = false;
@@ -436,7 +450,7 @@ spc2_status rehome_now(Sim &s) {
   launch_rehome(s);
   s.built = false;
   s.steps_since_rehome = 0;
-  return check_launch("re-homing");
+  return check_build(s, "re-homing");
 }
 
 // After every rehome_every steps, moves the particle arrays to the cell order
@@ -732,7 +746,7 @@ spc2_status spc2_eval_rhs(spc2_sim_t h, const double *k_prev, double k_coef, dou
   build(s, s.kev[1], k_coef * dt);
   StepArgs sa = step_args(s, dt, 0);
   rhs_pass1(s, EPI_K, s.kev[0][0], s.kev[0][1], s.kev[0][2], sa, nullptr, nullptr, nullptr);
-  if (spc2_status st = check_launch("eval_rhs")) return st;
+  if (spc2_status st = check_build(s, "eval_rhs")) return st;
   return download_aos(s, k_next, s.kev[0], 3);
 }
 
@@ -749,7 +763,7 @@ spc2_status spc2_eval_rhs_ito(spc2_sim_t h, double *derivative, double *addition
   StepArgs sa = step_args(s, 0.0, 0);
   rhs_pass1(s, EPI_ITO1, s.der[0], s.der[1], s.der[2], sa, nullptr, nullptr, nullptr);
   rhs_pass2(s, EPI_ITO2, s.add[0], s.add[1], sa);
-  if (spc2_status st = check_launch("eval_rhs_ito")) return st;
+  if (spc2_status st = check_build(s, "eval_rhs_ito")) return st;
   if (spc2_status st = download_aos(s, derivative, s.der, 3)) return st;
   return download_aos(s, additional, s.add, 2);
 }
@@ -863,12 +877,7 @@ spc2_status spc2_step_ex(spc2_sim_t h, int32_t method, double dt, int64_t step0,
         s.drift += (method == SPC2_SRK ? srk_step_reach(s, dt) : std::fabs(s.P.v0) * dt) * (1.0 + 1e-12);
     }
     maybe_rehome(s);
-    if (spc2_status st = check_launch("step")) {
-      // the next call stages and bins afresh
-      s.staged = false;
-      (void)hipMemsetAsync(s.count, 0, sizeof(int) * 4 * (size_t)s.count_stride, s.stream);
-      return st;
-    }
+    if (spc2_status st = check_build(s, "step")) return st;
   }
   HIP_TRY(hipStreamSynchronize(s.stream));
   return SPC2_OK;
@@ -1042,7 +1051,7 @@ spc2_status spc2_neighbour_counts(spc2_sim_t h, int32_t *n_rho, int32_t *n_xi_r)
   const int *id_of_slot = (s.verlet || !s.linked) ? s.hid : s.slot_id;
   launch_slot_to_id(s, id_of_slot, s.n_slot, s.io);
   launch_slot_to_id(s, id_of_slot, s.n2_slot, s.io + s.n);
-  if (spc2_status st = check_launch("neighbour counts")) return st;
+  if (spc2_status st = check_build(s, "neighbour counts")) return st;
   std::vector<double> a((size_t)s.n), b((size_t)s.n);
   HIP_TRY(hipMemcpyAsync(a.data(), s.io, sizeof(double) * (size_t)s.n, hipMemcpyDeviceToHost, s.stream));
   HIP_TRY(hipMemcpyAsync(b.data(), s.io + s.n, sizeof(double) * (size_t)s.n, hipMemcpyDeviceToHost, s.stream));
@@ -1094,7 +1103,7 @@ spc2_status spc2_get_cell_list(spc2_sim_t h, int32_t *cell_of, int32_t *cell_sta
   if (!s.linked) return fail(SPC2_ERR_INVALID, "no cell list on the all-pairs path");
   if (s.verlet) return fail(SPC2_ERR_INVALID, "no per-RHS cell list on the Verlet path");
   build(s, nullptr, 0.0);
-  if (spc2_status st = check_launch("cell list")) return st;
+  if (spc2_status st = check_build(s, "cell list")) return st;
   launch_from_home_int(s, s.cell_of, s.spare_i);
   HIP_TRY(hipMemcpyAsync(cell_of, s.spare_i, sizeof(int) * (size_t)s.n, hipMemcpyDeviceToHost, s.stream));
   HIP_TRY(hipMemcpyAsync(cell_start, s.start, sizeof(int) * ((size_t)s.nc + 1), hipMemcpyDeviceToHost, s.stream));

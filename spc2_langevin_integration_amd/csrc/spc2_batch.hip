@@ -715,7 +715,11 @@ spc2_status run_steps(spc2_batch &b, int method, double dt, int64_t nsteps, cons
       launch_rehome(b);
       b.since_rehome = 0;
     }
-    if (spc2_status st = check_launch("batch step")) return st;
+    if (spc2_status st = check_launch("batch step")) {
+      // a binning may have run without the scan that takes and clears its counts
+      (void)hipMemsetAsync(b.count_, 0, sizeof(int) * (size_t)b.nct, b.stream);
+      return st;
+    }
   }
   B_TRY(hipStreamSynchronize(b.stream));
   for (int r = 0; r < b.count; ++r) b.steps_done[r] += b.reps[r].steps;
