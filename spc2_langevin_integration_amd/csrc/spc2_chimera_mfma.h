@@ -45,7 +45,8 @@
 // 2 160 us).  On the way there: four groups per tile read held 168 registers (3
 // wavefronts, 735 us); the chunk's frame for the products instead of the cell's
 // needs a band 30 times wider, whose FP64 decisions cost more than the shift.
-// Taken from kMfmaPerCell = 20 particles per cell; in sparser cells more of a group's
+// Taken from kMfmaPerCell = 20 particles per cell to where the halo fits the LDS
+// (configure_segments_kp); in sparser cells more of a group's
 // 16 centres are padding.  At N = 200,000, pass 1 and both SRK passes, the scalar
 // walk against this: 24 and 71 against 34 and 75 us at 11 per cell, 27 and 81 against
 // 34 and 74 at 16, 33 and 96 against 33 and 80 at 24.  (A small system alone would
@@ -117,10 +118,28 @@ struct IntSums {
   bool odd;  // a partner whose features are not finite
 };
 
-// The scalar walk over the global tiles of slot k in cell c.
+// A packed feature's value in two byte products, of its two lower and its two upper
+// digits (128 as a byte is -128): -(d0 + 128 d1) and -(d2 + 128 d3) added to lo, hi.
+// |lo|, |hi| <= 8256 per feature, so that 2^17 of them stay within 32 bits.
+struct FixedHalves {
+  int lo = 0, hi = 0;
+  __device__ __forceinline__ void add(uint32_t v) {
+    lo = __builtin_amdgcn_sdot4((int)v, 0x000080ff, lo, false);
+    hi = __builtin_amdgcn_sdot4((int)v, (int)0x80ff0000u, hi, false);
+  }
+  __device__ __forceinline__ long long value() const { return -((long long)hi * 16384 + lo); }
+};
+constexpr int kHalvesRun = 1 << 17;
+
+// The scalar walk over the global tiles of slot k in cell c, four candidates
+// requested at a time, two byte products per feature and no branch but the band's.
+// Bound by the latency of its loads.  An SRK step at N = 20,000 in 10 x 10 cells, no
+// workgroup staged: 513 us; 1022 with the features unpacked and added in 64 bits
+// behind each decision, 738 with the FP32 form's walk (visit_global).
 template <int PASS>
 __device__ __forceinline__ int visit_integer(const KParams &P, const int *start, const Tiles &t, const uint2 *aq, int c,
                                              int k, IntSums<PASS> &o) {
+  constexpr int F = PASS == 1 ? 2 : 4;
   const int cx = c % P.nx, cy = c / P.nx;
   const float4 u = t.f4[k];
   int cand = 0;
@@ -130,21 +149,36 @@ __device__ __forceinline__ int visit_integer(const KParams &P, const int *start,
     for (int dxo = -1; dxo <= 1; ++dxo) {
       const int jc = row + adjust_cell(cx + dxo, P.nx);
       const float ox = __builtin_fmaf((float)dxo, P.hxf, -u.x);
-      cand += start[jc + 1] - start[jc];
+      const int end = start[jc + 1];
+      cand += end - start[jc];
+      for (int r0 = start[jc]; r0 < end; r0 += kHalvesRun) {
+        const int r1 = min(end, r0 + kHalvesRun);
+        FixedHalves h[F];
 #pragma unroll 1
-      for (int m = start[jc]; m < start[jc + 1]; ++m) {
-        if (m == k) continue;
-        const float4 v = t.f4[m];
-        const float dx = v.x + ox, dy = v.y + oy;
-        const float r2 = __builtin_fmaf(dx, dx, dy * dy);
-        bool in = r2 <= P.rho2f_hi;
-        if ((r2 >= P.rho2f_lo) & in) in = exact_r2(t.x, t.y, k, m, P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
-        if (!in) continue;
-        const Fixed<PASS> f(v, aq, m);
-        o.odd |= f.odd();
+        for (int m = r0; m < r1; m += 4) {
+          float4 v[4];
+          uint2 q[4];
 #pragma unroll
-        for (int q = 0; q < (PASS == 1 ? 2 : 4); ++q) o.v[q] += unpack_fixed(f.v[q]);
-        ++o.n;
+          for (int i = 0; i < 4; ++i) {
+            const int j = min(m + i, r1 - 1);
+            v[i] = t.f4[j];
+            if (PASS == 2) q[i] = aq[j];
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const float dx = v[i].x + ox, dy = v[i].y + oy;
+            const float r2 = __builtin_fmaf(dx, dx, dy * dy);
+            bool in = (r2 <= P.rho2f_hi) & (m + i < r1) & (m + i != k);
+            if ((r2 >= P.rho2f_lo) & in) in = exact_r2(t.x, t.y, k, m + i, P.Lx, P.r2Lx, P.Ly, P.r2Ly) <= P.rho2;
+            const Fixed<PASS> f(v[i], q + i, 0);
+            o.odd |= in & f.odd();
+#pragma unroll
+            for (int w = 0; w < F; ++w) h[w].add(in ? f.v[w] : 0u);
+            o.n += in;
+          }
+        }
+#pragma unroll
+        for (int w = 0; w < F; ++w) o.v[w] += h[w].value();
       }
     }
   }
