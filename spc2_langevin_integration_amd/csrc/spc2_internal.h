@@ -58,7 +58,7 @@ struct KParams {
   int seg_w, segs, lds_cap, chunk;
   int mfma;   // dense FP32 chimera cells: the matrix-core passes (spc2_chimera_mfma.h)
   double aj, raj;  // their scale of pass 2's a_j, a power of two >= |a_j|, and its reciprocal
-  int near[2];  // bytes of pass 1's and pass 2's words of near partners (NearWords)
+  int near[2];  // bytes of pass 1's and pass 2's words of near partners (NearWords), 0: not kept
   int bin_cap;  // entries of a cell's list (see Bins), a multiple of 4; 0: no lists
   int lanes;  // lanes per centre particle of the FP64 cell walks (a power of two; 1 in the FP32 form)
 };

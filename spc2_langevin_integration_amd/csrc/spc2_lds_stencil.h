@@ -397,7 +397,12 @@ __device__ __forceinline__ int visit_lds64(Acc &acc, const Src64 &src, const Seg
 // the partners' terms, and their order in each sum, are visit_lds's.  Two partners'
 // terms are formed together: at the sizes of one replica a SIMD holds one wavefront,
 // and the chain of operations bounds it.  N = 1000: 48 -> 33
-// us, N = 50,000: 51 -> 39, N = 400,000: 118 -> 109.
+// us, N = 50,000: 51 -> 39, N = 400,000: 118 -> 109.  In cells of fewer than
+// kNearPerCell = 42 particles: in fuller ones a wavefront's lanes lie in one cell and
+// read the same candidates at once, which visit_lds does from one LDS address.  An SRK
+// step on 50 x 50 cells with visit_lds and so: 81 and 69 us at 10 per cell, 154 and 149
+// at 30, 189 and 192 at 40, 295 and 409 at 60, 1245 and 1393 at 130; on 10 x 10 cells
+// 159 and 149 at 37, 179 and 179 at 45, 211 and 217 at 55.
 template <class Acc>
 __device__ __forceinline__ void visit_near32(Acc &acc, const Src32 &src, const SegShared &sh, int ncol, int qi, int ei,
                                              NearWords *near, const KParams &P) {
@@ -672,12 +677,16 @@ __device__ __forceinline__ void pass2_segment(const KParams &P, const int *__res
         else hi = mid - 1;
       }
       acc.init(lt.src(), ei, k, t, P, in);
-      if constexpr (HasNear32<Acc>::value)
-        visit_near32(acc, lt.src(), sh, g.ncol, lo, ei, near_words<PREC, 2>(dyn_lds, P), P);
-      else if constexpr (PREC == P32K)
-        visit_lds(acc, lt.src(), sh, g.ncol, lo, ei, P);
-      else
+      bool near = false;
+      if constexpr (HasNear32<Acc>::value) {
+        near = P.near[1] != 0;
+        if (near) visit_near32(acc, lt.src(), sh, g.ncol, lo, ei, near_words<PREC, 2>(dyn_lds, P), P);
+      }
+      if constexpr (PREC == P32K) {
+        if (!near) visit_lds(acc, lt.src(), sh, g.ncol, lo, ei, P);
+      } else {
         visit_lds64(acc, lt.src(), sh, g.ncol, lo, ei, gl, wraps(P, g), near_words<PREC, 2>(dyn_lds, P), P);
+      }
     } else {
       auto gs = global_src<PREC>(t, e, 2);
       acc.init(gs, k, k, t, P, in);

@@ -224,6 +224,7 @@ void pass2_sys(Sim &s, int epi, const EpiCtx &e) {
 constexpr int kLanes64 = 2;
 constexpr long long kLanesFill = 131072;
 constexpr double kMfmaPerCell = 20.0;
+constexpr double kNearPerCell = 42.0;
 
 // bytes per staged candidate of the larger pass
 int lds_elem_bytes(int prec) {
@@ -287,7 +288,7 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
   k.aj = k.raj = 1.0;
   k.bin_cap = 0;
   k.near[0] = prec == P64 ? (int)sizeof(NearWords) : 0;
-  k.near[1] = prec == P64 || (prec == P32K && system == SPC2_VORTEX) ? (int)sizeof(NearWords) : 0;
+  k.near[1] = prec == P64 ? (int)sizeof(NearWords) : 0;
   if (!k.linked) {
     k.seg_w = k.segs = 1;
     k.lds_cap = 0;
@@ -299,6 +300,7 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
   }
   target /= k.lanes;  // particles per workgroup
   const double per_cell = (double)k.n / ((double)k.nx * (double)k.ny);
+  if (prec == P32K && system == SPC2_VORTEX && per_cell < kNearPerCell) k.near[1] = (int)sizeof(NearWords);
   double halo;
   if (per_cell >= kChunkPerCell) {
     const int unit = 64 / k.lanes;  // a wavefront's particles

@@ -88,3 +88,9 @@ def test_dense_batch_equals_single(method):
             s.init_random_state(0.1)
             s.step(method, DT, 0, 3)
             assert np.array_equal(s.get_state(), g), f"n={p.n}"
+
+
+# both sides of the filling from which pass 2 no longer finds the near partners first; what 2560 candidates hold
+@pytest.mark.parametrize("filling,clump", [(41, 0.0), (43, 0.0), (60, 0.6), (145, 0.0), (170, 0.0), (300, 0.0)])
+def test_dense_vortex_cells(monkeypatch, filling, clump):
+    compare(monkeypatch, "vortex", "fp32k", filling, clump)
