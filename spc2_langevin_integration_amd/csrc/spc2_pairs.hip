@@ -223,6 +223,7 @@ void pass2_sys(Sim &s, int epi, const EpiCtx &e) {
 
 constexpr int kLanes64 = 2;
 constexpr long long kLanesFill = 131072;
+constexpr double kLanesPerCell = 170.0;
 constexpr double kMfmaPerCell = 20.0;
 constexpr double kNearPerCell = 42.0;
 
@@ -262,7 +263,11 @@ static int chunks_per_row(const KParams &k) {
 //   most 16, so that small systems fill the device; the plain form at least
 //   kLanes64, whose halved workgroups leave room for its words of bits.  The
 //   count depends on the system alone, so that a batch's replica sums as a single
-//   handle does.
+//   handle does.  The factored form has little to do per candidate: in cells from
+//   kLanesPerCell particles on, where no halo of its 40-byte candidates is staged
+//   whatever the lanes, their loads of different candidates at once cost more than
+//   they gain (chimera SRK step on 12 x 12 cells, 8 and 4 lanes against one: 934 and
+//   595 us at 200 per cell, 1838 and 861 at 300).
 // * Rows of at least kChunkPerCell particles per cell are cut into chunks of
 //   `target` slots rounded to whole wavefronts, so that every wavefront but a
 //   row's last is full.  A row gets workgroups for its mean count plus four
@@ -294,12 +299,12 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
     k.lds_cap = 0;
     return;
   }
-  if (prec != P32K) {
+  const double per_cell = (double)k.n / ((double)k.nx * (double)k.ny);
+  if (prec == P64 || (prec == P64F && per_cell < kLanesPerCell)) {
     const int least = prec == P64 ? kLanes64 : 1;
     while (k.lanes < least || (k.lanes < 16 && (long long)k.n * k.lanes < kLanesFill)) k.lanes *= 2;
   }
   target /= k.lanes;  // particles per workgroup
-  const double per_cell = (double)k.n / ((double)k.nx * (double)k.ny);
   if (prec == P32K && system == SPC2_VORTEX && per_cell < kNearPerCell) k.near[1] = (int)sizeof(NearWords);
   double halo;
   if (per_cell >= kChunkPerCell) {

@@ -94,3 +94,11 @@ def test_dense_batch_equals_single(method):
 @pytest.mark.parametrize("filling,clump", [(41, 0.0), (43, 0.0), (60, 0.6), (145, 0.0), (170, 0.0), (300, 0.0)])
 def test_dense_vortex_cells(monkeypatch, filling, clump):
     compare(monkeypatch, "vortex", "fp32k", filling, clump)
+
+
+# the FP64 forms: both sides of the filling from which the factored one takes a lane per particle; halos beyond the LDS
+@pytest.mark.parametrize("filling,clump", [(60, 0.6), (165, 0.0), (175, 0.0), (300, 0.0)])
+@pytest.mark.parametrize("prec", ["fp64", "fp64f"])
+@pytest.mark.parametrize("system", ["chimera", "vortex"])
+def test_dense_fp64_cells(monkeypatch, system, prec, filling, clump):
+    compare(monkeypatch, system, prec, filling, clump)
