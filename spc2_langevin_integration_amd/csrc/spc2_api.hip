@@ -174,7 +174,7 @@ spc2_status alloc_all(Sim &s) {
   for (auto &p : s.der) A(p, n);
   for (auto &p : s.add) A(p, n);
   A(s.gx, n); A(s.gy, n); A(s.gp, n);
-  A(s.cell_of, n); A(s.count, 4 * (size_t)s.count_stride); A(s.local, n); A(s.start, (size_t)s.count_stride + 1);
+  A(s.cell_of, n); A(s.count, s.count_ints()); A(s.local, (s.kp.bin_cap ? 3 : 1) * n); A(s.start, (size_t)s.count_stride + 1);
   if (s.kp.bin_cap) {
     A(s.bin_list, nc * (size_t)s.kp.bin_cap);
   } else if (s.linked) {
@@ -228,7 +228,7 @@ spc2_status alloc_all(Sim &s) {
   // Cleared on the handle's stream, so that the first kernels on that
   // (non-blocking) stream see zeros: the cell histogram must start at zero,
   // since the first binning's arrival ranks index the placement.
-  HIP_TRY(hipMemsetAsync(s.count, 0, sizeof(int) * 4 * (size_t)s.count_stride, s.stream));
+  HIP_TRY(hipMemsetAsync(s.count, 0, sizeof(int) * s.count_ints(), s.stream));
   HIP_TRY(hipMemsetAsync(s.omega, 0, sizeof(double) * n, s.stream));
   for (auto &kk : s.k)
     for (auto &p : kk) HIP_TRY(hipMemsetAsync(p, 0, sizeof(double) * n, s.stream));
@@ -268,7 +268,7 @@ spc2_status check_build(Sim &s, const char *what) {
   if (st) {
     s.staged = s.tile_fresh = s.built = false;
     s.vnext = 0;
-    (void)hipMemsetAsync(s.count, 0, sizeof(int) * 4 * (size_t)s.count_stride, s.stream);
+    (void)hipMemsetAsync(s.count, 0, sizeof(int) * s.count_ints(), s.stream);
   }
   return st;
 }

@@ -144,6 +144,14 @@ __device__ __forceinline__ EpiCtx rep_ctx(const EpiCtx &e, const Rep &R, int k) 
   return c;
 }
 
+// A replica's scalars.  Batches keep no lists (bin_cap 0), which the compiler is told,
+// so that the binning epilogues' chains leave no trace in the merged kernels.
+__device__ __forceinline__ KParams rep_params(const Rep &R) {
+  KParams P = R.kp;
+  P.bin_cap = 0;
+  return P;
+}
+
 // All-pairs replicas (rho > L/4): a wavefront sums one particle at a time, as a
 // single handle's, kApBatch particles in turn, and its first kApBatch lanes then
 // take their epilogues side by side: a batch fills the device with its linked
@@ -160,7 +168,7 @@ __device__ __forceinline__ void b_allpairs1(const Rep *reps, const int *ap_rep, 
   const Rep &R = reps[ap_rep[ab]];
   if (k >= R.steps) return;
   const int i0 = (ab - R.apoff) * kApPerBlock + threadIdx.x / kApLanes * kApBatch, g = threadIdx.x % kApLanes;
-  const KParams P = R.kp;
+  const KParams P = rep_params(R);
   const EpiCtx c = rep_ctx(e, R, k);
   Pass1Out o{};
   for (int r = 0; r < kApBatch && i0 + r < R.n; ++r) {
@@ -179,7 +187,7 @@ __device__ __forceinline__ void b_allpairs2_srk(const Rep *reps, const int *ap_r
   const Rep &R = reps[ap_rep[ab]];
   if (k >= R.steps) return;
   const int i0 = (ab - R.apoff) * kApPerBlock + threadIdx.x / kApLanes * kApBatch, g = threadIdx.x % kApLanes;
-  const KParams P = R.kp;
+  const KParams P = rep_params(R);
   const EpiCtx c = rep_ctx(e, R, k);
   const int o0 = R.poff;
   Pass2Out o{};
@@ -231,7 +239,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(PREC == P32K
   const int sg = xcd_segment(blockIdx.x - ap.pad, gridDim.x - ap.pad);
   const Rep &R = reps[seg_rep[sg]];
   if (k >= R.steps) return;  // the whole workgroup: the replica is done in this call
-  const KParams P = R.kp;
+  const KParams P = rep_params(R);
   const EpiCtx c = rep_ctx(e, R, k);
   if constexpr (PREC == P32K) {
     if (P.mfma) {
@@ -260,7 +268,7 @@ __global__ __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(PREC == P32K
   const int sg = xcd_segment(blockIdx.x - ap.pad, gridDim.x - ap.pad);
   const Rep &R = reps[seg_rep[sg]];
   if (k >= R.steps) return;
-  const KParams P = R.kp;
+  const KParams P = rep_params(R);
   const EpiCtx c = rep_ctx(e, R, k);
   if constexpr (PREC == P32K) {
     if (P.mfma) {
@@ -425,7 +433,7 @@ struct spc2_batch {
   float *snap = nullptr;
   hipEvent_t snap_ev = nullptr;
   bool snap_pending = false;
-  Bins bins() const { return Bins{cell_of, count_, nullptr, nullptr, local}; }
+  Bins bins() const { return Bins{cell_of, count_, nullptr, nullptr, nullptr, local}; }
   size_t lds[2] = {};  // dynamic LDS of the pass-1 and pass-2 launches
   int since_rehome = 0;
   bool fresh = true;  // a state came in since the last re-homing

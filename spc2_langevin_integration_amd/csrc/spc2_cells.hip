@@ -252,7 +252,7 @@ __global__ __launch_bounds__(kBlock) void k_rank_tiles(int n, int nx, int fixed,
 // scanned in LDS instead, two serial runs over it per thread: 35 us at 14,000 cells.)
 template <int PREC>
 __global__ __launch_bounds__(kBlock) void k_sort_tiles(int n, int nx, int nc, int fixed, int cap, double hx, double hy,
-                                                       Bins bins, int *other, const int *hid, int *start,
+                                                       Bins bins, int *other, int *other_used, const int *hid, int *start,
                                                        const double *gx, const double *gy, const double *gp,
                                                        int *slot_h, int *slot_id, Tiles t) {
   __shared__ int pre[kMaxBinRows];  // the rows' starts
@@ -261,6 +261,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_tiles(int n, int nx, int nc, in
   const int rows = (nc + kBinRow - 1) / kBinRow;
   const int4 *count = (const int4 *)bins.count;
   for (int q = h; q < 2 * kBinRow / 4 * rows; q += all) ((int4 *)other)[q] = make_int4(0, 0, 0, 0);
+  if (h == 0) *other_used = 0;
   constexpr int kPer = kMaxBinRows / kBlock;
   int own[kPer], sum = 0;
 #pragma unroll
@@ -310,7 +311,7 @@ __global__ __launch_bounds__(kBlock) void k_sort_tiles(int n, int nx, int nc, in
     lo += 4 * w + 2 < in_row ? v.z : 0;
     lo += 4 * w + 3 < in_row ? v.w : 0;
   }
-  const int dst = lo + rank_in_bin(bins, c, cap, bins.count[c], hid, id);
+  const int dst = lo + rank_in_bin(bins, c, cap, bins.count[c], id);
   write_slot<PREC>(dst, h, id, c, nx, fixed, hx, hy, gx, gy, gp, slot_h, slot_id, t);
 }
 
@@ -351,7 +352,7 @@ void launch_sort(Sim &s, const Bins &b) {
   const dim3 g(blocks_for(s.n)), blk(kBlock);
   if (s.kp.bin_cap)
     hipLaunchKernelGGL(k_sort_tiles<PREC>, g, blk, 0, s.stream, s.n, s.nx, s.nc,
-                       s.kp.mfma, s.kp.bin_cap, s.kp.hx, s.kp.hy, b, s.bins().count, s.hid, s.start, s.gx, s.gy, s.gp,
+                       s.kp.mfma, s.kp.bin_cap, s.kp.hx, s.kp.hy, b, s.bins().count, s.bins().used, s.hid, s.start, s.gx, s.gy, s.gp,
                        s.slot_h, s.slot_id, s.t);
   else
     hipLaunchKernelGGL(k_rank_tiles<PREC>, g, blk, 0, s.stream, s.n, s.nx, s.kp.mfma, s.kp.hx, s.kp.hy, s.tmp, s.tmpid,
@@ -383,7 +384,7 @@ void launch_cells(Sim &s) {
 void configure_bins(Sim &s) {
   s.kp.bin_cap = 0;
   s.count_stride = std::max(s.nc, 1);
-  if (!s.linked || s.verlet || s.nc > kBinRow * kMaxBinRows) return;
+  if (!s.linked || s.verlet || s.nc > kBinRow * kMaxBinRows || s.n >= (1 << 29)) return;  // (3 n ints of chains)
   s.count_stride = (s.nc + kBinRow - 1) / kBinRow * kBinRow;
   const double per_cell = (double)s.n / (double)s.nc;
   s.kp.bin_cap = (int)std::ceil((per_cell + 4.0 * std::sqrt(per_cell) + 8.0) / 4.0) * 4;

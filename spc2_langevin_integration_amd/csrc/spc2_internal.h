@@ -71,10 +71,10 @@ struct Tiles {
 };
 
 // One binning (bin_particle): cell of each home, count of each cell, and either the
-// arrival ranks by home (next) or the cells' lists of particle ids with their
-// overflow chains (links in next).
+// arrival ranks by home (next) or the cells' lists of particle ids with the chains of
+// what their lists do not hold (nodes in next, `used` its ints in use: at most 3 n).
 struct Bins {
-  int *cell_of, *count, *chain, *list, *next;
+  int *cell_of, *count, *chain, *used, *list, *next;
 };
 
 struct StepArgs {
@@ -115,15 +115,17 @@ struct Sim {
   // cell list (per home: cell_of, local; per slot: tmp/tmpid while placing,
   // then slot_h / slot_id = home / id of the particle in each cell-sorted slot);
   // with lists (bin_cap > 0) count holds two sets of count_stride counts and as many
-  // chains, of which bin_set takes the next binning, else one set of counts
+  // chains, of which bin_set takes the next binning, then the two sets' ints in use;
+  // else one set of counts
   int *cell_of = nullptr, *count = nullptr, *local = nullptr, *start = nullptr, *tmp = nullptr, *tmpid = nullptr,
       *bin_list = nullptr, *slot_h = nullptr, *slot_id = nullptr;
   int bin_set = 0, count_stride = 0;  // counts of a set, padded
   bool built = false;  // slot_h holds the cell order of the current homes
   Bins bins() const {
     int *c = count + (size_t)bin_set * 2 * (size_t)count_stride;
-    return Bins{cell_of, c, c + count_stride, bin_list, local};
+    return Bins{cell_of, c, c + count_stride, count + 4 * (size_t)count_stride + bin_set, bin_list, local};
   }
+  size_t count_ints() const { return 4 * (size_t)count_stride + 2; }
   int rehome_every = 16, steps_since_rehome = 0;
   // re-homing double buffers (state x, y, phi, omega, k_1..k_4) and id-order
   // transfer scratch for the ABI's host arrays

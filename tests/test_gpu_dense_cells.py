@@ -102,3 +102,25 @@ def test_dense_vortex_cells(monkeypatch, filling, clump):
 @pytest.mark.parametrize("system", ["chimera", "vortex"])
 def test_dense_fp64_cells(monkeypatch, system, prec, filling, clump):
     compare(monkeypatch, system, prec, filling, clump)
+
+
+# overfull cells side by side in one wavefront and whole wavefronts in one cell (homes in id order, then in cell order)
+@pytest.mark.parametrize("spots,share", [(1, 1.0), (3, 0.9), (40, 0.5), (300, 0.5)])
+@pytest.mark.parametrize("side", [4, 100])
+def test_overfull_cells_are_sorted(side, spots, share):
+    n = 20011
+    rng = np.random.default_rng(spots)
+    st = rng.uniform(0.0, 1.0, 3 * n)
+    k = int(share * n)
+    at = rng.uniform(0.05, 0.95, (spots, 2))[rng.integers(0, spots, k)]
+    for c in (0, 1):
+        st[c:3 * k:3] = at[:, c] + 1e-3 * rng.uniform(-1.0, 1.0, k)
+    st = st.reshape(n, 3)[rng.permutation(n)].ravel()
+    c = (st[1::3] * side).astype(int) * side + (st[0::3] * side).astype(int)
+    with spc2.Sim(spc2.params("chimera", "fp64", "cells", n=n, L=1.0, rho=1.0 / (side + 0.5))) as s:
+        for _ in range(3):
+            s.set_state(st)
+            cell_of, start, order = s.cell_list()
+            assert np.array_equal(cell_of, c)
+            assert np.array_equal(start, np.concatenate([[0], np.cumsum(np.bincount(c, minlength=side * side))]))
+            assert np.array_equal(order, np.argsort(c, kind="stable"))
