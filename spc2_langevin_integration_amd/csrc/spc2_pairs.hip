@@ -223,7 +223,9 @@ void pass2_sys(Sim &s, int epi, const EpiCtx &e) {
 
 constexpr int kLanes64 = 2;
 constexpr long long kLanesFill = 131072;
-constexpr double kLanesPerCell = 170.0;
+constexpr double kLanesPerCell[2] = {0.85, 1.5};  // chimera, vortex arrays
+constexpr double kDensePerCell = 170.0;
+constexpr int kDenseN = 16384;
 constexpr double kMfmaPerCell = 20.0;
 constexpr double kNearPerCell = 42.0;
 
@@ -263,11 +265,17 @@ static int chunks_per_row(const KParams &k) {
 //   most 16, so that small systems fill the device; the plain form at least
 //   kLanes64, whose halved workgroups leave room for its words of bits.  The
 //   count depends on the system alone, so that a batch's replica sums as a single
-//   handle does.  The factored form has little to do per candidate: in cells from
-//   kLanesPerCell particles on, where no halo of its 40-byte candidates is staged
-//   whatever the lanes, their loads of different candidates at once cost more than
-//   they gain (chimera SRK step on 12 x 12 cells, 8 and 4 lanes against one: 934 and
-//   595 us at 200 per cell, 1838 and 861 at 300).
+//   handle does.  In sparse cells no more lanes than kLanesPerCell times the mean
+//   filling: a stencil row of three cells has little for more, and a batch, which
+//   fills the device by itself, pays for their workgroups (64 chimera replicas of N
+//   = 2000, SRK step, 16 lanes and so: plain 348 and 123 us at 1 per cell, 367 and
+//   103 at 2, 382 and 152 at 4, 335 and 198 at 7; alone 39 and 29, 38 and 30, 37 and
+//   38, 38 and 40; one lane of the library's sines: 148 to 219).  Nor in cells from
+//   kDensePerCell particles on, of systems of at least kDenseN, where no halo is
+//   staged whatever the lanes and their loads of different candidates at once cost
+//   more than they gain (chimera SRK step in 10 x 10 and 14 x 14 cells of 200, with 8
+//   and 4 lanes: plain 612 and 1044 us, so 650 and 820; factored 686 and 1135, so 586
+//   and 599).
 // * Rows of at least kChunkPerCell particles per cell are cut into chunks of
 //   `target` slots rounded to whole wavefronts, so that every wavefront but a
 //   row's last is full.  A row gets workgroups for its mean count plus four
@@ -300,9 +308,12 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
     return;
   }
   const double per_cell = (double)k.n / ((double)k.nx * (double)k.ny);
-  if (prec == P64 || (prec == P64F && per_cell < kLanesPerCell)) {
+  if (prec != P32K) {
     const int least = prec == P64 ? kLanes64 : 1;
-    while (k.lanes < least || (k.lanes < 16 && (long long)k.n * k.lanes < kLanesFill)) k.lanes *= 2;
+    const int most = per_cell >= kDensePerCell && k.n >= kDenseN ? least : 16;
+    while (k.lanes < least ||
+           (k.lanes < most && k.lanes < kLanesPerCell[system] * per_cell && (long long)k.n * k.lanes < kLanesFill))
+      k.lanes *= 2;
   }
   target /= k.lanes;  // particles per workgroup
   if (prec == P32K && system == SPC2_VORTEX && per_cell < kNearPerCell) k.near[1] = (int)sizeof(NearWords);

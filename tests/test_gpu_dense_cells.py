@@ -1,5 +1,5 @@
-"""Cells of more particles than the staged halos hold, at the fillings where the
-choice of walk changes, against the oracle and with every walk over the global
+"""Cells of more particles than the staged halos hold, or of hardly any, at the
+fillings where the choice of walk changes, against the oracle and with every walk over the global
 tiles, bit for bit; batched replicas against single handles.  Bars: tests/_parity.py."""
 import os
 import sys
@@ -40,8 +40,8 @@ def state_of(n, clump=0.0):
     return st
 
 
-def compare(monkeypatch, system, prec, filling, clump):
-    p, orc = systems(system, prec, filling)
+def compare(monkeypatch, system, prec, filling, clump, side=SIDE):
+    p, orc = systems(system, prec, filling, side)
     st = state_of(p.n, clump)
     z = np.zeros(3 * p.n)
     U = np.random.default_rng(1).standard_normal(2 * p.n)
@@ -74,6 +74,30 @@ def compare(monkeypatch, system, prec, filling, clump):
                                            (60, 0.6), (130, 0.6)])
 def test_dense_chimera_cells(monkeypatch, filling, clump):
     compare(monkeypatch, "chimera", "fp32k", filling, clump)
+
+
+# the FP64 forms' lanes per particle in sparse cells: 1, 2, 4, 8 and 16 of them; a system of 16384 in dense cells
+@pytest.mark.parametrize("filling,side", [(0.3, 15), (1.1, 15), (1.4, 15), (2.6, 15), (5.5, 15), (9.5, 15), (172, 10)])
+@pytest.mark.parametrize("prec", ["fp64", "fp64f"])
+@pytest.mark.parametrize("system", ["chimera", "vortex"])
+def test_sparse_fp64_cells(monkeypatch, system, prec, filling, side):
+    compare(monkeypatch, system, prec, filling, 0.0, side)
+
+
+@pytest.mark.parametrize("method", ["se", "srk"])
+@pytest.mark.parametrize("prec", ["fp64", "fp64f"])
+def test_sparse_batch_equals_single(prec, method):
+    reps = [systems(("chimera", "vortex")[k % 2], prec, f, 12 + k % 5, seed=20 + k)[0]
+            for k, f in enumerate([0.3, 0.3, 1.3, 1.3, 2.7, 2.7, 6.0, 6.0, 175, 175])]
+    with spc2.Batch(reps) as b:
+        b.init_random_state(0.1)
+        b.step(DT, 3, method=method)
+        got = [b.get_state(r) for r in range(len(reps))]
+    for p, g in zip(reps, got):
+        with spc2.Sim(p) as s:
+            s.init_random_state(0.1)
+            s.step(method, DT, 0, 3)
+            assert np.array_equal(s.get_state(), g), f"n={p.n}"
 
 
 @pytest.mark.parametrize("method", ["se", "srk"])
