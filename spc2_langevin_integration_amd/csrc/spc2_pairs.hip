@@ -241,9 +241,12 @@ int lds_elem_bytes(int prec) {
 }  // namespace
 
 // Candidates of a matrix-core workgroup at the most, and what the rows' padding and
-// the far tile take of them: 76 KB of LDS, two workgroups per CU as with 60.
+// the far tile take of them: 76 KB of LDS, two workgroups of pass 2 per CU as with 60.
+// Chunks are kept to kMfmaHalo candidates where they can be, three workgroups of pass
+// 1 per CU (past it, SRK steps at 150 to 160 particles per cell take 10 to 19% longer).
 constexpr int kMfmaLdsBytes = 76 * 1024;
 constexpr int kMfmaCap = (kMfmaLdsBytes - MfmaLds<2>::tail_bytes) / MfmaLds<2>::tile_bytes * kMfmaTile;
+constexpr int kMfmaHalo = 2752;
 constexpr double kMfmaPad = 128.0;
 
 // its mean halo with a margin, for a chunk of row slots: the chunk's cells, a partial
@@ -290,10 +293,10 @@ static int chunks_per_row(const KParams &k) {
 //   where the two or so cells that such a chunk touches have too many neighbours for
 //   it (from 214 particles per cell on), the scalar walk of the FP32 form is the
 //   faster one.  An SRK step, before (chunks of 256 within 60 KB, every filling) and
-//   so, with the scalar walk's time: in 16 x 16 cells 94, 103 (235) us at 160 per
-//   cell, 950, 104 (683) at 180, 1091, 126 (735) at 200; in 50 x 50 cells 885, 338
-//   (486) at 130, 3933, 1004 (1877) at 200; and past the line with the matrix cores
-//   819 (897) at 240 in 16 x 16 cells, 6360 (4979) at 280 in 50 x 50.
+//   so, with the scalar walk's time: in 16 x 16 cells 94 and 94 us (235) at 160 per
+//   cell, 950 and 104 (683) at 180, 1091 and 123 (735) at 200; in 50 x 50 cells 885
+//   and 340 (486) at 130, 3933 and 759 (1877) at 200; past the line, on the matrix
+//   cores all the same, 6360 (4979) at 280.
 void configure_segments_kp(KParams &k, int prec, int system, double target) {
   k.chunk = 0;
   k.lanes = 1;
@@ -327,12 +330,13 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
     k.segs = chunks_per_row(k);
     k.seg_w = std::min(k.nx, (int)std::ceil(chunk / per_cell) + 1);
     halo = 1.25 * 3.0 * (chunk + 3.0 * per_cell);  // chunk's cells, a partial cell at each end, and the sides
-    const double two = 12.0 * per_cell;  // the halo of the shortest chunks: of two cells
-    if (prec == P32K && system == SPC2_CHIMERA && per_cell >= kMfmaPerCell &&
-        two + 4.0 * std::sqrt(two) + kMfmaPad <= kMfmaCap) {
+    // the halo of the shortest chunks: of two cells, with four standard deviations
+    const double two = 12.0 * per_cell + 4.0 * std::sqrt(12.0 * per_cell) + kMfmaPad;
+    if (prec == P32K && system == SPC2_CHIMERA && per_cell >= kMfmaPerCell && two <= kMfmaCap) {
       k.mfma = 1;
       k.chunk = std::min(chunk, kMfmaWindow);
-      while (k.chunk > 2 * kMfmaTile && mfma_halo(k.chunk, per_cell) > kMfmaCap) k.chunk /= 2;
+      while (k.chunk > 2 * kMfmaTile && mfma_halo(k.chunk, per_cell) > kMfmaHalo) k.chunk /= 2;
+      halo = std::max(mfma_halo(k.chunk, per_cell), two);
       k.segs = chunks_per_row(k);
       // |a_j| <= |sigma|: sigma times a mean of sines
       k.aj = std::exp2(std::ceil(std::log2(std::max(std::fabs(k.sigma) * 1.0001, 1e-200))));
@@ -347,7 +351,7 @@ void configure_segments_kp(KParams &k, int prec, int system, double target) {
   }
   int cap;
   if (k.mfma) {
-    cap = std::min(kMfmaCap, (int)std::ceil(mfma_halo(k.chunk, per_cell) / kMfmaTile) * kMfmaTile);
+    cap = std::min(kMfmaCap, (int)std::ceil(halo / kMfmaTile) * kMfmaTile);
   } else {
     cap = (int)std::ceil((halo + 160.0) / 64.0) * 64;
     cap = std::min(cap, (kLdsBytes - k.near[1]) / lds_elem_bytes(prec));
