@@ -267,6 +267,18 @@ struct ChimAcc<P64> {
     if (near<true>(s, m, P)) term<false>(In(s, m), true, P);
   }
   __device__ __forceinline__ void cohesion(const Src64 &, int, const KParams &) {}
+  // the sums of a pair of list entries, formed apart and then added (-0: so that the
+  // first term needs no addition)
+  __device__ __forceinline__ ChimAcc apart() const {
+    ChimAcc t = *this;
+    t.A = -0.0;
+    t.n = 0;
+    return t;
+  }
+  __device__ __forceinline__ void add(const ChimAcc &t) {
+    A += t.A;
+    n += t.n;
+  }
   // the totals of a particle's lanes
   __device__ __forceinline__ void reduce(int G) {
     A = lanes_total(A, G);
@@ -482,6 +494,18 @@ struct VortAcc<P64> {
   }
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
     if (near<true>(s, m, P) && term<false>(In(s, m), true, P)) cohesion(s, m, P);
+  }
+  __device__ __forceinline__ VortAcc apart() const {  // of the alignment terms
+    VortAcc t = *this;
+    t.A = t.B = -0.0;
+    t.n0 = t.n1 = 0;
+    return t;
+  }
+  __device__ __forceinline__ void add(const VortAcc &t) {
+    A += t.A;
+    B += t.B;
+    n0 += t.n0;
+    n1 += t.n1;
   }
   __device__ __forceinline__ void reduce(int G) {
     A = lanes_total(A, G);
@@ -814,6 +838,15 @@ struct Chim2Acc<P64> {
     if (near<true>(s, m, P)) term<false>(In(s, m), true, P);
   }
   __device__ __forceinline__ void cohesion(const Src64 &, int, const KParams &) {}
+  __device__ __forceinline__ Chim2Acc apart() const {
+    Chim2Acc t = *this;
+    t.a0 = t.a1 = -0.0;
+    return t;
+  }
+  __device__ __forceinline__ void add(const Chim2Acc &t) {
+    a0 += t.a0;
+    a1 += t.a1;
+  }
   __device__ __forceinline__ void reduce(int G) {
     a0 = lanes_total(a0, G);
     a1 = lanes_total(a1, G);
@@ -1068,6 +1101,15 @@ struct Vort2Acc<P64> {
   }
   __device__ __forceinline__ void pair(const Src64 &s, int m, const KParams &P) {
     if (near<true>(s, m, P) && term<false>(In(s, m), true, P)) cohesion(s, m, P);
+  }
+  __device__ __forceinline__ Vort2Acc apart() const {
+    Vort2Acc t = *this;
+    t.a0 = t.a1 = -0.0;
+    return t;
+  }
+  __device__ __forceinline__ void add(const Vort2Acc &t) {
+    a0 += t.a0;
+    a1 += t.a1;
   }
   __device__ __forceinline__ void reduce(int G) {
     a0 = lanes_total(a0, G);

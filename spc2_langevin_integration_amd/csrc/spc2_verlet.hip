@@ -889,15 +889,31 @@ __device__ __forceinline__ void walk_lds_rho_bits(Acc &acc, const int4 *l, const
   }
 }
 
-// FP64 forms: the entries of each group in turn.
+// FP64 forms: the entries of each group in turn; the plain form's alignment terms two
+// entries at a time, summed apart and then added, as walk64_lds takes them.
 template <class Acc, class S>
 __device__ __forceinline__ void walk64(Acc &acc, const S &src, const int4 *l, int cnt, const KParams &P) {
   for (int q = 0; q < cnt; q += 4) {
     const int4 g = l[(size_t)(q >> 2) * 64];
-    visit_entry(acc, src, g.x, P);
-    if (q + 1 < cnt) visit_entry(acc, src, g.y, P);
-    if (q + 2 < cnt) visit_entry(acc, src, g.z, P);
-    if (q + 3 < cnt) visit_entry(acc, src, g.w, P);
+    const int e[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+    for (int u = 0; u < 4; u += 2) {
+      if (q + u >= cnt) break;
+      if constexpr (HasNear<Acc>::value) {
+        Acc both = acc.apart();
+        const int j0 = e[u] >> 4, j1 = e[u + 1] >> 4;
+        using In = typename Acc::In;
+        const bool q0 = acc.template near<true>(src, j0, P) && both.template term<false>(In(src, j0), true, P);
+        const bool q1 = q + u + 1 < cnt && acc.template near<true>(src, j1, P) &&
+                        both.template term<false>(In(src, j1), true, P);
+        acc.add(both);
+        if (q0) acc.cohesion(src, j0, P);
+        if (q1) acc.cohesion(src, j1, P);
+      } else {
+        visit_entry(acc, src, e[u], P);
+        if (q + u + 1 < cnt) visit_entry(acc, src, e[u + 1], P);
+      }
+    }
   }
 }
 
@@ -1213,8 +1229,10 @@ __device__ __forceinline__ void walk64_lds(Acc &acc, const Src64 &src, const int
     hi >>= 32;
     if constexpr (HasNear<Acc>::value) {
       using In = typename Acc::In;
-      const bool q0 = acc.template term<FAST>(In(src, m0), acc.template near<true>(src, m0, P), P);
-      const bool q1 = acc.template term<FAST>(In(src, m1), two & acc.template near<true>(src, m1, P), P);
+      Acc both = acc.apart();
+      const bool q0 = both.template term<FAST>(In(src, m0), acc.template near<true>(src, m0, P), P);
+      const bool q1 = both.template term<FAST>(In(src, m1), two & acc.template near<true>(src, m1, P), P);
+      acc.add(both);
       if (q0) cq.push(m0);
       if (q1) cq.push(m1);
       if (cq.n > CohQueue64::kFull - 2 || q + 2 >= cnt) cq.drain(acc, src, P);
