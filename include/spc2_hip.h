@@ -32,7 +32,8 @@ typedef enum spc2_system { SPC2_CHIMERA = 0, SPC2_VORTEX = 1 } spc2_system;
 
 /* Arithmetic of the pair sums.
  *  SPC2_FP64: the reference method in FP64 (per-pair sin/cos/atan2, reference
- *             operation order, reference min-image), the plain GPU form.
+ *             min-image; the sums in shares of the reference order), the plain
+ *             GPU form.
  *  SPC2_FP32_KAHAN: pair sums in FP32 with Kahan compensation over cell-local
  *             FP32 coordinates; the phase enters through cos/sin of each
  *             particle's phase (angle-addition identity), so the pair loop has

@@ -1,9 +1,11 @@
 // Device-side building blocks shared by the spc2 kernels (gfx950).
 //
 // Every translation unit that includes this header is compiled with
-// -ffp-contract=off: the FP64 forms must round exactly like the reference
-// (no fused a*b+c), so each FP64 expression keeps the reference's left-to-right
-// evaluation order.  The FP32 forms use explicit fmaf where they want fusion.
+// -ffp-contract=off: each FP64 expression keeps the reference's left-to-right
+// evaluation order, and what is fused is written out.  The pair decisions (min-image,
+// squared separations, cutoff tests) round as the reference's; the FP64 sums are
+// formed in lanes' shares of its order, with sine, root and divisions of their own
+// (spc2_fp64_math.h), and agree to rounding.  The FP32 forms fuse where they want to.
 #pragma once
 
 #include <hip/hip_runtime.h>

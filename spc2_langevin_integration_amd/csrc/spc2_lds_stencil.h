@@ -6,11 +6,12 @@
 // consecutive slots of one cell row, which spans W cells) or, in sparse
 // systems, per row segment of W cells.  It stages the 3 x (W + 2) halo cells'
 // tiles in LDS with coalesced reads (cells of a row are contiguous in the
-// cell-sorted arrays), then each lane takes one centre particle.  In LDS the
-// three stencil cells of one stencil row are adjacent, so a particle visits its
-// 9 cells as 3 contiguous ranges, in the reference order (cells (-1,dy),
-// (0,dy), (1,dy), ascending particle index inside a cell).  A workgroup whose halo does not fit the LDS capacity
-// falls back to reading the same tiles from global memory with the same
+// cell-sorted arrays), then each lane takes one centre particle, or in the FP64 forms
+// its share of one's candidates.  In LDS the three stencil cells of one stencil row
+// are adjacent, so a particle's 9 cells are 3 contiguous ranges, in the reference
+// order (cells (-1,dy), (0,dy), (1,dy), ascending particle index inside a cell); a
+// lane takes a run of each in that order.  A workgroup whose halo does not fit the LDS
+// capacity falls back to reading the same tiles from global memory with the same
 // arithmetic and order.  Compiled with -ffp-contract=off.
 #pragma once
 

@@ -109,20 +109,17 @@ __device__ __forceinline__ double sep2(const Src64 &s, int m, double xi, double 
   return dx * dx + dy * dy;
 }
 
-// What a plain FP64 pass reads of a partner, so that walks can request it ahead.
+// What a plain FP64 pass reads of a partner for its term.
 struct InP {
-  double p = 0.0;
-  __device__ __forceinline__ InP() {}
+  double p;
   __device__ __forceinline__ InP(const Src64 &s, int m) : p(s.p[m]) {}
 };
 struct InPA {
-  double p = 0.0, aj = 0.0;
-  __device__ __forceinline__ InPA() {}
+  double p, aj;
   __device__ __forceinline__ InPA(const Src64 &s, int m) : p(s.p[m]), aj(s.aj[m]) {}
 };
 struct InXYP {
-  double x = 0.0, y = 0.0, p = 0.0;
-  __device__ __forceinline__ InXYP() {}
+  double x, y, p;
   __device__ __forceinline__ InXYP(const Src64 &s, int m) : x(s.x[m]), y(s.y[m]), p(s.p[m]) {}
   __device__ __forceinline__ double sep2(double xi, double yi, const KParams &P) const {
     const double dx = min_image(x - xi, P.Lx, P.r2Lx), dy = min_image(y - yi, P.Ly, P.r2Ly);
@@ -130,8 +127,7 @@ struct InXYP {
   }
 };
 struct InXYPA {
-  double x = 0.0, y = 0.0, p = 0.0, aj = 0.0;
-  __device__ __forceinline__ InXYPA() {}
+  double x, y, p, aj;
   __device__ __forceinline__ InXYPA(const Src64 &s, int m) : x(s.x[m]), y(s.y[m]), p(s.p[m]), aj(s.aj[m]) {}
 };
 
